@@ -93,10 +93,12 @@ def build_cpp_checks(verbose=False):
     out = os.path.join(cpp, "dropin_check")
     _run([CXX, "-std=c++17", "-O2", f"-I{INCLUDE}", src, "-o", out, f"-L{HERE}", "-lcqx",
           "-Wl,-rpath,$ORIGIN/../../cubiquity_amd"], verbose)
-    emu = os.path.join(cpp, "core_emulation.cpp")
-    if os.path.exists(emu):
-        _run([CXX, "-std=c++17", "-O2", "-ffp-contract=off", "-fno-fast-math", f"-I{os.path.join(cpp, 'host_shim')}",
-              f"-I{INCLUDE}", f"-I{CSRC}", emu, "-o", os.path.join(cpp, "core_emulation")], verbose)
+    for name in ("core_emulation", "packed_emulation"):
+        emu = os.path.join(cpp, name + ".cpp")
+        if os.path.exists(emu):
+            _run([CXX, "-std=c++17", "-O2", "-ffp-contract=off", "-fno-fast-math",
+                  f"-I{os.path.join(cpp, 'host_shim')}", f"-I{INCLUDE}", f"-I{CSRC}", emu, "-o",
+                  os.path.join(cpp, name)], verbose)
     return out
 
 

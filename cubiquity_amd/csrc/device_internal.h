@@ -4,6 +4,7 @@
 #include "cqx_internal.h"
 #include "trace_ranges.h"
 #include "traverse_core.h"
+#include "walk_packed.h"
 
 #include <hip/hip_runtime.h>
 
@@ -61,6 +62,11 @@ struct cqx_dvolume {
     cqx_subdag* sub = nullptr;
     uint64_t node_count = 0;
     uint64_t capacity = 0; // nodes the device buffer holds (headroom for appended edits)
+    // The packed copy of the store (walk_packed.h): present for stores of at most 2^24 nodes, used
+    // when packed_ok (the SubDAGs lie within its coordinate limit).
+    uint32_t* packed = nullptr;
+    uint64_t packed_capacity = 0;
+    bool packed_ok = false;
     uint32_t root = 0;
     cqx_subdag hsub[8];
     int max_height = 0; // largest SubDAG start height (stack rows needed: max_height + 1)
@@ -83,6 +89,22 @@ struct ScratchView {
 
 // Grows the context's staging buffer (host-buffer entry points) to at least `bytes`.
 cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
+// Brings the packed copy up to date after nodes [first, node_count), the SubDAGs or the buffers
+// changed (work queued on the null stream), and drops the path tracer's plan if its graph no longer
+// fits. A copy that cannot be allocated is left out.
+cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);
+
+// The packed word of a child: its index and the occupancy mask of its node.
+__device__ __forceinline__ uint32_t pack_child(const uint32_t* __restrict__ nodes, uint32_t child)
+{
+    if (child == 0) return 0u;
+    const uint4* q = reinterpret_cast<const uint4*>(nodes) + uint64_t(child) * 2;
+    const uint4 a = q[0], b = q[1];
+    const uint32_t mask = (a.x ? 1u : 0u) | (a.y ? 2u : 0u) | (a.z ? 4u : 0u) | (a.w ? 8u : 0u) | (b.x ? 16u : 0u) |
+                          (b.y ? 32u : 0u) | (b.z ? 64u : 0u) | (b.w ? 128u : 0u);
+    return cqxd::packed_word(child, mask);
+}
+
 // Launches the traversal of `n` rays (or of *n_dev rays, at most n, when n_dev is not null).
 // Counters and binning buffers are the context's, or `sv`'s when it is given (then nothing is
 // allocated).

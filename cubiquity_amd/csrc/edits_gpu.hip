@@ -977,8 +977,8 @@ cqx_status ensure_store(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t count)
     return CQX_OK;
 }
 
-// Sets the volume's root and recomputes its SubDAGs on the device.
-cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root)
+// Sets the volume's root and recomputes its SubDAGs on the device; nodes from first_new on are new.
+cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root, uint64_t first_new)
 {
     uint32_t* d = nullptr;
     cqx_status st = buf(vol->edits, kBufSubRoot, 2, &d);
@@ -1001,6 +1001,9 @@ cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root)
     vol->root = root;
     std::memcpy(vol->hsub, s, sizeof(s));
     vol->max_height = max_height;
+    st = cqx::refresh_packed(ctx, vol, first_new);
+    if (st != CQX_OK) return st;
+    HIP_TRY(hipStreamSynchronize(nullptr));
     return CQX_OK;
 }
 
@@ -1270,7 +1273,7 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
     E->indexed = out[0];
     ms[4] = ms_since(t_phase);
     t_phase = clock::now();
-    st = set_root(ctx, vol, out[1]);
+    st = set_root(ctx, vol, out[1], base);
     if (st != CQX_OK) return st;
     ms[5] = ms_since(t_phase);
     cqx::log_debug("device edits: %llu spheres over %u regions of side 2^%d (%d runs); %llu listed, %llu appended, "
@@ -1303,7 +1306,7 @@ cqx_status cqx_volume_undo(cqx_ctx* ctx, cqx_dvolume* vol)
     E->roots[E->current] = vol->root;
     if (E->current > 0) E->current--;
     HIP_TRY(hipDeviceSynchronize());
-    return set_root(ctx, vol, E->roots[E->current]);
+    return set_root(ctx, vol, E->roots[E->current], vol->node_count);
 }
 
 cqx_status cqx_volume_redo(cqx_ctx* ctx, cqx_dvolume* vol)
@@ -1314,7 +1317,7 @@ cqx_status cqx_volume_redo(cqx_ctx* ctx, cqx_dvolume* vol)
     E->roots[E->current] = vol->root;
     if (E->current + 1 < E->roots.size()) E->current++;
     HIP_TRY(hipDeviceSynchronize());
-    return set_root(ctx, vol, E->roots[E->current]);
+    return set_root(ctx, vol, E->roots[E->current], vol->node_count);
 }
 
 cqx_status cqx_volume_download(cqx_ctx* ctx, const cqx_dvolume* vol, uint64_t first, uint64_t count, uint32_t* nodes)

@@ -9,6 +9,11 @@
 //                           global counter with one atomic, handed out by ballot prefix
 //                           (variant 2); variant 3 also keeps the current node's 8 children in
 //                           registers
+//   k_walk_lane / k_walk_persistent
+//                           the same two launches over a volume's packed copy (walk_packed.h),
+//                           taken by variants 1 and 2 with the full stack
+//   k_pack_nodes / k_pack_subdags
+//                           build and extend that copy
 //   k_ray_bounds / k_bin_grid / k_bin_count / k_bin_columns / k_bin_scan / k_bin_scatter
 //                           optional prepass of the persistent variants: rays binned by origin
 //                           into a coarse Morton grid over the origins' bounds, handed out cell
@@ -341,6 +346,211 @@ __global__ void __launch_bounds__(256) k_intersect_pair(SingleSource src, uint64
             if (w1) walk_step_on(P, S[1], stk[1], stride, c1);
         }
     }
+}
+
+// ---- the packed walk ---------------------------------------------------------------------------
+// k_walk_lane and k_walk_persistent are k_intersect_lane and k_intersect_persistent on a volume's
+// packed copy (walk_packed.h): the same launches (variants 1 and 2) with the same records, taken
+// whenever every volume of the launch has one.
+
+struct PackedSingle {
+    static constexpr bool kUniform = true;
+    PackedParams P;
+    const cqx_ray* __restrict__ rays;
+    cqx_hit* __restrict__ hits;
+    const uint32_t* __restrict__ order = nullptr;
+    __device__ __forceinline__ void fetch(uint64_t id, PackedParams&, const float*& ray, cqx_hit*& out) const
+    {
+        const uint64_t r = order ? uint64_t(order[id]) : id;
+        ray = reinterpret_cast<const float*>(rays + r);
+        out = hits + r;
+    }
+};
+
+struct PackedDesc {
+    const uint32_t* packed;
+    const cqx_subdag* sub;
+    const cqx_ray* rays;
+    cqx_hit* hits;
+    uint64_t first;
+    uint32_t surf;
+    uint32_t fp_disabled;
+    float max_footprint, lod_hi, lod_lo;
+};
+
+struct PackedBatch {
+    static constexpr bool kUniform = false;
+    const PackedDesc* __restrict__ desc;
+    uint32_t n_batches;
+    uint32_t max_iters;
+    uint32_t top;
+    __device__ __forceinline__ void fetch(uint64_t id, PackedParams& T, const float*& ray, cqx_hit*& out) const
+    {
+        uint32_t lo = 0, hi = n_batches; // invariant: desc[lo].first <= id < desc[hi].first
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (desc[mid].first <= id) lo = mid;
+            else hi = mid;
+        }
+        const PackedDesc& b = desc[lo];
+        T.packed = b.packed;
+        T.sub = b.sub;
+        T.surf = b.surf;
+        T.fp_disabled = b.fp_disabled;
+        T.max_footprint = b.max_footprint;
+        T.lod_hi = b.lod_hi;
+        T.lod_lo = b.lod_lo;
+        T.max_iters = max_iters;
+        T.top = top;
+        const uint64_t k = id - b.first;
+        ray = reinterpret_cast<const float*>(b.rays + k);
+        out = b.hits + k;
+    }
+};
+
+__device__ __forceinline__ const PackedParams& uniform_params(const PackedSingle& s, const PackedParams&) { return s.P; }
+__device__ __forceinline__ const PackedParams& uniform_params(const PackedBatch&, const PackedParams& lane) { return lane; }
+
+__device__ __forceinline__ void setup_packed(PackedRay& S, const float* r)
+{
+    float v[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) v[i] = __builtin_nontemporal_load(r + i);
+    ray_setup(S, v[0], v[1], v[2], v[3], v[4], v[5]);
+    S.plain = ray_plain(S) ? 1u : 0u;
+}
+
+// Up to `steps` steps of the wave's walking lanes: the plain rays' step when every walking lane may
+// take it (its ray plain, its iterations far enough from the cap), the general one otherwise.
+template <bool kLod>
+__device__ __forceinline__ void walk_burst(const PackedParams& P, PackedRay& S, char* lds, uint32_t base, uint32_t steps)
+{
+    const bool walking = S.phase == kWalk;
+    const uint32_t room = P.max_iters >= 2u * steps ? P.max_iters - 2u * steps : 0u;
+    const bool odd = walking && (!S.plain || S.iters > room || P.max_iters < 2u * steps);
+    if (__ballot(odd)) {
+        for (uint32_t k = 0; k < steps; k++)
+            if (S.phase == kWalk) walk_step_packed_any(P, S, lds, base);
+    } else {
+        for (uint32_t k = 0; k < steps; k++)
+            if (S.phase == kWalk) walk_step_packed<kLod>(P, S, lds, base);
+    }
+}
+
+template <bool kLod>
+__global__ void __launch_bounds__(256) k_walk_lane(PackedParams P, const cqx_ray* __restrict__ rays, uint64_t n,
+                                                   const uint32_t* __restrict__ n_dev, cqx_hit* __restrict__ hits)
+{
+    extern __shared__ char lds_rows[];
+    if (n_dev) {
+        const uint64_t nd = *n_dev;
+        n = nd < n ? nd : n;
+    }
+    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t base = (threadIdx.x >> 6) * (P.top + 1u) * kRowBytes + (threadIdx.x & 63u) * 4u;
+    const uint32_t occ = occupied_octants(P.sub);
+    PackedRay S;
+    setup_packed(S, reinterpret_cast<const float*>(rays + i));
+    while (!is_finished(S.phase)) {
+        enter_octants_packed(P.sub, P, S, lds_rows, base, occ);
+        while (S.phase == kWalk) walk_burst<kLod>(P, S, lds_rows, base, 8u);
+    }
+    cqx_hit h;
+    emit_packed(P, S, h);
+    store_record(hits + i, h);
+}
+
+template <typename Source, bool kLod>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6))) k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev,
+                                                         unsigned long long* __restrict__ counters, uint32_t regroup,
+                                                         uint32_t refill, uint32_t rows, uint32_t chunk)
+{
+    extern __shared__ char lds_rows[];
+    if (n_dev) {
+        const uint64_t nd = *n_dev;
+        n = nd < n ? nd : n;
+    }
+    PackedParams P;
+    cqx_hit* dst = nullptr;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t base = (threadIdx.x >> 6) * rows * kRowBytes + lane * 4u;
+    const uint64_t per_q = (n + kQueues - 1) / kQueues;
+    uint32_t qc = blockIdx.x % kQueues; // current queue
+    uint32_t drained = 0;               // queues found empty so far
+    uint64_t c_next = 0, c_end = 0;     // ray ids claimed by this wave
+
+    PackedRay S;
+    S.phase = kIdle;
+    uint32_t occ = 0xffu;
+    __shared__ cqx_subdag lds_sub[8];
+    if constexpr (Source::kUniform) {
+        occ = occupied_octants(src.P.sub);
+        if (threadIdx.x < 8) lds_sub[threadIdx.x] = src.P.sub[threadIdx.x];
+        __syncthreads();
+    }
+    const auto enter = [&](PackedRay& R) {
+        if constexpr (Source::kUniform) enter_octants_packed(lds_sub, src.P, R, lds_rows, base, occ);
+        else enter_octants_packed(P.sub, P, R, lds_rows, base, occ);
+    };
+
+    for (;;) {
+        const uint64_t walking = __ballot(S.phase == kWalk);
+        const uint32_t nwait = 64u - uint32_t(__popcll(walking));
+        if (nwait >= refill || walking == 0) {
+            enter(S);
+            if (is_finished(S.phase)) {
+                cqx_hit out;
+                emit_packed(uniform_params(src, P), S, out);
+                store_record(dst, out);
+                S.phase = kIdle;
+            }
+            while (c_next == c_end && drained < kQueues) {
+                const uint64_t q_begin = per_q * qc;
+                const uint64_t q_end = q_begin + per_q < n ? q_begin + per_q : n;
+                const uint64_t q_len = q_end > q_begin ? q_end - q_begin : 0;
+                unsigned long long claim = 0;
+                if (lane == 0) claim = atomicAdd(&counters[qc * kCounterStride], (unsigned long long)chunk);
+                claim = __shfl(claim, 0);
+                if (claim < q_len) {
+                    c_next = q_begin + claim;
+                    c_end = q_begin + (claim + chunk < q_len ? claim + chunk : q_len);
+                } else {
+                    qc = (qc + 1) % kQueues;
+                    drained++;
+                }
+            }
+            const uint64_t idle = __ballot(S.phase == kIdle);
+            if (S.phase == kIdle) {
+                const uint32_t rank = uint32_t(__popcll(idle & ((1ull << lane) - 1ull)));
+                const uint64_t k = c_next + rank;
+                if (k < c_end) {
+                    const float* r;
+                    src.fetch(k, P, r, dst);
+                    setup_packed(S, r);
+                    enter(S);
+                }
+            }
+            const uint64_t nidle = uint64_t(__popcll(idle));
+            c_next = c_next + nidle < c_end ? c_next + nidle : c_end;
+            if (drained == kQueues && __ballot(S.phase != kIdle) == 0) break;
+        }
+        walk_burst<kLod>(uniform_params(src, P), S, lds_rows, base, regroup);
+    }
+}
+
+// Packed words of store words [first, first + count): each child's index and the occupancy mask of
+// its node. One thread per word; the mask is one 32-byte read of the child's node.
+__global__ void __launch_bounds__(256) k_pack_nodes(const uint32_t* __restrict__ nodes, uint32_t* __restrict__ packed,
+                                                    uint64_t first, uint64_t count)
+{
+    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < count) packed[first + i] = cqx::pack_child(nodes, nodes[first + i]);
+}
+
+__global__ void k_pack_subdags(const uint32_t* __restrict__ nodes, cqx_subdag* __restrict__ sub)
+{
+    if (threadIdx.x < 8) sub[threadIdx.x].pad0 = cqx::pack_child(nodes, sub[threadIdx.x].node);
 }
 
 // ---- ray binning -------------------------------------------------------------------------------
@@ -720,6 +930,48 @@ cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes)
     return CQX_OK;
 }
 
+cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
+{
+    uint32_t* const old = vol->packed;
+    const bool old_ok = vol->packed_ok;
+    if (vol->node_count > kPackedNodes) {
+        if (old) {
+            HIP_TRY(hipDeviceSynchronize()); // launches in flight may read it
+            release(old);
+            vol->packed = nullptr;
+            vol->packed_capacity = 0;
+        }
+    } else if (vol->node_count > vol->packed_capacity) {
+        const uint64_t cap = std::min<uint64_t>(std::max(vol->capacity, vol->node_count), kPackedNodes);
+        HIP_TRY(hipDeviceSynchronize());
+        release(old);
+        vol->packed = nullptr;
+        vol->packed_capacity = 0;
+        if (hipMalloc(&vol->packed, size_t(cap) * 32) == hipSuccess) {
+            vol->packed_capacity = cap;
+            first = 0;
+        } else {
+            vol->packed = nullptr; // traversal then runs on the raw store
+            (void)hipGetLastError();
+        }
+    }
+    if (vol->packed) {
+        const uint64_t words = (vol->node_count - first) * 8;
+        if (words)
+            hipLaunchKernelGGL(k_pack_nodes, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, 0, vol->nodes, vol->packed,
+                               first * 8, words);
+        hipLaunchKernelGGL(k_pack_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, vol->sub);
+        HIP_TRY(hipGetLastError());
+    }
+    vol->packed_ok = vol->packed && packed_eligible(vol->node_count, vol->hsub);
+    if (ctx->pt_plan && (vol->packed != old || vol->packed_ok != old_ok)) {
+        HIP_TRY(hipDeviceSynchronize());
+        destroy_pt_plan(ctx->pt_plan); // its captured graph holds the old copy or the other walk
+        ctx->pt_plan = nullptr;
+    }
+    return CQX_OK;
+}
+
 cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray* rays, uint64_t n,
                             const uint32_t* n_dev, uint32_t flags, float max_footprint, cqx_hit* hits,
                             const cqx_launch_cfg* cfg, hipStream_t stream, const ScratchView* sv)
@@ -754,6 +1006,23 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
     const size_t lds = size_t(rows) * block * sizeof(uint32_t);
     if (lds > size_t(ctx->lds_per_block)) return fail(CQX_ERR_LIMIT, "stack needs %zu B of LDS per block", lds);
 
+    // The packed walk serves the full-stack launches of variants 1 and 2; the others (and volumes past
+    // its limits) keep the walk over the raw store.
+    const bool packed = vol->packed_ok && !short_stack && (variant == 1 || variant == 2);
+    PackedParams PP{};
+    bool lod = false;
+    if (packed) {
+        PP.packed = vol->packed;
+        PP.sub = vol->sub;
+        PP.surf = P.surf;
+        PP.max_iters = P.max_iters;
+        PP.top = uint32_t(vol->max_height);
+        PP.fp_disabled = P.fp_disabled;
+        PP.max_footprint = max_footprint;
+        lod_thresholds(max_footprint, PP.lod_hi, PP.lod_lo);
+        lod = !std::isinf(PP.lod_hi);
+    }
+
     const uint32_t bin_bits = cfg ? cfg->bin_bits : 0u;
     const uint32_t* order = nullptr;
     if (bin_bits) {
@@ -770,7 +1039,13 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
     if (variant == 1) {
         const uint64_t blocks = (n + block - 1) / block;
         if (blocks > 0x7fffffffull) return fail(CQX_ERR_LIMIT, "too many rays for one launch");
-        hipLaunchKernelGGL(k_intersect_lane, dim3(uint32_t(blocks)), dim3(block), lds, stream, P, rays, n, n_dev, hits);
+        if (packed && lod)
+            hipLaunchKernelGGL(k_walk_lane<true>, dim3(uint32_t(blocks)), dim3(block), lds, stream, PP, rays, n, n_dev,
+                               hits);
+        else if (packed)
+            hipLaunchKernelGGL(k_walk_lane<false>, dim3(uint32_t(blocks)), dim3(block), lds, stream, PP, rays, n, n_dev,
+                               hits);
+        else hipLaunchKernelGGL(k_intersect_lane, dim3(uint32_t(blocks)), dim3(block), lds, stream, P, rays, n, n_dev, hits);
     } else if (variant == 5) {
         uint32_t blocks, regroup, refill, chunk;
         cqx_status st = persistent_shape(ctx, cfg, block, (n + 1) / 2, blocks, regroup, refill, chunk);
@@ -799,7 +1074,14 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
             return fail(CQX_ERR_LIMIT, "stack and SubDAG copy need %zu B of LDS per block", lds_total + kSubdagCopyBytes);
         SingleSource src{ P, rays, hits, order };
         hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, stream, counters);
-        if (variant == 2 && short_stack)
+        const PackedSingle psrc{ PP, rays, hits, order };
+        if (packed && lod)
+            hipLaunchKernelGGL((k_walk_persistent<PackedSingle, true>), dim3(blocks), dim3(block), lds, stream, psrc, n,
+                               n_dev, counters, regroup, refill, rows, chunk);
+        else if (packed)
+            hipLaunchKernelGGL((k_walk_persistent<PackedSingle, false>), dim3(blocks), dim3(block), lds, stream, psrc, n,
+                               n_dev, counters, regroup, refill, rows, chunk);
+        else if (variant == 2 && short_stack)
             hipLaunchKernelGGL((k_intersect_persistent<SingleSource, false, false, true>), dim3(blocks), dim3(block), lds,
                                stream, src, n, n_dev, counters, regroup, refill, rows, 0u, chunk);
         else if (variant == 3 && short_stack)
@@ -917,6 +1199,15 @@ cqx_status cqx_volume_upload(cqx_ctx* ctx, const uint32_t* nodes, uint64_t node_
         delete v;
         return fail(CQX_ERR_HIP, "upload of the node store failed");
     }
+    st = cqx::refresh_packed(ctx, v, 0);
+    if (st == CQX_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = fail(CQX_ERR_HIP, "packing the node store failed");
+    if (st != CQX_OK) {
+        release(v->packed);
+        release(v->nodes);
+        release(v->sub);
+        delete v;
+        return st;
+    }
     *out = v;
     return CQX_OK;
 }
@@ -983,6 +1274,9 @@ cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nod
     vol->root = root;
     std::memcpy(vol->hsub, s, sizeof(s));
     vol->max_height = max_height;
+    st = cqx::refresh_packed(ctx, vol, first);
+    if (st != CQX_OK) return st;
+    HIP_TRY(hipStreamSynchronize(nullptr));
     return CQX_OK;
 }
 
@@ -997,6 +1291,7 @@ cqx_status cqx_volume_free(cqx_ctx* ctx, cqx_dvolume* vol)
         ctx->pt_plan = nullptr;
     }
     release(vol->nodes);
+    release(vol->packed);
     release(vol->sub);
     cqx::destroy_device_edits(vol->edits);
     delete vol;
@@ -1079,6 +1374,8 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     if (!batches) return fail(CQX_ERR_INVALID_ARG, "null batch array");
     if (cfg && cfg->bin_bits) return fail(CQX_ERR_INVALID_ARG, "ray binning applies to cqx_intersect only");
     std::vector<BatchDesc> desc(n_batches);
+    std::vector<PackedDesc> pdesc(n_batches);
+    bool packed = true, lod = false;
     uint64_t total = 0;
     int max_height = 0;
     for (uint32_t i = 0; i < n_batches; i++) {
@@ -1093,8 +1390,22 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
         desc[i].first = total;
         desc[i].flags = b.flags;
         desc[i].max_footprint = b.max_footprint;
+        PackedDesc& p = pdesc[i];
+        p.packed = b.volume->packed;
+        p.sub = b.volume->sub;
+        p.rays = b.rays;
+        p.hits = b.hits;
+        p.first = total;
+        p.surf = (b.flags & CQX_SURFACE_PROPERTIES) ? 1u : 0u;
+        p.fp_disabled = footprint_is_disabled(b.max_footprint) ? 1u : 0u;
+        p.max_footprint = b.max_footprint;
+        lod_thresholds(b.max_footprint, p.lod_hi, p.lod_lo);
         total += b.n;
-        if (b.n) max_height = std::max(max_height, b.volume->max_height);
+        if (b.n) {
+            max_height = std::max(max_height, b.volume->max_height);
+            packed = packed && b.volume->packed_ok;
+            lod = lod || !std::isinf(p.lod_hi);
+        }
     }
     if (total == 0) return CQX_OK;
     if (total > (uint64_t(1) << 38)) return fail(CQX_ERR_LIMIT, "more than 2^38 rays in one launch");
@@ -1118,7 +1429,9 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     hipStream_t s = hipStream_t(stream_ptr);
     // The descriptor table is per context: wait for an earlier batched launch on this stream.
     HIP_TRY(hipStreamSynchronize(s));
-    const size_t bytes = desc.size() * sizeof(BatchDesc);
+    // one volume past the packed walk's limits, or a launch it does not serve: all on the raw stores
+    packed = packed && !short_stack && !(cfg && cfg->variant == 3);
+    const size_t bytes = packed ? pdesc.size() * sizeof(PackedDesc) : desc.size() * sizeof(BatchDesc);
     if (bytes > ctx->batch_bytes) {
         release(ctx->batch_desc);
         ctx->batch_desc = nullptr;
@@ -1126,7 +1439,8 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
         if (hipMalloc(&ctx->batch_desc, bytes) != hipSuccess) return fail(CQX_ERR_OOM, "descriptor allocation failed");
         ctx->batch_bytes = bytes;
     }
-    HIP_TRY(hipMemcpy(ctx->batch_desc, desc.data(), bytes, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(ctx->batch_desc, packed ? static_cast<const void*>(pdesc.data()) : desc.data(), bytes,
+                      hipMemcpyHostToDevice));
     uint32_t blocks, regroup, refill, chunk;
     st = persistent_shape(ctx, cfg, block, total, blocks, regroup, refill, chunk);
     if (st != CQX_OK) return st;
@@ -1135,7 +1449,14 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned long long*>(ctx->d_counter));
     unsigned long long* counters = reinterpret_cast<unsigned long long*>(ctx->d_counter);
     const bool cache = cfg && cfg->variant == 3;
-    if (cache && short_stack)
+    const PackedBatch psrc{ static_cast<const PackedDesc*>(ctx->batch_desc), n_batches, src.max_iters, uint32_t(max_height) };
+    if (packed && lod)
+        hipLaunchKernelGGL((k_walk_persistent<PackedBatch, true>), dim3(blocks), dim3(block), lds, s, psrc, total,
+                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk);
+    else if (packed)
+        hipLaunchKernelGGL((k_walk_persistent<PackedBatch, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
+                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk);
+    else if (cache && short_stack)
         hipLaunchKernelGGL((k_intersect_persistent<BatchSource, true, false, true>), dim3(blocks), dim3(block), lds, s,
                            src, total, (const uint32_t*)nullptr, counters, regroup, refill, rows, 0u, chunk);
     else if (short_stack)

@@ -151,7 +151,8 @@ __device__ __forceinline__ void result_miss(cqx_hit& out)
 }
 
 // Ray setup, raytracing.cpp:415-434.
-__device__ __forceinline__ void ray_setup(RayState& S, float rox, float roy, float roz, float rdx, float rdy, float rdz)
+template <typename Ray>
+__device__ __forceinline__ void ray_setup(Ray& S, float rox, float roy, float roz, float rdx, float rdy, float rdz)
 {
     const uint32_t sbx = rdx < 0.0f, sby = rdy < 0.0f, sbz = rdz < 0.0f;
     S.sign_bits = sbx | (sby << 1) | (sbz << 2);
@@ -180,7 +181,8 @@ __device__ __forceinline__ void ray_setup(RayState& S, float rox, float roy, flo
 
 // Next octant in order of axis crossings, raytracing.cpp:469-475. The walk is over when all
 // octants were visited (a miss) or when no axis steps (the reference would loop forever).
-__device__ __forceinline__ void octant_advance(RayState& S)
+template <typename Ray>
+__device__ __forceinline__ void octant_advance(Ray& S)
 {
     const float m = min3f(S.distx, S.disty, S.distz);
     uint32_t step = 0;

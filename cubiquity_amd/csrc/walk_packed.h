@@ -1,0 +1,442 @@
+// The ESVO walk over the packed copy of a node store: the traversal every launch on an eligible
+// volume runs (see packed_eligible), with the records of traverse_core.h bit for bit.
+//
+// What it is built around, measured on gfx950 (one instruction type in a loop, 8 waves per SIMD,
+// cycles per wave instruction per SIMD):
+//   * 2 cycles: v_add/sub/mul/fma_f32, v_mov, v_add/sub_u32, v_and/or/xor/not, right shifts, with
+//     VGPR, inline-constant or literal operands;
+//   * 4 cycles: compares, v_cndmask, min/max, int <-> float conversions, left shifts, bit-field and
+//     other three-operand integer forms, and the 2-cycle ones with an SGPR operand.
+// The walk is bound by these issue cycles (the step of traverse_core.h costs about 415 of them with
+// its three paths live, 42 steps per ray on the 1024^3 benchmark), then by the L2's rate for
+// scattered child reads (256 G reads/s for lines that hit L2). Hence:
+//   * Packed words. Each child word of the copy holds the child's index << 8 | its occupancy mask
+//     (bit c: its child c is not empty). The walk knows from the node's own word which children are
+//     empty and reads memory for occupied ones only: 23 reads per ray instead of 43.
+//   * One step = one advance over an empty child (with its pop), where the lane stands on one, then
+//     the read of an occupied child and the descent into it: 28 steps per ray instead of 42.
+//   * Positions are floats holding kBias + integer: exact for |p| <= 2^22, so plane positions need
+//     float additions only, and the bits below the bias are those of the integer for the pop's
+//     exclusive or and masks.
+//   * Per-axis choices are sign masks (a float difference's sign bit shifted over the word) instead
+//     of compare + select, and min/max of three values one instruction.
+// Measured against the raw-store walk (MI355X, default launch): 1024^3, 2^24 incoherent rays 3.13 ->
+// 2.21 ms; 4096^3, 4.0 M rays without surface properties 2.00 -> 1.18 ms; 1280x720 primary rays at
+// 1024^3 with LOD 0.30 -> 0.24 ms; reads from L2 5.5e8 -> 2.6e8 per 2^24-ray launch.
+// The sign masks and one-instruction minima need values without NaN, -0 and underflow: ray_plain() is true for rays where
+// none can occur. A wave with another ray among its walking lanes takes walk_step_packed_any, which
+// keeps the compare-selects of the reference.
+#pragma once
+
+#include "traverse_core.h"
+
+#include <cmath>
+#include <cstring>
+
+namespace cqxd {
+
+constexpr float kBias = 12582912.0f;         // 1.5 * 2^23
+constexpr uint32_t kBiasBits = 0x4b400000u;  // its bits: as_uint(kBias + p) = kBiasBits + p
+constexpr int32_t kPackedExtent = 1 << 22;   // SubDAG corners lie in [-2^22, 2^22]
+constexpr uint32_t kPackedNodes = 1u << 24;  // node indices of a packed store
+constexpr uint32_t kRowBytes = 64u * 4u;     // one stack row: a word per lane of the wave
+
+struct PackedParams {
+    const uint32_t* __restrict__ packed; // node_count x 8 packed words
+    const cqx_subdag* __restrict__ sub;  // 8 SubDAGs, pad0 holding the node's packed word
+    uint32_t surf;
+    uint32_t max_iters;
+    uint32_t top;     // largest SubDAG height of the launch: the row of height h is top - h
+    float lod_hi;     // child of size s and exit time t large: 0 <= t <= lod_hi * s or t <= lod_lo * s < 0
+    float lod_lo;
+    uint32_t fp_disabled;
+    float max_footprint;
+};
+
+// Word for a child with index `index` whose occupancy mask is `mask` (0 for an empty child).
+__host__ __device__ inline uint32_t packed_word(uint32_t index, uint32_t mask) { return index ? (index << 8) | mask : 0u; }
+
+// The footprint test size / t > F (one correctly rounded division; size a power of two) as thresholds
+// on t / size, which is exact: with u = t / size, RN(1 / u) > F holds for 0 <= u <= hi and for
+// u <= lo < 0 (RN(1 / u) is monotonic on either side of 0). hi = infinity: for every u >= 0.
+inline void lod_thresholds(float F, float& hi, float& lo)
+{
+    hi = -1.0f;
+    lo = -INFINITY;
+    const auto value = [](uint32_t b) { float f; std::memcpy(&f, &b, 4); return f; };
+    if (F < 0.0f) { // u > 0: always; u < 0: |u| at least the smallest magnitude b with RN(-1 / |u|) > F
+        hi = INFINITY;
+        uint32_t a = 0u, b = 0x7f800000u;
+        while (b - a > 1) {
+            const uint32_t m = a + (b - a) / 2;
+            (-1.0f / value(m) > F ? b : a) = m;
+        }
+        lo = -value(b);
+    } else if (F < INFINITY) { // 0 <= u <= the largest magnitude a with RN(1 / u) > F
+        uint32_t a = 0u, b = 0x7f800000u;
+        while (b - a > 1) {
+            const uint32_t m = a + (b - a) / 2;
+            (1.0f / value(m) > F ? a : b) = m;
+        }
+        hi = value(a);
+    }
+}
+
+// Whether a store with these SubDAGs can be walked packed: node indices below 2^24, positions whose
+// biased floats are exact, and heights as the walk's child sizes state them.
+inline bool packed_eligible(uint64_t node_count, const cqx_subdag (&sub)[8])
+{
+    if (node_count > kPackedNodes) return false;
+    for (const cqx_subdag& s : sub) {
+        if (s.node == 0) continue;
+        if (s.height < 0 || s.height > 22 || (s.height == 0 && s.node >= kMaterialCount)) return false;
+        for (int a = 0; a < 3; a++)
+            if (s.lower[a] < -kPackedExtent || int64_t(s.lower[a]) + (int64_t(1) << s.height) > kPackedExtent) return false;
+    }
+    return true;
+}
+
+// A state of the walk (RayState of traverse_core.h, in the packed walk's terms).
+struct PackedRay {
+    float ox, oy, oz; // reflected, shifted origin
+    float dx, dy, dz; // |direction|
+    float ix, iy, iz; // 1 / |direction|
+    float distx, disty, distz;
+    uint32_t sign_bits;
+    uint32_t oct;
+    uint32_t node;    // packed word of the current node
+    uint32_t word;    // the hit child's packed word once the phase is kHit
+    float bx, by, bz; // lower corner of the current child, plus kBias
+    float s;          // its size
+    uint32_t cid;
+    uint32_t sp;      // byte offset of the stack row of the current node's height
+    uint32_t zstart;  // 32 - the SubDAG's height
+    float last_exit;
+    uint32_t entries, iters;
+    uint32_t phase;
+    uint32_t plain;   // ray_plain()
+};
+
+__device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); }
+__device__ __forceinline__ float bitsf(uint32_t u) { return __uint_as_float(u); }
+
+// Minimum and maximum of values that are neither NaN nor -0, in one instruction.
+__device__ __forceinline__ float plain_min3(float a, float b, float c)
+{
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return min3f(a, b, c);
+#endif
+}
+__device__ __forceinline__ float plain_max3(float a, float b, float c)
+{
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return max3f(a, b, c);
+#endif
+}
+// max(x, smallest denormal)
+__device__ __forceinline__ float at_least_denorm(float x)
+{
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_max_f32 %0, 1, %1" : "=v"(r) : "v"(x)); // inline constant 1: the bits of 2^-149
+    return r;
+#else
+    return smax(bitsf(1u), x);
+#endif
+}
+// All bits set where a < b (0 otherwise), for a, b finite: with denormals a - b is negative exactly then.
+__device__ __forceinline__ uint32_t less_mask(float a, float b) { return uint32_t(int32_t(fbits(a - b)) >> 31); }
+
+// Rays whose walk meets no NaN, no -0 and no underflow: for coordinates p with |p| <= 2^22, p - o is
+// 0 or at least 2^-25 in magnitude (o = fl(ray origin + 0.5) is a multiple of 2^-25) and at most
+// 2^60, and 1/|d| within [2^-60, 2^60], so every (p - o) * (1/|d|) is +0 or a normal number.
+__device__ __forceinline__ bool ray_plain(const PackedRay& S)
+{
+    const float o = (fabsf(S.ox) + fabsf(S.oy)) + fabsf(S.oz); // NaN and infinity stay
+    const float d = (S.dx + S.dy) + S.dz;
+    return (o <= 5.0e17f) & (d <= 1.0e18f) & (S.dx >= 1.0e-18f) & (S.dy >= 1.0e-18f) & (S.dz >= 1.0e-18f);
+}
+
+__device__ __forceinline__ uint32_t& stack_word(char* lds, uint32_t off) { return *reinterpret_cast<uint32_t*>(lds + off); }
+
+// Byte offset of the row of height `h` given the lane's base (its column's first row).
+__device__ __forceinline__ uint32_t packed_row(uint32_t base, uint32_t top, int32_t h) { return base + (top - uint32_t(h)) * kRowBytes; }
+
+// octant_enter of traverse_core.h. `base`: byte offset of the lane's stack column; `tab`: the 8
+// SubDAGs, their packed root words in pad0.
+__device__ __forceinline__ void octant_enter_packed(const cqx_subdag* tab, const PackedParams& P, PackedRay& S, char* lds,
+                                                    uint32_t base, uint32_t occ)
+{
+    const uint32_t o = S.oct ^ S.sign_bits;
+    const cqx_subdag sd = ((occ >> o) & 1u) ? tab[o] : cqx_subdag{};
+    if (sd.node > 0) {
+        const int32_t sbx = S.sign_bits & 1u, sby = (S.sign_bits >> 1) & 1u, sbz = (S.sign_bits >> 2) & 1u;
+        const int32_t size = int32_t(1u << sd.height);
+        const int32_t px = wsub(wmul(sd.lower[0], 1 - 2 * sbx), wmul(sbx, size));
+        const int32_t py = wsub(wmul(sd.lower[1], 1 - 2 * sby), wmul(sby, size));
+        const int32_t pz = wsub(wmul(sd.lower[2], 1 - 2 * sbz), wmul(sbz, size));
+        const float nsz = float(size); // heights of a packed store are at most 22
+        const float entry = max3f((float(px) - S.ox) * S.ix, (float(py) - S.oy) * S.iy, (float(pz) - S.oz) * S.iz);
+        const float exitt = min3f(((float(px) + nsz) - S.ox) * S.ix, ((float(py) + nsz) - S.oy) * S.iy,
+                                  ((float(pz) + nsz) - S.oz) * S.iz);
+        if (entry < exitt) {
+            // ancestors not pushed yet read as node 0, as in the reference's zeroed stack
+            for (uint32_t r = P.top - uint32_t(sd.height); r <= P.top; r++) stack_word(lds, base + r * kRowBytes) = 0u;
+            S.sp = packed_row(base, P.top, sd.height);
+            S.zstart = 32u - uint32_t(sd.height);
+            S.node = uint32_t(sd.pad0);
+            const int32_t csize = int32_t(uint32_t(size) / 2u);
+            bool bx, by, bz;
+            S.cid = first_child(entry, S.ox, S.oy, S.oz, S.ix, S.iy, S.iz, wadd(px, csize), wadd(py, csize),
+                                wadd(pz, csize), bx, by, bz);
+            S.bx = kBias + float(wadd(px, bx ? csize : 0));
+            S.by = kBias + float(wadd(py, by ? csize : 0));
+            S.bz = kBias + float(wadd(pz, bz ? csize : 0));
+            S.s = float(csize);
+            S.last_exit = exitt;
+            S.entries++;
+            S.phase = kWalk;
+            return;
+        }
+    }
+    octant_advance(S);
+}
+
+__device__ __forceinline__ void enter_octants_packed(const cqx_subdag* tab, const PackedParams& P, PackedRay& S, char* lds,
+                                                     uint32_t base, uint32_t occ)
+{
+    if (S.phase == kLeave) octant_advance(S);
+    while (S.phase == kOctant) octant_enter_packed(tab, P, S, lds, base, occ);
+}
+
+// The occupied child's word: slot cid ^ signBits of the current node.
+__device__ __forceinline__ uint32_t packed_fetch(const PackedParams& P, const PackedRay& S, uint32_t slot)
+{
+    const uint32_t off = ((S.node >> 3) & ~31u) | (slot << 2); // index * 32 + slot * 4 < 2^29
+    return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(P.packed) + off);
+}
+
+// Exit times of the current child (its upper planes), and their minimum.
+__device__ __forceinline__ float packed_exits(const PackedRay& S, float& t1x, float& t1y, float& t1z)
+{
+    t1x = (((S.bx - kBias) + S.s) - S.ox) * S.ix;
+    t1y = (((S.by - kBias) + S.s) - S.oy) * S.iy;
+    t1z = (((S.bz - kBias) + S.s) - S.oz) * S.iz;
+    return plain_min3(t1x, t1y, t1z);
+}
+
+// Pop to the highest boundary crossed (raytracing.cpp:339-364); obx.. the position before the
+// advance. False when the walk left the SubDAG.
+__device__ __forceinline__ bool packed_pop(PackedRay& S, char* lds, uint32_t base, uint32_t top, float obx, float oby,
+                                           float obz)
+{
+    const uint32_t ux = fbits(S.bx), uy = fbits(S.by), uz = fbits(S.bz);
+    const uint32_t diff = (ux ^ fbits(obx)) | (uy ^ fbits(oby)) | (uz ^ fbits(obz));
+    const uint32_t z = uint32_t(__builtin_clz(diff)); // the highest bit is 31 - z; the node's height 32 - z
+    if (z < S.zstart) {
+        S.phase = kLeave;
+        return false;
+    }
+    S.sp = base + (top - 32u) * kRowBytes + z * kRowBytes;
+    S.node = stack_word(lds, S.sp);
+    const uint32_t keep = uint32_t(int32_t(0x80000000u) >> z); // clears the bits below the boundary's
+    const uint32_t m = 31u - z;
+    S.cid = ((ux >> m) & 1u) | (((uy >> m) & 1u) << 1) | (((uz >> m) & 1u) << 2);
+    S.bx = bitsf(ux & keep);
+    S.by = bitsf(uy & keep);
+    S.bz = bitsf(uz & keep);
+    S.s = bitsf((158u - z) << 23); // 2^(31 - z)
+    S.last_exit = 0.0f;
+    S.entries++;
+    return true;
+}
+
+// One step of a plain ray (ray_plain) whose phase is kWalk: an advance if the current child is empty,
+// then the descent into (or hit of) the current child if it is occupied. Counts up to two
+// iterations; the caller keeps iters + 2 <= max_iters.
+template <bool kLod>
+__device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRay& S, char* lds, uint32_t base)
+{
+    float t1x, t1y, t1z;
+    float tcx = packed_exits(S, t1x, t1y, t1z);
+    uint32_t slot = S.cid ^ S.sign_bits;
+    uint32_t occupied = (S.node >> slot) & 1u;
+    if (!occupied) {
+        // Advance to the next sibling, raytracing.cpp:328-332: the axes whose exit is the minimum.
+        S.iters++;
+        const uint32_t fx = uint32_t(int32_t(fbits(t1x - tcx) - 1u) >> 31), fy = uint32_t(int32_t(fbits(t1y - tcx) - 1u) >> 31),
+                       fz = uint32_t(int32_t(fbits(t1z - tcx) - 1u) >> 31);
+        const float obx = S.bx, oby = S.by, obz = S.bz;
+        S.bx = obx + bitsf(fbits(S.s) & fx);
+        S.by = oby + bitsf(fbits(S.s) & fy);
+        S.bz = obz + bitsf(fbits(S.s) & fz);
+        const uint32_t flips = (fx & 1u) | (fy & 2u) | (fz & 4u);
+        const uint32_t carry = S.cid & flips;
+        S.cid ^= flips;
+        if (carry && !packed_pop(S, lds, base, P.top, obx, oby, obz)) return;
+        tcx = packed_exits(S, t1x, t1y, t1z);
+        slot = S.cid ^ S.sign_bits;
+        occupied = (S.node >> slot) & 1u;
+    }
+    if (occupied) {
+        const uint32_t child = packed_fetch(P, S, slot);
+        S.iters++;
+        const float half = S.s * 0.5f;
+        const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
+        // entry time of the child; children behind the origin (entry <= 0) compare their centre
+        // planes with "t <= 0", which is t < 2^-149 (findFirstChild, raytracing.cpp:178-196)
+        const float tce = at_least_denorm(plain_max3((px - S.ox) * S.ix, (py - S.oy) * S.iy, (pz - S.oz) * S.iz));
+        const uint32_t mx = less_mask(((px + half) - S.ox) * S.ix, tce);
+        const uint32_t my = less_mask(((py + half) - S.oy) * S.iy, tce);
+        const uint32_t mz = less_mask(((pz + half) - S.oz) * S.iz, tce);
+        bool internal = child >= (kMaterialCount << 8);
+        if (kLod) internal = internal & (tcx <= P.lod_hi * S.s);
+        if (tcx < 0.0f) internal = internal & (tcx <= P.lod_lo * S.s);
+        if (internal) {
+            if (S.s < 1.5f) {
+                S.phase = kAnomaly; // deeper than a valid DAG
+                return;
+            }
+            if (tcx < S.last_exit) stack_word(lds, S.sp) = S.node;
+            S.last_exit = tcx;
+            S.sp += kRowBytes;
+            S.node = child;
+            S.s = half;
+            S.entries++;
+            S.bx += bitsf(fbits(half) & mx);
+            S.by += bitsf(fbits(half) & my);
+            S.bz += bitsf(fbits(half) & mz);
+            S.cid = (mx & 1u) | (my & 2u) | (mz & 4u);
+        } else {
+            S.word = child;
+            S.phase = kHit;
+        }
+    }
+}
+
+// hasLargeFootprint with the reference's division (footprint_large of traverse_core.h).
+__device__ __forceinline__ bool packed_footprint_large(const PackedParams& P, float size, float tcx)
+{
+    if (P.fp_disabled && size > 0.0f) return fbits(tcx) <= 0x7f800000u || tcx < -size;
+    return (size / tcx) > P.max_footprint;
+}
+
+// One iteration of the walk (walk_step_on of traverse_core.h) of any ray, with the reference's
+// compare-selects and its iteration cap.
+__device__ __forceinline__ void walk_step_packed_any(const PackedParams& P, PackedRay& S, char* lds, uint32_t base)
+{
+    if (S.iters >= P.max_iters) {
+        S.phase = kAnomaly;
+        return;
+    }
+    S.iters++;
+    const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
+    const float t1x = ((px + S.s) - S.ox) * S.ix, t1y = ((py + S.s) - S.oy) * S.iy, t1z = ((pz + S.s) - S.oz) * S.iz;
+    const float tcx = min3f(t1x, t1y, t1z);
+    const uint32_t slot = S.cid ^ S.sign_bits;
+    if ((S.node >> slot) & 1u) {
+        const uint32_t child = packed_fetch(P, S, slot);
+        if (child < (kMaterialCount << 8) || !packed_footprint_large(P, S.s, tcx)) {
+            S.word = child;
+            S.phase = kHit;
+            return;
+        }
+        if (S.s < 1.5f) {
+            S.phase = kAnomaly;
+            return;
+        }
+        const float tce = max3f((px - S.ox) * S.ix, (py - S.oy) * S.iy, (pz - S.oz) * S.iz);
+        if (tcx < S.last_exit) stack_word(lds, S.sp) = S.node;
+        S.last_exit = tcx;
+        S.sp += kRowBytes;
+        S.node = child;
+        const float half = S.s * 0.5f;
+        S.s = half;
+        S.entries++;
+        const float cx = px + half, cy = py + half, cz = pz + half;
+        const bool behind = tce <= 0.0f;
+        const bool bx = ((cx - S.ox) * S.ix < tce) | (behind & (S.ox >= cx));
+        const bool by = ((cy - S.oy) * S.iy < tce) | (behind & (S.oy >= cy));
+        const bool bz = ((cz - S.oz) * S.iz < tce) | (behind & (S.oz >= cz));
+        S.bx += bx ? half : 0.0f;
+        S.by += by ? half : 0.0f;
+        S.bz += bz ? half : 0.0f;
+        S.cid = (bx ? 1u : 0u) | (by ? 2u : 0u) | (bz ? 4u : 0u);
+        return;
+    }
+    const uint32_t flips = (t1x <= tcx ? 1u : 0u) | (t1y <= tcx ? 2u : 0u) | (t1z <= tcx ? 4u : 0u);
+    const float obx = S.bx, oby = S.by, obz = S.bz;
+    S.bx = obx + ((flips & 1u) ? S.s : 0.0f);
+    S.by = oby + ((flips & 2u) ? S.s : 0.0f);
+    S.bz = obz + ((flips & 4u) ? S.s : 0.0f);
+    const uint32_t carry = S.cid & flips;
+    S.cid ^= flips;
+    if (carry) packed_pop(S, lds, base, P.top, obx, oby, obz);
+}
+
+// Record of a finished ray: emit_record of traverse_core.h from the packed walk's state. The
+// nearest material takes the first occupied child from the node's mask: one read per level.
+__device__ __forceinline__ void emit_packed(const PackedParams& P, const PackedRay& S, cqx_hit& out)
+{
+    result_miss(out);
+    out.entries = S.entries;
+    out.iters = S.iters;
+    if (S.phase == kAnomaly) {
+        out.info = CQX_HIT_ANOMALY;
+        return;
+    }
+    if (S.phase != kHit) return;
+    const uint32_t slot = S.cid ^ S.sign_bits;
+    const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
+    const float t0x = (px - S.ox) * S.ix, t0y = (py - S.oy) * S.iy, t0z = (pz - S.oz) * S.iz;
+    const float tce = max3f(t0x, t0y, t0z);
+    const int32_t bsize = S.s > 0.0f ? int32_t(S.s) : 1; // a SubDAG of height 0: the node itself, of side 1
+    uint32_t info = 1u | (slot << 1) | (uint32_t(find_msb(uint32_t(bsize))) << 4);
+    if (P.surf) {
+        uint32_t m = S.word;
+        uint32_t entries = S.entries;
+        while (m >= (kMaterialCount << 8)) {
+            entries++;
+            const uint32_t mask = m & 0xffu;
+            if (mask == 0) {
+                out.entries = entries;
+                out.info = CQX_HIT_ANOMALY;
+                return;
+            }
+            uint32_t ids = (0x76534210u | 0x88888888u) ^ (S.sign_bits * 0x11111111u);
+            while (!((mask >> (ids & 7u)) & 1u)) ids >>= 4;
+            m = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(P.packed) +
+                                                   (((m >> 3) & ~31u) | ((ids & 7u) << 2)));
+        }
+        out.entries = entries;
+        // normal = vec3(equal(tEntry, childT0)) * -rayDirSign, raytracing.cpp:317-318
+        const float sx = (S.sign_bits & 1u) ? -1.0f : 1.0f, sy = (S.sign_bits & 2u) ? -1.0f : 1.0f,
+                    sz = (S.sign_bits & 4u) ? -1.0f : 1.0f;
+        const float nx = float(tce == t0x) * -sx, ny = float(tce == t0y) * -sy, nz = float(tce == t0z) * -sz;
+        info |= ((nx != 0.0f ? 1u : 0u) | ((fbits(nx) >> 31) << 1)) << 9;
+        info |= ((ny != 0.0f ? 1u : 0u) | ((fbits(ny) >> 31) << 1)) << 11;
+        info |= ((nz != 0.0f ? 1u : 0u) | ((fbits(nz) >> 31) << 1)) << 13;
+        info |= (m >> 8) << 16;
+    }
+    const int32_t ipx = int32_t(fbits(S.bx) - kBiasBits), ipy = int32_t(fbits(S.by) - kBiasBits),
+                  ipz = int32_t(fbits(S.bz) - kBiasBits);
+    const int32_t vx = entered_voxel(S.ox, S.dx, tce, ipx, bsize, t0x == tce);
+    const int32_t vy = entered_voxel(S.oy, S.dy, tce, ipy, bsize, t0y == tce);
+    const int32_t vz = entered_voxel(S.oz, S.dz, tce, ipz, bsize, t0z == tce);
+    out.voxel[0] = (S.sign_bits & 1u) ? ~vx : vx;
+    out.voxel[1] = (S.sign_bits & 2u) ? ~vy : vy;
+    out.voxel[2] = (S.sign_bits & 4u) ? ~vz : vz;
+    out.t = tce;
+    out.node = S.node >> 8;
+    out.info = info;
+}
+
+} // namespace cqxd

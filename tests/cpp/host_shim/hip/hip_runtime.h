@@ -14,3 +14,9 @@ inline uint32_t __float_as_uint(float f)
     std::memcpy(&u, &f, 4);
     return u;
 }
+inline float __uint_as_float(uint32_t u)
+{
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
