@@ -12,8 +12,7 @@
 //   k_walk_lane / k_walk_persistent
 //                           the same two launches over a volume's packed copy (walk_packed.h),
 //                           taken by variants 1 and 2 with the full stack
-//   k_pack_nodes / k_pack_subdags
-//                           build and extend that copy
+//   k_pack_nodes            builds and extends that copy
 //   k_ray_bounds / k_bin_grid / k_bin_count / k_bin_columns / k_bin_scan / k_bin_scatter
 //                           optional prepass of the persistent variants: rays binned by origin
 //                           into a coarse Morton grid over the origins' bounds, handed out cell
@@ -416,8 +415,15 @@ __device__ __forceinline__ void setup_packed(PackedRay& S, const float* r)
     float v[6];
 #pragma unroll
     for (int i = 0; i < 6; i++) v[i] = __builtin_nontemporal_load(r + i);
-    ray_setup(S, v[0], v[1], v[2], v[3], v[4], v[5]);
-    S.plain = ray_plain(S) ? 1u : 0u;
+    ray_setup_packed(S, v[0], v[1], v[2], v[3], v[4], v[5]);
+}
+
+// The lane's stack_base(): its wave's `rows` rows of the workgroup's LDS, its own word of each.
+__device__ __forceinline__ uint32_t lane_stack(char* rows_lds, uint32_t rows, uint32_t top)
+{
+    // the low 32 bits of a generic LDS address are the LDS address
+    const uint32_t lds = uint32_t(reinterpret_cast<uintptr_t>(rows_lds));
+    return stack_base(lds + (threadIdx.x >> 6) * rows * kRowBytes + (threadIdx.x & 63u) * 4u, top);
 }
 
 // Up to `steps` steps of the wave's walking lanes: the plain rays' step when every walking lane may
@@ -448,8 +454,8 @@ __global__ void __launch_bounds__(256) k_walk_lane(PackedParams P, const cqx_ray
     }
     const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t base = (threadIdx.x >> 6) * (P.top + 1u) * kRowBytes + (threadIdx.x & 63u) * 4u;
-    const uint32_t occ = occupied_octants(P.sub);
+    const uint32_t base = lane_stack(lds_rows, P.top + 1u, P.top);
+    const uint32_t occ = P.sub[0].pad1;
     PackedRay S;
     setup_packed(S, reinterpret_cast<const float*>(rays + i));
     while (!is_finished(S.phase)) {
@@ -461,10 +467,17 @@ __global__ void __launch_bounds__(256) k_walk_lane(PackedParams P, const cqx_ray
     store_record(hits + i, h);
 }
 
+__device__ __forceinline__ uint64_t uniform64(uint64_t v)
+{
+    return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v)))) |
+           uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v >> 32)))) << 32;
+}
+
+// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take it to 6.
 template <typename Source, bool kLod>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6))) k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev,
-                                                         unsigned long long* __restrict__ counters, uint32_t regroup,
-                                                         uint32_t refill, uint32_t rows, uint32_t chunk)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6)))
+k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
+                  uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk)
 {
     extern __shared__ char lds_rows[];
     if (n_dev) {
@@ -474,31 +487,34 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source
     PackedParams P;
     cqx_hit* dst = nullptr;
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t base = (threadIdx.x >> 6) * rows * kRowBytes + lane * 4u;
+    uint32_t base;
+    if constexpr (Source::kUniform) base = lane_stack(lds_rows, rows, src.P.top);
+    else base = lane_stack(lds_rows, rows, src.top);
+
+    PackedRay S;
+    S.phase = kIdle;
+    __shared__ cqx_subdag lds_sub[8];
+    const cqx_subdag* tab = lds_sub;
+    uint32_t occ = 0u; // occupied octants of the launch's (a lane's) volume
+    if constexpr (Source::kUniform) {
+        occ = src.P.sub[0].pad1;
+        if (threadIdx.x < 8) lds_sub[threadIdx.x] = src.P.sub[threadIdx.x];
+        __syncthreads();
+    }
     const uint64_t per_q = (n + kQueues - 1) / kQueues;
     uint32_t qc = blockIdx.x % kQueues; // current queue
     uint32_t drained = 0;               // queues found empty so far
     uint64_t c_next = 0, c_end = 0;     // ray ids claimed by this wave
 
-    PackedRay S;
-    S.phase = kIdle;
-    uint32_t occ = 0xffu;
-    __shared__ cqx_subdag lds_sub[8];
-    if constexpr (Source::kUniform) {
-        occ = occupied_octants(src.P.sub);
-        if (threadIdx.x < 8) lds_sub[threadIdx.x] = src.P.sub[threadIdx.x];
-        __syncthreads();
-    }
-    const auto enter = [&](PackedRay& R) {
-        if constexpr (Source::kUniform) enter_octants_packed(lds_sub, src.P, R, lds_rows, base, occ);
-        else enter_octants_packed(P.sub, P, R, lds_rows, base, occ);
-    };
-
     for (;;) {
+        // A service pass runs once `refill` lanes wait, or none walks: misses of lanes that left their
+        // last SubDAG, records of the finished lanes, new rays for the idle ones, then the next SubDAG
+        // of every lane between SubDAGs (one copy of that code, for new and continuing rays; a ray
+        // that turns out to miss there has its record written by the next pass).
         const uint64_t walking = __ballot(S.phase == kWalk);
         const uint32_t nwait = 64u - uint32_t(__popcll(walking));
         if (nwait >= refill || walking == 0) {
-            enter(S);
+            resolve_leave(S, occ);
             if (is_finished(S.phase)) {
                 cqx_hit out;
                 emit_packed(uniform_params(src, P), S, out);
@@ -511,7 +527,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source
                 const uint64_t q_len = q_end > q_begin ? q_end - q_begin : 0;
                 unsigned long long claim = 0;
                 if (lane == 0) claim = atomicAdd(&counters[qc * kCounterStride], (unsigned long long)chunk);
-                claim = __shfl(claim, 0);
+                claim = uniform64(claim);
                 if (claim < q_len) {
                     c_next = q_begin + claim;
                     c_end = q_begin + (claim + chunk < q_len ? claim + chunk : q_len);
@@ -522,18 +538,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source
             }
             const uint64_t idle = __ballot(S.phase == kIdle);
             if (S.phase == kIdle) {
-                const uint32_t rank = uint32_t(__popcll(idle & ((1ull << lane) - 1ull)));
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
                 const uint64_t k = c_next + rank;
                 if (k < c_end) {
                     const float* r;
                     src.fetch(k, P, r, dst);
                     setup_packed(S, r);
-                    enter(S);
+                    if constexpr (!Source::kUniform) {
+                        tab = P.sub;
+                        occ = P.sub[0].pad1;
+                    }
                 }
             }
             const uint64_t nidle = uint64_t(__popcll(idle));
             c_next = c_next + nidle < c_end ? c_next + nidle : c_end;
             if (drained == kQueues && __ballot(S.phase != kIdle) == 0) break;
+            enter_octants_packed(tab, uniform_params(src, P), S, lds_rows, base, occ);
         }
         walk_burst<kLod>(uniform_params(src, P), S, lds_rows, base, regroup);
     }
@@ -548,9 +569,27 @@ __global__ void __launch_bounds__(256) k_pack_nodes(const uint32_t* __restrict__
     if (i < count) packed[first + i] = cqx::pack_child(nodes, nodes[first + i]);
 }
 
-__global__ void k_pack_subdags(const uint32_t* __restrict__ nodes, cqx_subdag* __restrict__ sub)
+__global__ void __launch_bounds__(64) k_pack_subdags(const uint32_t* __restrict__ nodes, cqx_subdag* __restrict__ sub)
 {
-    if (threadIdx.x < 8) sub[threadIdx.x].pad0 = cqx::pack_child(nodes, sub[threadIdx.x].node);
+    const uint32_t node = threadIdx.x < 8 ? sub[threadIdx.x].node : 0u;
+    const uint32_t occ = uint32_t(__ballot(node > 0));
+    if (threadIdx.x >= 8) return;
+    sub[threadIdx.x].pad0 = cqx::pack_child(nodes, node);
+    sub[threadIdx.x].pad1 = occ;
+}
+
+// The device copy of SubDAGs s: pad0 the packed word of each one's node, pad1 the occupied ones' mask.
+void device_subdags(const uint32_t* nodes, const cqx_subdag (&s)[8], cqx_subdag (&out)[8])
+{
+    uint32_t occ = 0;
+    for (int c = 0; c < 8; c++) {
+        out[c] = s[c];
+        uint32_t mask = 0;
+        for (int k = 0; k < 8; k++) mask |= (nodes[size_t(s[c].node) * 8 + k] ? 1u : 0u) << k;
+        out[c].pad0 = packed_word(s[c].node, mask);
+        occ |= (s[c].node ? 1u : 0u) << c;
+    }
+    for (cqx_subdag& d : out) d.pad1 = occ;
 }
 
 // ---- ray binning -------------------------------------------------------------------------------
@@ -852,12 +891,15 @@ cqx_status bin_rays(cqx_ctx* ctx, const cqx_ray* rays, uint64_t n, const BinBox&
 // `chunk`: ray ids a wave claims per atomic, about a 32nd of a wave's share (64 to 4096). Smaller
 // claims end the launch with less left over in single waves, and with the 8 per-XCD counters on
 // separate cache lines their atomics are cheap: a quarter of the share was 4-9 % slower.
-cqx_status persistent_shape(const cqx_ctx* ctx, const cqx_launch_cfg* cfg, uint32_t block, uint64_t n,
+// Defaults: the best launch of a sweep on the 1024^3 incoherent workload; the packed walk's steps do
+// more, and its service passes cost less, so it regroups every 12 steps (2.03 ms against 2.06 at 8), and
+// up to 2^23 rays runs 24 waves per CU (4.0 M rays at 4096^3: 1.03 ms against 1.09 at 32; 2^24 at 1024^3:
+// 2.14 against 2.04): the fewer waves share a SIMD, the sooner the last rays end.
+cqx_status persistent_shape(const cqx_ctx* ctx, const cqx_launch_cfg* cfg, uint32_t block, uint64_t n, bool packed,
                             uint32_t& blocks, uint32_t& regroup, uint32_t& refill, uint32_t& chunk)
 {
-    // built-in defaults: the best launch of a sweep on the 1024^3 incoherent workload
-    const uint32_t waves_per_cu = (cfg && cfg->waves_per_cu) ? cfg->waves_per_cu : 32u;
-    regroup = (cfg && cfg->regroup_interval) ? cfg->regroup_interval : 8u;
+    const uint32_t waves_per_cu = (cfg && cfg->waves_per_cu) ? cfg->waves_per_cu : packed && n <= (1u << 23) ? 24u : 32u;
+    regroup = (cfg && cfg->regroup_interval) ? cfg->regroup_interval : packed ? 12u : 8u;
     refill = (cfg && cfg->refill_lanes) ? cfg->refill_lanes : 16u;
     if (waves_per_cu > 64 || regroup > 4096 || refill > 64)
         return fail(CQX_ERR_INVALID_ARG, "persistent launch parameters out of range");
@@ -960,7 +1002,6 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
         if (words)
             hipLaunchKernelGGL(k_pack_nodes, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, 0, vol->nodes, vol->packed,
                                first * 8, words);
-        hipLaunchKernelGGL(k_pack_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, vol->sub);
         HIP_TRY(hipGetLastError());
     }
     vol->packed_ok = vol->packed && packed_eligible(vol->node_count, vol->hsub);
@@ -1048,7 +1089,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
         else hipLaunchKernelGGL(k_intersect_lane, dim3(uint32_t(blocks)), dim3(block), lds, stream, P, rays, n, n_dev, hits);
     } else if (variant == 5) {
         uint32_t blocks, regroup, refill, chunk;
-        cqx_status st = persistent_shape(ctx, cfg, block, (n + 1) / 2, blocks, regroup, refill, chunk);
+        cqx_status st = persistent_shape(ctx, cfg, block, (n + 1) / 2, false, blocks, regroup, refill, chunk);
         if (st != CQX_OK) return st;
         const size_t lds2 = 2 * lds;
         if (lds2 > size_t(ctx->lds_per_block))
@@ -1059,7 +1100,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
                            refill, rows, chunk);
     } else if (variant >= 2 && variant <= 4) {
         uint32_t blocks, regroup, refill, chunk;
-        cqx_status st = persistent_shape(ctx, cfg, block, n, blocks, regroup, refill, chunk);
+        cqx_status st = persistent_shape(ctx, cfg, block, n, packed, blocks, regroup, refill, chunk);
         if (st != CQX_OK) return st;
         uint32_t top_nodes = 0;
         size_t lds_total = lds;
@@ -1192,15 +1233,14 @@ cqx_status cqx_volume_upload(cqx_ctx* ctx, const uint32_t* nodes, uint64_t node_
         delete v;
         return fail(CQX_ERR_OOM, "device allocation of %zu bytes failed", bytes);
     }
-    if (hipMemcpy(v->nodes, nodes, bytes, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(v->sub, s, sizeof(s), hipMemcpyHostToDevice) != hipSuccess) {
-        release(v->nodes);
-        release(v->sub);
-        delete v;
-        return fail(CQX_ERR_HIP, "upload of the node store failed");
-    }
-    st = cqx::refresh_packed(ctx, v, 0);
-    if (st == CQX_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = fail(CQX_ERR_HIP, "packing the node store failed");
+    cqx_subdag ds[8];
+    device_subdags(nodes, s, ds);
+    st = hipMemcpy(v->nodes, nodes, bytes, hipMemcpyHostToDevice) == hipSuccess ? cqx::refresh_packed(ctx, v, 0)
+                                                                              : fail(CQX_ERR_HIP, "upload of the node store failed");
+    // (the copy is queued behind the packing: both are done when it returns)
+    if (st == CQX_OK && (hipMemcpy(v->sub, ds, sizeof(ds), hipMemcpyHostToDevice) != hipSuccess ||
+                         hipStreamSynchronize(nullptr) != hipSuccess))
+        st = fail(CQX_ERR_HIP, "upload of the SubDAGs failed");
     if (st != CQX_OK) {
         release(v->packed);
         release(v->nodes);
@@ -1263,6 +1303,7 @@ cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nod
         HIP_TRY(hipMemcpy(vol->nodes + first * 8, nodes + first * 8, size_t(node_count - first) * 32,
                           hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(vol->sub, s, sizeof(s), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_pack_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, vol->sub);
     const uint64_t kOffset32Nodes = uint64_t(1) << 27; // the child-offset width the traversal uses
     if (ctx->pt_plan && (old_nodes != vol->nodes || max_height != vol->max_height ||
                          (vol->node_count <= kOffset32Nodes) != (node_count <= kOffset32Nodes))) {
@@ -1442,7 +1483,7 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     HIP_TRY(hipMemcpy(ctx->batch_desc, packed ? static_cast<const void*>(pdesc.data()) : desc.data(), bytes,
                       hipMemcpyHostToDevice));
     uint32_t blocks, regroup, refill, chunk;
-    st = persistent_shape(ctx, cfg, block, total, blocks, regroup, refill, chunk);
+    st = persistent_shape(ctx, cfg, block, total, packed, blocks, regroup, refill, chunk);
     if (st != CQX_OK) return st;
     BatchSource src{ static_cast<const BatchDesc*>(ctx->batch_desc), n_batches,
                      (cfg && cfg->max_iters) ? cfg->max_iters : cqx::kDefaultMaxIters };

@@ -43,7 +43,7 @@ constexpr uint32_t kRowBytes = 64u * 4u;     // one stack row: a word per lane o
 
 struct PackedParams {
     const uint32_t* __restrict__ packed; // node_count x 8 packed words
-    const cqx_subdag* __restrict__ sub;  // 8 SubDAGs, pad0 holding the node's packed word
+    const cqx_subdag* __restrict__ sub;  // 8 SubDAGs: pad0 the node's packed word, pad1 the mask of the occupied ones
     uint32_t surf;
     uint32_t max_iters;
     uint32_t top;     // largest SubDAG height of the launch: the row of height h is top - h
@@ -101,7 +101,6 @@ struct PackedRay {
     float ox, oy, oz; // reflected, shifted origin
     float dx, dy, dz; // |direction|
     float ix, iy, iz; // 1 / |direction|
-    float distx, disty, distz;
     uint32_t sign_bits;
     uint32_t oct;
     uint32_t node;    // packed word of the current node
@@ -152,6 +151,20 @@ __device__ __forceinline__ float at_least_denorm(float x)
     return smax(bitsf(1u), x);
 #endif
 }
+// 1 / d correctly rounded for d in [1e-18, 1e18] (a normal result): the hardware's reciprocal (within
+// 1 ulp) and two Newton corrections by fused multiply-adds, the last one Markstein's correctly
+// rounding step; 24 issue cycles against 38 for the general division's scaling and fix-up. Equal to
+// the division for every float of that range (all 1.0e9 compared on the GPU).
+__device__ __forceinline__ float plain_rcp(float d)
+{
+#if defined(__AMDGCN__)
+    float r = __builtin_amdgcn_rcpf(d);
+    r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+    return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+#else
+    return 1.0f / d;
+#endif
+}
 // All bits set where a < b (0 otherwise), for a, b finite: with denormals a - b is negative exactly then.
 __device__ __forceinline__ uint32_t less_mask(float a, float b) { return uint32_t(int32_t(fbits(a - b)) >> 31); }
 
@@ -165,56 +178,163 @@ __device__ __forceinline__ bool ray_plain(const PackedRay& S)
     return (o <= 5.0e17f) & (d <= 1.0e18f) & (S.dx >= 1.0e-18f) & (S.dy >= 1.0e-18f) & (S.dz >= 1.0e-18f);
 }
 
-__device__ __forceinline__ uint32_t& stack_word(char* lds, uint32_t off) { return *reinterpret_cast<uint32_t*>(lds + off); }
+// The octants a ray crosses, in order (raytracing.cpp:424-434, :469-475).
+struct OctantChain {
+    float distx, disty, distz;
+    uint32_t oct;
+    uint32_t phase;
+};
 
-// Byte offset of the row of height `h` given the lane's base (its column's first row).
-__device__ __forceinline__ uint32_t packed_row(uint32_t base, uint32_t top, int32_t h) { return base + (top - uint32_t(h)) * kRowBytes; }
-
-// octant_enter of traverse_core.h. `base`: byte offset of the lane's stack column; `tab`: the 8
-// SubDAGs, their packed root words in pad0.
-__device__ __forceinline__ void octant_enter_packed(const cqx_subdag* tab, const PackedParams& P, PackedRay& S, char* lds,
-                                                    uint32_t base, uint32_t occ)
+__device__ __forceinline__ OctantChain octant_chain(const PackedRay& S)
 {
-    const uint32_t o = S.oct ^ S.sign_bits;
-    const cqx_subdag sd = ((occ >> o) & 1u) ? tab[o] : cqx_subdag{};
-    if (sd.node > 0) {
-        const int32_t sbx = S.sign_bits & 1u, sby = (S.sign_bits >> 1) & 1u, sbz = (S.sign_bits >> 2) & 1u;
-        const int32_t size = int32_t(1u << sd.height);
-        const int32_t px = wsub(wmul(sd.lower[0], 1 - 2 * sbx), wmul(sbx, size));
-        const int32_t py = wsub(wmul(sd.lower[1], 1 - 2 * sby), wmul(sby, size));
-        const int32_t pz = wsub(wmul(sd.lower[2], 1 - 2 * sbz), wmul(sbz, size));
-        const float nsz = float(size); // heights of a packed store are at most 22
-        const float entry = max3f((float(px) - S.ox) * S.ix, (float(py) - S.oy) * S.iy, (float(pz) - S.oz) * S.iz);
-        const float exitt = min3f(((float(px) + nsz) - S.ox) * S.ix, ((float(py) + nsz) - S.oy) * S.iy,
-                                  ((float(pz) + nsz) - S.oz) * S.iz);
-        if (entry < exitt) {
-            // ancestors not pushed yet read as node 0, as in the reference's zeroed stack
-            for (uint32_t r = P.top - uint32_t(sd.height); r <= P.top; r++) stack_word(lds, base + r * kRowBytes) = 0u;
-            S.sp = packed_row(base, P.top, sd.height);
-            S.zstart = 32u - uint32_t(sd.height);
-            S.node = uint32_t(sd.pad0);
-            const int32_t csize = int32_t(uint32_t(size) / 2u);
-            bool bx, by, bz;
-            S.cid = first_child(entry, S.ox, S.oy, S.oz, S.ix, S.iy, S.iz, wadd(px, csize), wadd(py, csize),
-                                wadd(pz, csize), bx, by, bz);
-            S.bx = kBias + float(wadd(px, bx ? csize : 0));
-            S.by = kBias + float(wadd(py, by ? csize : 0));
-            S.bz = kBias + float(wadd(pz, bz ? csize : 0));
-            S.s = float(csize);
-            S.last_exit = exitt;
-            S.entries++;
-            S.phase = kWalk;
-            return;
-        }
-    }
-    octant_advance(S);
+    OctantChain c;
+    c.distx = (-S.ox) / S.dx;
+    c.disty = (-S.oy) / S.dy;
+    c.distz = (-S.oz) / S.dz;
+    c.oct = 0;
+    if (c.distx < 0.0f) { c.oct += 1; c.distx += kFltMax; }
+    if (c.disty < 0.0f) { c.oct += 2; c.disty += kFltMax; }
+    if (c.distz < 0.0f) { c.oct += 4; c.distz += kFltMax; }
+    c.phase = kOctant;
+    return c;
 }
 
+// Ray setup, raytracing.cpp:415-434. The octant distances are not kept: only a ray that has to go on
+// to another octant needs them (octant_chain). A plain ray's first octant follows from the signs of
+// its origin (o > 0 exactly when (-o) / d < 0).
+__device__ __forceinline__ void ray_setup_packed(PackedRay& S, float rox, float roy, float roz, float rdx, float rdy,
+                                                 float rdz)
+{
+    const bool sbx = rdx < 0.0f, sby = rdy < 0.0f, sbz = rdz < 0.0f;
+    S.sign_bits = (sbx ? 1u : 0u) | (sby ? 2u : 0u) | (sbz ? 4u : 0u);
+    S.ox = (rox + 0.5f) * (sbx ? -1.0f : 1.0f);
+    S.oy = (roy + 0.5f) * (sby ? -1.0f : 1.0f);
+    S.oz = (roz + 0.5f) * (sbz ? -1.0f : 1.0f);
+    S.dx = fabsf(rdx);
+    S.dy = fabsf(rdy);
+    S.dz = fabsf(rdz);
+    S.entries = 0;
+    S.iters = 0;
+    S.phase = kOctant;
+    const bool plain = ray_plain(S);
+    S.plain = plain ? 1u : 0u;
+    if (plain) {
+        S.ix = plain_rcp(S.dx);
+        S.iy = plain_rcp(S.dy);
+        S.iz = plain_rcp(S.dz);
+        S.oct = (S.ox > 0.0f ? 1u : 0u) | (S.oy > 0.0f ? 2u : 0u) | (S.oz > 0.0f ? 4u : 0u);
+    } else {
+        S.ix = 1.0f / S.dx;
+        S.iy = 1.0f / S.dy;
+        S.iz = 1.0f / S.dz;
+        S.oct = octant_chain(S).oct;
+    }
+}
+
+// The stack word at byte offset `off`: on the GPU an LDS address (lds_address() + the offset in the
+// workgroup's rows), so that no base is added on each access; `lds` is the host's buffer.
+__device__ __forceinline__ void stack_store(char* lds, uint32_t off, uint32_t v)
+{
+#if defined(__AMDGCN__)
+    *reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(off) = v;
+#else
+    std::memcpy(lds + off, &v, 4);
+#endif
+}
+__device__ __forceinline__ uint32_t stack_load(const char* lds, uint32_t off)
+{
+#if defined(__AMDGCN__)
+    return *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>(off);
+#else
+    uint32_t v;
+    std::memcpy(&v, lds + off, 4);
+    return v;
+#endif
+}
+
+// A lane's stack base: row(h) = base + (32 - h) rows, for the column (first row) at `column`.
+__device__ __forceinline__ uint32_t stack_base(uint32_t column, uint32_t top) { return column + (top - 32u) * kRowBytes; }
+
+// Whether an occupied octant (occ: bit i for SubDAG i) can follow the ray's current one: a plain ray
+// crosses octants by setting bits of `oct`, one after the other, so only supersets of it are ahead.
+// Other rays: always true.
+__device__ __forceinline__ bool octants_ahead(const PackedRay& S, uint32_t occ)
+{
+    const uint32_t o = S.oct ^ S.sign_bits;
+    uint32_t m = occ & ~(1u << o);
+    m &= (S.oct & 1u) ? ((o & 1u) ? 0xaau : 0x55u) : 0xffu;
+    m &= (S.oct & 2u) ? ((o & 2u) ? 0xccu : 0x33u) : 0xffu;
+    m &= (S.oct & 4u) ? ((o & 4u) ? 0xf0u : 0x0fu) : 0xffu;
+    return !S.plain || m != 0;
+}
+
+// The slab test of the current octant's SubDAG and the walk's first child (raytracing.cpp:443-458,
+// :220-250); the phase becomes kWalk, or kLeave when the ray misses the SubDAG. `base`: the lane's
+// stack_base(); `tab`: the 8 SubDAGs with their packed root words (pad0).
+__device__ __forceinline__ void octant_enter_packed(const cqx_subdag* tab, const PackedParams& P, PackedRay& S, char* lds,
+                                                    uint32_t base)
+{
+    const cqx_subdag& sd = tab[S.oct ^ S.sign_bits];
+    const int32_t height = sd.height;
+    const float nsz = bitsf(uint32_t(127 + height) << 23); // 2^height
+    // reflected lower corner: lower, or -lower - size
+    const float lx = float(sd.lower[0]), ly = float(sd.lower[1]), lz = float(sd.lower[2]);
+    const float px = (S.sign_bits & 1u) ? -lx - nsz : lx, py = (S.sign_bits & 2u) ? -ly - nsz : ly,
+                pz = (S.sign_bits & 4u) ? -lz - nsz : lz;
+    const float entry = max3f((px - S.ox) * S.ix, (py - S.oy) * S.iy, (pz - S.oz) * S.iz);
+    const float exitt = min3f(((px + nsz) - S.ox) * S.ix, ((py + nsz) - S.oy) * S.iy, ((pz + nsz) - S.oz) * S.iz);
+    S.phase = kLeave;
+    if (!(entry < exitt)) return;
+    // ancestors not pushed yet read as node 0, as in the reference's zeroed stack
+    for (uint32_t r = 32u - P.top; r <= 32u; r++) stack_store(lds, base + r * kRowBytes, 0u);
+    S.zstart = 32u - uint32_t(height);
+    S.sp = base + S.zstart * kRowBytes;
+    S.node = sd.pad0;
+    const float half = height > 0 ? nsz * 0.5f : 0.0f;
+    const float cx = px + half, cy = py + half, cz = pz + half;
+    const bool behind = entry <= 0.0f; // findFirstChild, raytracing.cpp:178-196
+    const bool bx = ((cx - S.ox) * S.ix < entry) | (behind & (S.ox >= cx));
+    const bool by = ((cy - S.oy) * S.iy < entry) | (behind & (S.oy >= cy));
+    const bool bz = ((cz - S.oz) * S.iz < entry) | (behind & (S.oz >= cz));
+    S.cid = (bx ? 1u : 0u) | (by ? 2u : 0u) | (bz ? 4u : 0u);
+    S.bx = kBias + (bx ? cx : px);
+    S.by = kBias + (by ? cy : py);
+    S.bz = kBias + (bz ? cz : pz);
+    S.s = half;
+    S.last_exit = exitt;
+    S.entries++;
+    S.phase = kWalk;
+}
+
+// Moves a lane that is between SubDAGs (kOctant: at its current octant; kLeave: past it) into the walk
+// of the next SubDAG it enters, or to the end of its walk.
 __device__ __forceinline__ void enter_octants_packed(const cqx_subdag* tab, const PackedParams& P, PackedRay& S, char* lds,
                                                      uint32_t base, uint32_t occ)
 {
-    if (S.phase == kLeave) octant_advance(S);
-    while (S.phase == kOctant) octant_enter_packed(tab, P, S, lds, base, occ);
+    while (S.phase == kOctant || S.phase == kLeave) {
+        if (S.phase == kLeave || !((occ >> (S.oct ^ S.sign_bits)) & 1u)) {
+            if (!octants_ahead(S, occ)) {
+                S.phase = kMiss;
+            } else {
+                OctantChain c = octant_chain(S); // replayed up to the current octant: the same steps
+                while (c.oct < S.oct && c.phase == kOctant) octant_advance(c);
+                do octant_advance(c);
+                while (c.phase == kOctant && !((occ >> (c.oct ^ S.sign_bits)) & 1u));
+                S.oct = c.oct;
+                S.phase = c.phase;
+            }
+        }
+        if (S.phase == kOctant) octant_enter_packed(tab, P, S, lds, base);
+    }
+}
+
+// What a service pass does first for a lane that left its SubDAG: with no occupied octant ahead its
+// walk is a miss, and its record can be written in the same pass.
+__device__ __forceinline__ void resolve_leave(PackedRay& S, uint32_t occ)
+{
+    if (S.phase != kLeave) return;
+    // the usual volume has one occupied octant: the one just left
+    if ((occ & (occ - 1u)) == 0 ? S.plain != 0 : !octants_ahead(S, occ)) S.phase = kMiss;
 }
 
 // The occupied child's word: slot cid ^ signBits of the current node.
@@ -235,8 +355,7 @@ __device__ __forceinline__ float packed_exits(const PackedRay& S, float& t1x, fl
 
 // Pop to the highest boundary crossed (raytracing.cpp:339-364); obx.. the position before the
 // advance. False when the walk left the SubDAG.
-__device__ __forceinline__ bool packed_pop(PackedRay& S, char* lds, uint32_t base, uint32_t top, float obx, float oby,
-                                           float obz)
+__device__ __forceinline__ bool packed_pop(PackedRay& S, char* lds, uint32_t base, float obx, float oby, float obz)
 {
     const uint32_t ux = fbits(S.bx), uy = fbits(S.by), uz = fbits(S.bz);
     const uint32_t diff = (ux ^ fbits(obx)) | (uy ^ fbits(oby)) | (uz ^ fbits(obz));
@@ -245,8 +364,8 @@ __device__ __forceinline__ bool packed_pop(PackedRay& S, char* lds, uint32_t bas
         S.phase = kLeave;
         return false;
     }
-    S.sp = base + (top - 32u) * kRowBytes + z * kRowBytes;
-    S.node = stack_word(lds, S.sp);
+    S.sp = base + z * kRowBytes;
+    S.node = stack_load(lds, S.sp);
     const uint32_t keep = uint32_t(int32_t(0x80000000u) >> z); // clears the bits below the boundary's
     const uint32_t m = 31u - z;
     S.cid = ((ux >> m) & 1u) | (((uy >> m) & 1u) << 1) | (((uz >> m) & 1u) << 2);
@@ -281,7 +400,7 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
         const uint32_t flips = (fx & 1u) | (fy & 2u) | (fz & 4u);
         const uint32_t carry = S.cid & flips;
         S.cid ^= flips;
-        if (carry && !packed_pop(S, lds, base, P.top, obx, oby, obz)) return;
+        if (carry && !packed_pop(S, lds, base, obx, oby, obz)) return;
         tcx = packed_exits(S, t1x, t1y, t1z);
         slot = S.cid ^ S.sign_bits;
         occupied = (S.node >> slot) & 1u;
@@ -305,7 +424,7 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
                 S.phase = kAnomaly; // deeper than a valid DAG
                 return;
             }
-            if (tcx < S.last_exit) stack_word(lds, S.sp) = S.node;
+            if (tcx < S.last_exit) stack_store(lds, S.sp, S.node);
             S.last_exit = tcx;
             S.sp += kRowBytes;
             S.node = child;
@@ -354,7 +473,7 @@ __device__ __forceinline__ void walk_step_packed_any(const PackedParams& P, Pack
             return;
         }
         const float tce = max3f((px - S.ox) * S.ix, (py - S.oy) * S.iy, (pz - S.oz) * S.iz);
-        if (tcx < S.last_exit) stack_word(lds, S.sp) = S.node;
+        if (tcx < S.last_exit) stack_store(lds, S.sp, S.node);
         S.last_exit = tcx;
         S.sp += kRowBytes;
         S.node = child;
@@ -379,7 +498,16 @@ __device__ __forceinline__ void walk_step_packed_any(const PackedParams& P, Pack
     S.bz = obz + ((flips & 4u) ? S.s : 0.0f);
     const uint32_t carry = S.cid & flips;
     S.cid ^= flips;
-    if (carry) packed_pop(S, lds, base, P.top, obx, oby, obz);
+    if (carry) packed_pop(S, lds, base, obx, oby, obz);
+}
+
+// First voxel of the hit block entered by a plain ray (entered_voxel of traverse_core.h): floor(o + d t)
+// clamped to the block, as floats (exact integers below 2^23).
+__device__ __forceinline__ uint32_t entered_voxel_plain(float o, float d, float t, float lo, float hi, bool entry_axis)
+{
+    const float q = floorf(o + d * t);
+    const float c = smin(smax(q, lo), hi);
+    return fbits((entry_axis ? lo : c) + kBias) - kBiasBits;
 }
 
 // Record of a finished ray: emit_record of traverse_core.h from the packed walk's state. The
@@ -389,17 +517,15 @@ __device__ __forceinline__ void emit_packed(const PackedParams& P, const PackedR
     result_miss(out);
     out.entries = S.entries;
     out.iters = S.iters;
-    if (S.phase == kAnomaly) {
-        out.info = CQX_HIT_ANOMALY;
-        return;
-    }
+    out.info = S.phase == kAnomaly ? CQX_HIT_ANOMALY : 0u;
     if (S.phase != kHit) return;
     const uint32_t slot = S.cid ^ S.sign_bits;
     const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
     const float t0x = (px - S.ox) * S.ix, t0y = (py - S.oy) * S.iy, t0z = (pz - S.oz) * S.iz;
     const float tce = max3f(t0x, t0y, t0z);
-    const int32_t bsize = S.s > 0.0f ? int32_t(S.s) : 1; // a SubDAG of height 0: the node itself, of side 1
-    uint32_t info = 1u | (slot << 1) | (uint32_t(find_msb(uint32_t(bsize))) << 4);
+    const bool ex = tce == t0x, ey = tce == t0y, ez = tce == t0z;
+    const float bsize = S.s > 0.0f ? S.s : 1.0f; // a SubDAG of height 0: the node itself, of side 1
+    uint32_t info = 1u | (slot << 1) | (((fbits(bsize) >> 23) - 127u) << 4);
     if (P.surf) {
         uint32_t m = S.word;
         uint32_t entries = S.entries;
@@ -417,23 +543,29 @@ __device__ __forceinline__ void emit_packed(const PackedParams& P, const PackedR
                                                    (((m >> 3) & ~31u) | ((ids & 7u) << 2)));
         }
         out.entries = entries;
-        // normal = vec3(equal(tEntry, childT0)) * -rayDirSign, raytracing.cpp:317-318
-        const float sx = (S.sign_bits & 1u) ? -1.0f : 1.0f, sy = (S.sign_bits & 2u) ? -1.0f : 1.0f,
-                    sz = (S.sign_bits & 4u) ? -1.0f : 1.0f;
-        const float nx = float(tce == t0x) * -sx, ny = float(tce == t0y) * -sy, nz = float(tce == t0z) * -sz;
-        info |= ((nx != 0.0f ? 1u : 0u) | ((fbits(nx) >> 31) << 1)) << 9;
-        info |= ((ny != 0.0f ? 1u : 0u) | ((fbits(ny) >> 31) << 1)) << 11;
-        info |= ((nz != 0.0f ? 1u : 0u) | ((fbits(nz) >> 31) << 1)) << 13;
+        // normal = vec3(equal(tEntry, childT0)) * -rayDirSign, raytracing.cpp:317-318: magnitude 1 on
+        // the entry axes, and the sign bit of -rayDirSign on every axis (0 * -1 = -0)
+        info |= (ex ? 1u << 9 : 0u) | (ey ? 1u << 11 : 0u) | (ez ? 1u << 13 : 0u);
+        info |= (S.sign_bits & 1u) ? 0u : 1u << 10;
+        info |= (S.sign_bits & 2u) ? 0u : 1u << 12;
+        info |= (S.sign_bits & 4u) ? 0u : 1u << 14;
         info |= (m >> 8) << 16;
     }
-    const int32_t ipx = int32_t(fbits(S.bx) - kBiasBits), ipy = int32_t(fbits(S.by) - kBiasBits),
-                  ipz = int32_t(fbits(S.bz) - kBiasBits);
-    const int32_t vx = entered_voxel(S.ox, S.dx, tce, ipx, bsize, t0x == tce);
-    const int32_t vy = entered_voxel(S.oy, S.dy, tce, ipy, bsize, t0y == tce);
-    const int32_t vz = entered_voxel(S.oz, S.dz, tce, ipz, bsize, t0z == tce);
-    out.voxel[0] = (S.sign_bits & 1u) ? ~vx : vx;
-    out.voxel[1] = (S.sign_bits & 2u) ? ~vy : vy;
-    out.voxel[2] = (S.sign_bits & 4u) ? ~vz : vz;
+    uint32_t vx, vy, vz;
+    if (S.plain) {
+        const float ext = bsize - 1.0f;
+        vx = entered_voxel_plain(S.ox, S.dx, tce, px, px + ext, ex);
+        vy = entered_voxel_plain(S.oy, S.dy, tce, py, py + ext, ey);
+        vz = entered_voxel_plain(S.oz, S.dz, tce, pz, pz + ext, ez);
+    } else {
+        const int32_t size = int32_t(bsize);
+        vx = uint32_t(entered_voxel(S.ox, S.dx, tce, int32_t(px), size, ex));
+        vy = uint32_t(entered_voxel(S.oy, S.dy, tce, int32_t(py), size, ey));
+        vz = uint32_t(entered_voxel(S.oz, S.dz, tce, int32_t(pz), size, ez));
+    }
+    out.voxel[0] = int32_t(vx ^ (0u - (S.sign_bits & 1u)));
+    out.voxel[1] = int32_t(vy ^ (0u - ((S.sign_bits >> 1) & 1u)));
+    out.voxel[2] = int32_t(vz ^ (0u - (S.sign_bits >> 2)));
     out.t = tce;
     out.node = S.node >> 8;
     out.info = info;

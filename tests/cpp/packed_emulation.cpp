@@ -69,21 +69,22 @@ int main(int argc, char** argv)
     const uint64_t n = rb.size() / 24;
     std::vector<cqx_hit> out(n);
     std::vector<char> stack(33 * kRowBytes);
+    const uint32_t base = stack_base(0u, P.top);
     uint64_t plain = 0;
     for (uint64_t i = 0; i < n; i++) {
         PackedRay S{};
         const float* r = rays + 6 * i;
-        ray_setup(S, r[0], r[1], r[2], r[3], r[4], r[5]);
-        const bool fast = !any && ray_plain(S);
+        ray_setup_packed(S, r[0], r[1], r[2], r[3], r[4], r[5]);
+        const bool fast = !any && S.plain;
         plain += fast;
         while (!is_finished(S.phase)) {
-            enter_octants_packed(sub, P, S, stack.data(), 0, occ);
+            enter_octants_packed(sub, P, S, stack.data(), base, occ);
             while (S.phase == kWalk) {
                 if (fast && P.max_iters >= 2 && S.iters <= P.max_iters - 2) {
-                    if (lod) walk_step_packed<true>(P, S, stack.data(), 0);
-                    else walk_step_packed<false>(P, S, stack.data(), 0);
+                    if (lod) walk_step_packed<true>(P, S, stack.data(), base);
+                    else walk_step_packed<false>(P, S, stack.data(), base);
                 } else {
-                    walk_step_packed_any(P, S, stack.data(), 0);
+                    walk_step_packed_any(P, S, stack.data(), base);
                 }
             }
         }
