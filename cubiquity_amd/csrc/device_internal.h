@@ -105,12 +105,21 @@ __device__ __forceinline__ uint32_t pack_child(const uint32_t* __restrict__ node
     return cqxd::packed_word(child, mask);
 }
 
+// Ids per wave of a launch of at most n secondary rays whose count is on the device (launch_intersect's
+// `dealt`).
+uint32_t dealt_ids(uint64_t n);
+
+// Whether the caller left every field open that shapes a launch (cfg null or those fields zero).
+bool launch_open(const cqx_launch_cfg* cfg);
+
 // Launches the traversal of `n` rays (or of *n_dev rays, at most n, when n_dev is not null).
 // Counters and binning buffers are the context's, or `sv`'s when it is given (then nothing is
-// allocated).
+// allocated). `dealt` != 0, on a packed volume: that many ids per wave, dealt at launch (up to 64: one
+// ray per lane), whatever cfg says of the shape.
 cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray* rays, uint64_t n,
                             const uint32_t* n_dev, uint32_t flags, float max_footprint, cqx_hit* hits,
-                            const cqx_launch_cfg* cfg, hipStream_t stream, const ScratchView* sv = nullptr);
+                            const cqx_launch_cfg* cfg, hipStream_t stream, const ScratchView* sv = nullptr,
+                            uint32_t dealt = 0);
 
 // Threads per block of the kernels that compact lists with block_slots.
 constexpr uint32_t kCompactBlock = 1024;

@@ -9,9 +9,9 @@
 //                           global counter with one atomic, handed out by ballot prefix
 //                           (variant 2); variant 3 also keeps the current node's 8 children in
 //                           registers
-//   k_walk_lane / k_walk_persistent
-//                           the same two launches over a volume's packed copy (walk_packed.h),
-//                           taken by variants 1 and 2 with the full stack
+//   k_walk                  the same two launches over a volume's packed copy (walk_packed.h), taken
+//                           by variants 1 and 2 with the full stack
+//   k_sample_rays           whether a batch's rays are coherent, for the launches gated on it
 //   k_pack_nodes            builds and extends that copy
 //   k_ray_bounds / k_bin_grid / k_bin_count / k_bin_columns / k_bin_scan / k_bin_scatter
 //                           optional prepass of the persistent variants: rays binned by origin
@@ -67,6 +67,8 @@ __global__ void __launch_bounds__(256) k_intersect_lane(TraceParams P, const cqx
 // exits when every queue is drained and all its lanes are idle.
 constexpr int kQueues = 8;
 constexpr int kCounterStride = 16; // queue counters 128 bytes apart: one cache line each
+constexpr int kFlagWord = 8;       // the sampled flag of gated launches, in the first counter's line
+static_assert(kFlagWord < kCounterStride && kFlagWord % kCounterStride != 0, "a word no counter uses");
 
 __global__ void k_reset_counters(unsigned long long* counters)
 {
@@ -348,9 +350,8 @@ __global__ void __launch_bounds__(256) k_intersect_pair(SingleSource src, uint64
 }
 
 // ---- the packed walk ---------------------------------------------------------------------------
-// k_walk_lane and k_walk_persistent are k_intersect_lane and k_intersect_persistent on a volume's
-// packed copy (walk_packed.h): the same launches (variants 1 and 2) with the same records, taken
-// whenever every volume of the launch has one.
+// k_walk serves the launches of k_intersect_lane and k_intersect_persistent (variants 1 and 2) on a
+// volume's packed copy (walk_packed.h) with the same records, whenever every volume of the launch has one.
 
 struct PackedSingle {
     static constexpr bool kUniform = true;
@@ -443,43 +444,26 @@ __device__ __forceinline__ void walk_burst(const PackedParams& P, PackedRay& S, 
     }
 }
 
-template <bool kLod>
-__global__ void __launch_bounds__(256) k_walk_lane(PackedParams P, const cqx_ray* __restrict__ rays, uint64_t n,
-                                                   const uint32_t* __restrict__ n_dev, cqx_hit* __restrict__ hits)
-{
-    extern __shared__ char lds_rows[];
-    if (n_dev) {
-        const uint64_t nd = *n_dev;
-        n = nd < n ? nd : n;
-    }
-    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t base = lane_stack(lds_rows, P.top + 1u, P.top);
-    const uint32_t occ = P.sub[0].pad1;
-    PackedRay S;
-    setup_packed(S, reinterpret_cast<const float*>(rays + i));
-    while (!is_finished(S.phase)) {
-        enter_octants_packed(P.sub, P, S, lds_rows, base, occ);
-        while (S.phase == kWalk) walk_burst<kLod>(P, S, lds_rows, base, 8u);
-    }
-    cqx_hit h;
-    emit_packed(P, S, h);
-    store_record(hits + i, h);
-}
-
 __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 {
     return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v)))) |
            uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v >> 32)))) << 32;
 }
 
+// What a wave does is the same in both forms; they differ in where its ray ids come from.
+//   dealt (kDealt)  wave w owns ids [w * chunk, (w + 1) * chunk): no counters, no claims, the hardware's
+//                   dispatcher balances the load. With chunk <= 64 and refill 64 it is one ray per lane.
+//   claimed         persistent waves claim `chunk` ids at a time from the queues' counters
+// `gate`: a launch that runs only when the sampled flag there equals `want` (k_sample_rays).
 // At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take it to 6.
-template <typename Source, bool kLod>
+template <typename Source, bool kLod, bool kDealt>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6)))
-k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
-                  uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk)
+k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
+       uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk, const unsigned long long* __restrict__ gate,
+       uint32_t want)
 {
     extern __shared__ char lds_rows[];
+    if (gate && *gate != want) return;
     if (n_dev) {
         const uint64_t nd = *n_dev;
         n = nd < n ? nd : n;
@@ -505,6 +489,13 @@ k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, un
     uint32_t qc = blockIdx.x % kQueues; // current queue
     uint32_t drained = 0;               // queues found empty so far
     uint64_t c_next = 0, c_end = 0;     // ray ids claimed by this wave
+    if constexpr (kDealt) {
+        const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+        const uint64_t at = (uint64_t(blockIdx.x) * (blockDim.x >> 6) + wave) * chunk;
+        c_next = at < n ? at : n;
+        c_end = at + chunk < n ? at + chunk : n;
+        drained = kQueues;
+    }
 
     for (;;) {
         // A service pass runs once `refill` lanes wait, or none walks: misses of lanes that left their
@@ -553,11 +544,37 @@ k_walk_persistent(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, un
             }
             const uint64_t nidle = uint64_t(__popcll(idle));
             c_next = c_next + nidle < c_end ? c_next + nidle : c_end;
-            if (drained == kQueues && __ballot(S.phase != kIdle) == 0) break;
+            if (drained == kQueues && c_next == c_end && __ballot(S.phase != kIdle) == 0) break;
             enter_octants_packed(tab, uniform_params(src, P), S, lds_rows, base, occ);
         }
         walk_burst<kLod>(uniform_params(src, P), S, lds_rows, base, regroup);
     }
+}
+
+// Whether a batch's rays are coherent (camera rays, sun shadow rays): of 64 pairs of neighbouring rays
+// spread over the array, at least 56 have nearly equal directions (cosine above 0.97) and origins
+// within a 16th of the largest SubDAG's side of each other.
+__device__ __forceinline__ bool rays_coherent(const cqx_ray* rays, uint64_t n, uint32_t top)
+{
+    if (n < 128) return false;
+    const uint64_t i = (n / 64u) * (threadIdx.x & 63u);
+    const float* a = reinterpret_cast<const float*>(rays + i);
+    const float* b = a + 6;
+    const float ox = a[0] - b[0], oy = a[1] - b[1], oz = a[2] - b[2];
+    const float near = bitsf((127u + top) << 23) * 0.0625f;
+    const float dot = (a[3] * b[3] + a[4] * b[4]) + a[5] * b[5];
+    const float aa = (a[3] * a[3] + a[4] * a[4]) + a[5] * a[5], bb = (b[3] * b[3] + b[4] * b[4]) + b[5] * b[5];
+    const bool same = dot > 0.0f && dot * dot > 0.94f * (aa * bb) && (ox * ox + oy * oy) + oz * oz < near * near;
+    return __popcll(__ballot(same)) >= 56;
+}
+
+// One wave: the queue counters cleared, and the batch's coherence where the gated launches read it.
+__global__ void __launch_bounds__(64) k_sample_rays(unsigned long long* counters, const cqx_ray* __restrict__ rays,
+                                                    uint64_t n, uint32_t top)
+{
+    if (threadIdx.x < kQueues) counters[threadIdx.x * kCounterStride] = 0;
+    const bool coherent = rays_coherent(rays, n, top);
+    if (threadIdx.x == 0) counters[kFlagWord] = coherent ? 1u : 0u;
 }
 
 // Packed words of store words [first, first + count): each child's index and the occupancy mask of
@@ -1013,9 +1030,84 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
     return CQX_OK;
 }
 
+// The shape of an open launch on a packed volume, by its size. What each line rests on (MI355X, us,
+// incoherent / camera rays at 1024^3 unless stated; K: ids per wave in 64s with refill 16, lane: 64 per
+// wave without refill, p: claimed by persistent waves):
+//   n                lane          K = 2         K = 4         p
+//   921600           272 / 138     256 / 173     268 / 275     278 / 224
+//   2.0 M            504 / 196     440 / 219     396 / 299     419 / 306
+//   4.0 M (4096^3)   1496          1259          1157          1037
+//   8.0 M            / 439         / 468         / 494         / 717
+//   2^24             3615          2918          2393          2035
+// Up to kLaneRays one ray per lane: close to the best for either kind. Beyond, the kinds part: a sample
+// of the rays decides on the device between one ray per lane for coherent ones and, for the others,
+// dealt runs of 4 x 64 up to kDealtRays, claims by persistent waves past it (whose tail no longer
+// matters there). The sample and the launch that returns at once take about 10 us.
+constexpr uint64_t kLaneRays = 1u << 20;
+constexpr uint64_t kDealtRays = 5u << 19; // 2.6 M
+constexpr uint64_t kGateRays = uint64_t(1) << 31; // the lane launch's grid stays below 2^32 threads
+
+// Rays per wave of a one-ray-per-lane launch. A lone wave on a SIMD issues an instruction every 6
+// cycles against 2 to 4 with company, and a wave with fewer rays takes fewer of a step's paths, so a
+// batch that cannot fill the chip is spread: at most 4 rays per wave up to 4096 waves, then 2048 waves
+// (two per SIMD) up to 64. Measured (us, spread / 64 per wave, 1024^3): 64 rays 51 / 66, 1024 66 / 73,
+// 8192 80 / 100, 65536 108 / 120.
+uint32_t lanes_per_wave(uint64_t n)
+{
+    uint32_t g = 1;
+    while (g < 64 && uint64_t(g) * (g < 4 ? 4096 : 2048) < n) g *= 2;
+    return g;
+}
+
+// Ids per wave of a launch over secondary rays (path-tracer bounces, shadow rays) whose count, at most
+// n and usually half of it, is known on the device only: neighbours start near each other, so that
+// short runs hold longer than for random rays, and no counters are cleared and claimed between two
+// launches. Frame times (ms) at K = 64, 128, 256 ids per wave, and claimed by 24 waves per CU: 2.1 M
+// paths 512^3 adjoint 0.85 / 0.89 / 1.01 / 1.08, 4.9 M at 512^3 1.02 / 1.04 / 1.10 / 1.17, 7.4 M at 1024^3
+// 1.79 / 1.75 / 1.84, 14.7 M at 1024^3 3.07 / 2.87 / 2.79 / 2.78.
+uint32_t dealt_ids(uint64_t n)
+{
+    return n <= (1u << 22) ? lanes_per_wave(n) : n <= (1u << 23) ? 128u : 256u;
+}
+
+bool launch_open(const cqx_launch_cfg* c)
+{
+    return !c || (!c->variant && !c->block && !c->waves_per_cu && !c->regroup_interval && !c->refill_lanes &&
+                  !c->bin_bits && !c->stack_rows);
+}
+
+namespace {
+
+// k_walk over one volume, dealt (chunk ids per wave) or claimed.
+template <bool kDealt>
+void launch_walk(const PackedSingle& src, bool lod, uint64_t blocks, uint32_t block, hipStream_t stream, uint64_t n,
+                 const uint32_t* n_dev, unsigned long long* counters, uint32_t regroup, uint32_t refill, uint32_t chunk,
+                 const unsigned long long* gate = nullptr, uint32_t want = 0)
+{
+    const uint32_t rows = src.P.top + 1u;
+    const size_t lds = size_t(rows) * block * sizeof(uint32_t);
+    if (lod)
+        hipLaunchKernelGGL((k_walk<PackedSingle, true, kDealt>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
+                           n_dev, counters, regroup, refill, rows, chunk, gate, want);
+    else
+        hipLaunchKernelGGL((k_walk<PackedSingle, false, kDealt>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
+                           n_dev, counters, regroup, refill, rows, chunk, gate, want);
+}
+
+// Dealt, `chunk` ids per wave: up to 64, one ray per lane; more, with refills.
+void launch_dealt(const PackedSingle& src, bool lod, uint32_t block, hipStream_t stream, uint64_t n, const uint32_t* n_dev,
+                  uint32_t chunk, const unsigned long long* gate = nullptr, uint32_t want = 0)
+{
+    const uint64_t per_block = uint64_t(block / 64) * chunk;
+    launch_walk<true>(src, lod, (n + per_block - 1) / per_block, block, stream, n, n_dev, nullptr, 12u,
+                      chunk > 64 ? 16u : 64u, chunk, gate, want);
+}
+
+} // namespace
+
 cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray* rays, uint64_t n,
                             const uint32_t* n_dev, uint32_t flags, float max_footprint, cqx_hit* hits,
-                            const cqx_launch_cfg* cfg, hipStream_t stream, const ScratchView* sv)
+                            const cqx_launch_cfg* cfg, hipStream_t stream, const ScratchView* sv, uint32_t dealt)
 {
     unsigned long long* const counters =
         reinterpret_cast<unsigned long long*>(sv ? sv->counters : static_cast<void*>(ctx->d_counter));
@@ -1077,16 +1169,32 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
             if (bst != CQX_OK) return bst;
         }
     }
-    if (variant == 1) {
+    if (packed) {
+        const PackedSingle src{ PP, rays, hits, order };
+        const bool open = launch_open(cfg);
+        uint32_t blocks = 0, regroup = 0, refill = 0, chunk = 0;
+        if (variant == 2) {
+            const cqx_status st = persistent_shape(ctx, cfg, block, n, true, blocks, regroup, refill, chunk);
+            if (st != CQX_OK) return st;
+        }
+        if (variant == 1 && (n + block - 1) / block > 0x7fffffffull) return fail(CQX_ERR_LIMIT, "too many rays for one launch");
+        if (dealt) launch_dealt(src, lod, 64u, stream, n, n_dev, dealt);
+        else if (variant == 1) launch_dealt(src, lod, block, stream, n, n_dev, lanes_per_wave(n));
+        else if (open && n <= kLaneRays) launch_dealt(src, lod, 64u, stream, n, n_dev, lanes_per_wave(n));
+        else if (open && !n_dev && n < kGateRays) {
+            const unsigned long long* const flag = counters + kFlagWord;
+            hipLaunchKernelGGL(k_sample_rays, dim3(1), dim3(64), 0, stream, counters, rays, n, PP.top);
+            launch_dealt(src, lod, 256u, stream, n, nullptr, 64u, flag, 1u);
+            if (n <= kDealtRays) launch_dealt(src, lod, 64u, stream, n, nullptr, 256u, flag, 0u);
+            else launch_walk<false>(src, lod, blocks, block, stream, n, nullptr, counters, regroup, refill, chunk, flag, 0u);
+        } else {
+            hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, stream, counters);
+            launch_walk<false>(src, lod, blocks, block, stream, n, n_dev, counters, regroup, refill, chunk);
+        }
+    } else if (variant == 1) {
         const uint64_t blocks = (n + block - 1) / block;
         if (blocks > 0x7fffffffull) return fail(CQX_ERR_LIMIT, "too many rays for one launch");
-        if (packed && lod)
-            hipLaunchKernelGGL(k_walk_lane<true>, dim3(uint32_t(blocks)), dim3(block), lds, stream, PP, rays, n, n_dev,
-                               hits);
-        else if (packed)
-            hipLaunchKernelGGL(k_walk_lane<false>, dim3(uint32_t(blocks)), dim3(block), lds, stream, PP, rays, n, n_dev,
-                               hits);
-        else hipLaunchKernelGGL(k_intersect_lane, dim3(uint32_t(blocks)), dim3(block), lds, stream, P, rays, n, n_dev, hits);
+        hipLaunchKernelGGL(k_intersect_lane, dim3(uint32_t(blocks)), dim3(block), lds, stream, P, rays, n, n_dev, hits);
     } else if (variant == 5) {
         uint32_t blocks, regroup, refill, chunk;
         cqx_status st = persistent_shape(ctx, cfg, block, (n + 1) / 2, false, blocks, regroup, refill, chunk);
@@ -1100,7 +1208,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
                            refill, rows, chunk);
     } else if (variant >= 2 && variant <= 4) {
         uint32_t blocks, regroup, refill, chunk;
-        cqx_status st = persistent_shape(ctx, cfg, block, n, packed, blocks, regroup, refill, chunk);
+        cqx_status st = persistent_shape(ctx, cfg, block, n, false, blocks, regroup, refill, chunk);
         if (st != CQX_OK) return st;
         uint32_t top_nodes = 0;
         size_t lds_total = lds;
@@ -1115,14 +1223,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
             return fail(CQX_ERR_LIMIT, "stack and SubDAG copy need %zu B of LDS per block", lds_total + kSubdagCopyBytes);
         SingleSource src{ P, rays, hits, order };
         hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, stream, counters);
-        const PackedSingle psrc{ PP, rays, hits, order };
-        if (packed && lod)
-            hipLaunchKernelGGL((k_walk_persistent<PackedSingle, true>), dim3(blocks), dim3(block), lds, stream, psrc, n,
-                               n_dev, counters, regroup, refill, rows, chunk);
-        else if (packed)
-            hipLaunchKernelGGL((k_walk_persistent<PackedSingle, false>), dim3(blocks), dim3(block), lds, stream, psrc, n,
-                               n_dev, counters, regroup, refill, rows, chunk);
-        else if (variant == 2 && short_stack)
+        if (variant == 2 && short_stack)
             hipLaunchKernelGGL((k_intersect_persistent<SingleSource, false, false, true>), dim3(blocks), dim3(block), lds,
                                stream, src, n, n_dev, counters, regroup, refill, rows, 0u, chunk);
         else if (variant == 3 && short_stack)
@@ -1492,11 +1593,13 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     const bool cache = cfg && cfg->variant == 3;
     const PackedBatch psrc{ static_cast<const PackedDesc*>(ctx->batch_desc), n_batches, src.max_iters, uint32_t(max_height) };
     if (packed && lod)
-        hipLaunchKernelGGL((k_walk_persistent<PackedBatch, true>), dim3(blocks), dim3(block), lds, s, psrc, total,
-                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk);
+        hipLaunchKernelGGL((k_walk<PackedBatch, true, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
+                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk,
+                           (const unsigned long long*)nullptr, 0u);
     else if (packed)
-        hipLaunchKernelGGL((k_walk_persistent<PackedBatch, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
-                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk);
+        hipLaunchKernelGGL((k_walk<PackedBatch, false, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
+                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk,
+                           (const unsigned long long*)nullptr, 0u);
     else if (cache && short_stack)
         hipLaunchKernelGGL((k_intersect_persistent<BatchSource, true, false, true>), dim3(blocks), dim3(block), lds, s,
                            src, total, (const uint32_t*)nullptr, counters, regroup, refill, rows, 0u, chunk);

@@ -305,8 +305,11 @@ cqx_status cqx_volume_download(cqx_ctx* ctx, const cqx_dvolume* vol, uint64_t fi
 cqx_status cqx_volume_info(const cqx_dvolume* vol, const uint32_t** dev_nodes, uint64_t* node_count,
                            uint32_t* root, cqx_subdag sub[8]);
 
-/* Launch parameters of the traversal kernel. Zero fields take the tuned or built-in defaults
- * (variant 2, 256 threads, 32 waves per CU, regroup 8, refill 16). */
+/* Launch parameters of the traversal kernel. With every field that shapes the launch zero (or no
+ * configuration at all) the library picks the launch by the batch's size and, past 2^20 rays, by
+ * whether a sample of the rays is coherent; otherwise zero fields take the built-in defaults
+ * (variant 2, 256 threads, 32 waves per CU, or 24 up to 2^23 rays, regroup 12, refill 16; stores of
+ * more than 2^24 nodes or volumes past 2^22 voxels from the origin: 32 waves, regroup 8). */
 typedef struct {
     uint32_t variant;          /* 0 auto (the autotuner's choice), 1 one ray per lane, 2 persistent waves
                                   (walk steps + service passes, rays claimed in chunks), 3 = 2 with the
@@ -427,9 +430,9 @@ typedef struct {
 /* mode 0: wavefront (traversal kernel per bounce, captured in a hipGraph, replayed per call);
  * mode 1: megakernel (one lane per path). Both give the same image bit for bit. `image` is a
  * device pointer; synchronizes `stream` before returning. cfg NULL or variant 0: the camera
- * rays are traced one per lane (64 per workgroup unless cfg sets block), the bounce rays on
- * persistent waves (24 per CU unless cfg sets waves_per_cu); the other fields of cfg apply as
- * given. An explicit variant applies to every depth. */
+ * rays are traced one per lane (64 per workgroup unless cfg sets block), the bounce rays by the
+ * library's choice, or on persistent waves (24 per CU unless cfg sets waves_per_cu) when cfg sets a
+ * field that shapes a launch; the other fields of cfg apply as given. An explicit variant applies to every depth. */
 cqx_status cqx_pathtrace(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_params* params, uint32_t mode,
                          const cqx_launch_cfg* cfg, float* image, void* stream);
 
@@ -460,8 +463,8 @@ cqx_status cqx_pathtrace_adjoint(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx
  * rays: device, n x 6 floats (the camera rays of PathtracingDemo::raytrace, :214-225); out_rgb:
  * device, n x 3 floats, overwritten or, with accumulate, added to (the demo's mImage +=).
  * cfg NULL or variant 0: the primaries one per lane (64 per workgroup unless cfg sets block),
- * the secondary rays on persistent waves (16 per CU unless cfg sets waves_per_cu); the other
- * fields of cfg apply as given. An explicit variant applies to every traversal of the frame.
+ * the secondary rays by the library's choice, or on persistent waves (16 per CU unless cfg sets
+ * waves_per_cu) when cfg sets a field that shapes a launch; the other fields of cfg apply as given. An explicit variant applies to every traversal of the frame.
  * Asynchronous on `stream`; one call in flight per context. n <= 2^30. */
 typedef struct {
     const float* colours; /* host, 256 x 3: the material colours (cqx_materials_colour_table) */

@@ -103,3 +103,65 @@ def test_packed_walk_refuses_volumes_past_its_limits(tmp_path, cq, oracle):
     with pytest.raises(subprocess.CalledProcessError) as e:
         _run(tmp_path, cq, hv.nodes, sub, np.zeros((1, 6), np.float32), "plain", True, -1.0)
     assert e.value.returncode == 6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 4097, 8193, 16385, 65537, 131073, (1 << 20) - 1, (1 << 20) + 1, 2621440,
+                               2621441, (1 << 23) + 63])
+@pytest.mark.parametrize("kind", ["incoherent", "camera"])
+def test_open_launch_shapes(cq, oracle, gpu_ctx, vol128, n, kind):
+    """The library's launches at the sizes where they change (rays per wave, dealt runs, sampled
+    coherence, persistent waves): every record equals the raw store's walk, the small ones the oracle."""
+    import torch
+
+    if kind == "camera":
+        from cubiquity_amd import workloads as W
+
+        c, side = W.RAYCAST_128.camera, int(np.ceil(np.sqrt(n)))
+        rays = cq.camera_rays(c.eye, c.target, c.fov_y, side, side)[:n]
+    else:
+        rays = cq.incoherent_rays(vol128, 7, 5 + n, n)
+    dv = gpu_ctx.upload(vol128)
+    r = torch.from_numpy(np.ascontiguousarray(rays)).cuda()
+    for surf, fp in ((True, -1.0), (False, 0.0035)):
+        got = cq.intersectVolume(gpu_ctx, dv, r, surf, fp)
+        raw = cq.intersectVolume(gpu_ctx, dv, r, surf, fp, cfg=cq.LaunchCfg(variant=3))
+        assert torch.equal(got, raw), int((got != raw).any(dim=1).sum())
+        if n <= 70000:
+            ref = oracle.intersect(vol128.nodes, oracle.find_subdags(vol128.nodes, vol128.root), rays, surf, fp, threads=8)
+            assert records_equal(got.cpu().numpy().view(cq.HIT_DTYPE).reshape(-1), ref).all()
+    dv.free()
+
+
+@pytest.mark.gpu
+def test_gpu_volumes_past_the_packed_limits(cq, oracle, gpu_ctx):
+    """A volume whose corners lie past 2^22 takes the raw walk, alone and in a batch with one that
+    does not, and comes back to the packed one after an undo on the device."""
+    import torch
+
+    rng = np.random.Generator(np.random.PCG64(3))
+    near = [[20.0 * i, 3.0, 5.0 * i, 4.0, 1 + i % 3] for i in range(16)]
+    far = [[float(1 << 22) + 50.0, 3.0, 3.0, 4.0, 2]] + near[1:]
+    hv = cq.HostVolume.from_dense(np.ones((4, 4, 4), np.uint8), (0, 0, 0))
+    dv = gpu_ctx.upload(hv)
+    dv.edit_spheres(near)
+    dv.checkpoint()
+    o = rng.uniform(-40.0, 400.0, (5000, 3))
+    d = rng.normal(size=(5000, 3))
+    rays = np.concatenate([o, d / np.linalg.norm(d, axis=1, keepdims=True)], 1).astype(np.float32)
+    r = torch.from_numpy(rays).cuda()
+
+    def check():
+        nodes = dv.download()
+        ref = oracle.intersect(nodes, oracle.find_subdags(nodes, dv.root), rays, True, threads=8)
+        hits = torch.zeros((5000, 32), dtype=torch.uint8, device="cuda")
+        cq.intersect_batched(gpu_ctx, [(dv, r, hits, True, -1.0)])
+        for got in (cq.intersectVolume(gpu_ctx, dv, r), hits):
+            assert records_equal(got.cpu().numpy().view(cq.HIT_DTYPE).reshape(-1), ref).all()
+
+    check()
+    dv.edit_spheres(far)
+    check()
+    dv.undo()
+    check()
+    dv.free()
