@@ -105,6 +105,9 @@ __device__ __forceinline__ uint32_t pack_child(const uint32_t* __restrict__ node
     return cqxd::packed_word(child, mask);
 }
 
+// Rays per wave of a one-ray-per-lane launch of n rays (at most 64).
+uint32_t lanes_per_wave(uint64_t n);
+
 // Ids per wave of a launch of at most n secondary rays whose count is on the device (launch_intersect's
 // `dealt`).
 uint32_t dealt_ids(uint64_t n);

@@ -378,9 +378,22 @@ struct PackedDesc {
     float max_footprint, lod_hi, lod_lo;
 };
 
+// Where the descriptors are: in the kernel's arguments up to kInlineBatches (no table to copy, and so no
+// wait for the launch that read the table before), in device memory past that.
+constexpr uint32_t kInlineBatches = 40; // 64 bytes each
+struct InlineDescs {
+    PackedDesc d[kInlineBatches];
+    __device__ __forceinline__ const PackedDesc& operator[](uint32_t i) const { return d[i]; }
+};
+struct TableDescs {
+    const PackedDesc* __restrict__ d;
+    __device__ __forceinline__ const PackedDesc& operator[](uint32_t i) const { return d[i]; }
+};
+
+template <typename Descs>
 struct PackedBatch {
     static constexpr bool kUniform = false;
-    const PackedDesc* __restrict__ desc;
+    Descs desc;
     uint32_t n_batches;
     uint32_t max_iters;
     uint32_t top;
@@ -409,7 +422,11 @@ struct PackedBatch {
 };
 
 __device__ __forceinline__ const PackedParams& uniform_params(const PackedSingle& s, const PackedParams&) { return s.P; }
-__device__ __forceinline__ const PackedParams& uniform_params(const PackedBatch&, const PackedParams& lane) { return lane; }
+template <typename Descs>
+__device__ __forceinline__ const PackedParams& uniform_params(const PackedBatch<Descs>&, const PackedParams& lane)
+{
+    return lane;
+}
 
 __device__ __forceinline__ void setup_packed(PackedRay& S, const float* r)
 {
@@ -1247,6 +1264,46 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
 
 } // namespace cqx
 
+namespace {
+
+// Up to this many rays an open batched launch deals its ids to the waves, 64 or fewer each (lanes_per_wave):
+// batches of camera rays keep together and no counters are cleared, claimed and found empty. Past it
+// the claims of persistent waves win. Measured (MI355X, us, dealt / claimed): 27 k rays of 5 volumes
+// 75 / 88, 1.65 M of 24 216 / 300, 2.47 M of 32 294 / 351, 11.1 M of 64 1508 / 1258.
+constexpr uint64_t kDealtBatchRays = 1u << 22;
+
+struct WalkLaunch {
+    bool lod, dealt;
+    uint32_t top, block, blocks, regroup, refill, chunk;
+    unsigned long long* counters;
+};
+
+template <typename Batch, bool kLod>
+void launch_batch_as(const Batch& src, const WalkLaunch& w, uint64_t total, hipStream_t s)
+{
+    const uint32_t rows = w.top + 1u;
+    const uint32_t* const no_count = nullptr;
+    const unsigned long long* const no_gate = nullptr;
+    if (w.dealt) {
+        const uint32_t ids = cqx::lanes_per_wave(total);
+        hipLaunchKernelGGL((k_walk<Batch, kLod, true>), dim3(uint32_t((total + ids - 1) / ids)), dim3(64), size_t(rows) * 256,
+                           s, src, total, no_count, w.counters, 12u, 64u, rows, ids, no_gate, 0u);
+    } else {
+        hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, w.counters);
+        hipLaunchKernelGGL((k_walk<Batch, kLod, false>), dim3(w.blocks), dim3(w.block), size_t(rows) * w.block * 4, s, src,
+                           total, no_count, w.counters, w.regroup, w.refill, rows, w.chunk, no_gate, 0u);
+    }
+}
+
+template <typename Batch>
+void launch_batch(const Batch& src, const WalkLaunch& w, uint64_t total, hipStream_t s)
+{
+    if (w.lod) launch_batch_as<Batch, true>(src, w, total, s);
+    else launch_batch_as<Batch, false>(src, w, total, s);
+}
+
+} // namespace
+
 extern "C" {
 
 cqx_status cqx_create(int device, cqx_ctx** out)
@@ -1569,10 +1626,24 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     if (lds + kSubdagCopyBytes > size_t(ctx->lds_per_block))
         return fail(CQX_ERR_LIMIT, "stack needs %zu B of LDS per block", lds + kSubdagCopyBytes);
     hipStream_t s = hipStream_t(stream_ptr);
-    // The descriptor table is per context: wait for an earlier batched launch on this stream.
-    HIP_TRY(hipStreamSynchronize(s));
     // one volume past the packed walk's limits, or a launch it does not serve: all on the raw stores
     packed = packed && !short_stack && !(cfg && cfg->variant == 3);
+    uint32_t blocks, regroup, refill, chunk;
+    st = persistent_shape(ctx, cfg, block, total, packed, blocks, regroup, refill, chunk);
+    if (st != CQX_OK) return st;
+    const uint32_t max_iters = (cfg && cfg->max_iters) ? cfg->max_iters : cqx::kDefaultMaxIters;
+    unsigned long long* counters = reinterpret_cast<unsigned long long*>(ctx->d_counter);
+    const WalkLaunch walk{ lod, cqx::launch_open(cfg) && total <= kDealtBatchRays, uint32_t(max_height), block, blocks,
+                           regroup, refill, chunk, counters };
+    if (packed && n_batches <= kInlineBatches) {
+        PackedBatch<InlineDescs> src{ {}, n_batches, max_iters, uint32_t(max_height) };
+        std::copy(pdesc.begin(), pdesc.end(), src.desc.d);
+        launch_batch(src, walk, total, s);
+        HIP_TRY(hipGetLastError());
+        return CQX_OK;
+    }
+    // The descriptor table is per context: wait for an earlier batched launch on this stream.
+    HIP_TRY(hipStreamSynchronize(s));
     const size_t bytes = packed ? pdesc.size() * sizeof(PackedDesc) : desc.size() * sizeof(BatchDesc);
     if (bytes > ctx->batch_bytes) {
         release(ctx->batch_desc);
@@ -1583,24 +1654,16 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     }
     HIP_TRY(hipMemcpy(ctx->batch_desc, packed ? static_cast<const void*>(pdesc.data()) : desc.data(), bytes,
                       hipMemcpyHostToDevice));
-    uint32_t blocks, regroup, refill, chunk;
-    st = persistent_shape(ctx, cfg, block, total, packed, blocks, regroup, refill, chunk);
-    if (st != CQX_OK) return st;
-    BatchSource src{ static_cast<const BatchDesc*>(ctx->batch_desc), n_batches,
-                     (cfg && cfg->max_iters) ? cfg->max_iters : cqx::kDefaultMaxIters };
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned long long*>(ctx->d_counter));
-    unsigned long long* counters = reinterpret_cast<unsigned long long*>(ctx->d_counter);
+    if (packed) {
+        launch_batch(PackedBatch<TableDescs>{ { static_cast<const PackedDesc*>(ctx->batch_desc) }, n_batches, max_iters,
+                                              uint32_t(max_height) }, walk, total, s);
+        HIP_TRY(hipGetLastError());
+        return CQX_OK;
+    }
+    BatchSource src{ static_cast<const BatchDesc*>(ctx->batch_desc), n_batches, max_iters };
+    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, counters);
     const bool cache = cfg && cfg->variant == 3;
-    const PackedBatch psrc{ static_cast<const PackedDesc*>(ctx->batch_desc), n_batches, src.max_iters, uint32_t(max_height) };
-    if (packed && lod)
-        hipLaunchKernelGGL((k_walk<PackedBatch, true, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
-                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk,
-                           (const unsigned long long*)nullptr, 0u);
-    else if (packed)
-        hipLaunchKernelGGL((k_walk<PackedBatch, false, false>), dim3(blocks), dim3(block), lds, s, psrc, total,
-                           (const uint32_t*)nullptr, counters, regroup, refill, rows, chunk,
-                           (const unsigned long long*)nullptr, 0u);
-    else if (cache && short_stack)
+    if (cache && short_stack)
         hipLaunchKernelGGL((k_intersect_persistent<BatchSource, true, false, true>), dim3(blocks), dim3(block), lds, s,
                            src, total, (const uint32_t*)nullptr, counters, regroup, refill, rows, 0u, chunk);
     else if (short_stack)

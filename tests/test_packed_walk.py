@@ -165,3 +165,26 @@ def test_gpu_volumes_past_the_packed_limits(cq, oracle, gpu_ctx):
     dv.undo()
     check()
     dv.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batches,n", [(1, 1), (3, 0), (40, 777), (41, 777), (40, 110000)])
+def test_batched_launch_shapes(cq, gpu_ctx, vol128, rays128, batches, n):
+    """Descriptors in the kernel's arguments and in a table, dealt and claimed ids, empty batches: every
+    record equals the batch's own launch over the raw store."""
+    import torch
+
+    dv = gpu_ctx.upload(vol128)
+    rays = torch.from_numpy(np.concatenate([rays128["incoherent"], rays128["camera"]])).cuda()
+    items = []
+    for i in range(batches):
+        m = 0 if n and i % 5 == 4 else n + 7 * i
+        r = rays.roll(i * 911, 0).repeat((m + len(rays) - 1) // len(rays), 1)[:m] if m else rays[:0]
+        hits = torch.zeros((max(1, m), 32), dtype=torch.uint8, device="cuda")
+        items.append((dv, r.contiguous(), hits, i % 2 == 0, 0.0035 if i % 3 == 2 else -1.0))
+    cq.intersect_batched(gpu_ctx, items)
+    for i, (v, r, hits, surf, fp) in enumerate(items):
+        if len(r):
+            raw = cq.intersectVolume(gpu_ctx, v, r, surf, fp, cfg=cq.LaunchCfg(variant=3))
+            assert torch.equal(hits[: len(r)], raw), i
+    dv.free()
