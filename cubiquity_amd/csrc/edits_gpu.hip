@@ -87,21 +87,8 @@ __device__ __forceinline__ uint64_t hash_node(const DNode& n)
     return h;
 }
 
-// Index of a store node with this content, or kEmptySlot. kCoherent: for a kernel that inserts
-// into the index and appends nodes while it looks them up.
-template <bool kCoherent = false>
-__device__ uint32_t index_find(const uint32_t* __restrict__ nodes, const uint32_t* __restrict__ slots, uint64_t mask,
-                               const DNode& n)
-{
-    for (uint64_t i = hash_node(n) & mask;; i = (i + 1) & mask) {
-        const uint32_t s = kCoherent ? __hip_atomic_load(slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : slots[i];
-        if (s == kEmptySlot) return kEmptySlot;
-        if (node_eq(kCoherent ? load_node_coherent(nodes, s) : load_node(nodes, s), n)) return s;
-    }
-}
-
 // Adds store node j to the index: an empty slot is claimed with a compare-and-swap; where an equal
-// node already sits, the lower index stays.
+// node already sits, the lower index stays. kCoherent: for a kernel that appends nodes meanwhile.
 template <bool kCoherent = false>
 __device__ void index_insert(const uint32_t* __restrict__ nodes, uint32_t* __restrict__ slots, uint64_t mask, uint32_t j,
                              const DNode& n)
@@ -783,45 +770,201 @@ struct TopArgs {
     uint32_t* old;        // per entry of level >= 1: the node it held before the edits
 };
 
+// Index of a store node with this content, or kEmptySlot, while nodes are appended and inserted: 4
+// slots are read at once, since a probe is a chain of memory latencies.
+__device__ uint32_t index_find(const uint32_t* nodes, const uint32_t* slots, uint64_t mask, const DNode& n)
+{
+    for (uint64_t i = hash_node(n) & mask;; i += 4) {
+        uint32_t s[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            s[j] = __hip_atomic_load(slots + ((i + j) & mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (s[j] == kEmptySlot) return kEmptySlot;
+            if (node_eq(load_node_coherent(nodes, s[j]), n)) return s[j];
+        }
+    }
+}
+
+// The levels of at most 64 entries ("small"; with a level every one above it is), on one wave with an
+// entry per lane, their schedule, old nodes and results in LDS and equal new nodes found by comparing
+// lanes. Above a volume's own height a level holds an entry or a few and depends on the one below, so
+// the time is a chain of memory latencies: per level one read going down, and going up the index slots,
+// a node and the insertion, the old node's words being read a level ahead. At 2048^3, 1000 spheres of
+// radius 2 to 16 (4700 regions, 24 of the 27 levels small): k_edit_top 780 us with every level on the
+// workgroup (5 barriers and as many passes through memory each, fences at device scope), 200 us so.
+constexpr uint32_t kTopLevels = 28; // 32 - hs for hs >= 5, and level 0
+struct SmallTop {
+    uint32_t off[kTopLevels + 1]; // lvl_off
+    uint32_t first;               // the lowest small level, >= 1
+    uint32_t kids[kTopLevels * 64]; // of small entry e (at e - off[first]): cbeg | octant in the parent << 26 | count << 29
+    uint32_t old[kTopLevels * 64];  // the node it held before the edits
+    uint32_t below[64];
+};
+
+__device__ __forceinline__ uint32_t key_octant(const DRegionKey& k)
+{
+    return (k.x & 1u) | (k.y & 1u) << 1 | (k.z & 1u) << 2;
+}
+
+// The schedule into LDS, by the whole workgroup; ends with a barrier.
+__device__ void top_stage(const TopArgs& A, SmallTop& S, uint32_t t, uint32_t T)
+{
+    if (t < A.levels + 2) S.off[t] = A.lvl_off[t];
+    __syncthreads();
+    if (t == 0) {
+        uint32_t l = 1;
+        while (S.off[l + 1] - S.off[l] > 64) l++;
+        S.first = l;
+    }
+    __syncthreads();
+    const uint32_t b = S.off[S.first], n = S.off[A.levels + 1] - b;
+    for (uint32_t i = t; i < n; i += T) {
+        const uint32_t cb = A.cbeg[b + i];
+        S.kids[i] = (cb - S.off[S.first - 1]) | key_octant(A.keys[b + i]) << 26 | (A.cend[b + i] - cb - 1) << 29;
+    }
+    __syncthreads();
+}
+
+// Old nodes of the small levels and of the level below them, top down.
+__device__ void top_small_down(const TopArgs& A, SmallTop& S, uint32_t lane)
+{
+    const uint32_t b0 = S.off[S.first];
+    if (lane == 0) S.old[S.off[A.levels] - b0] = A.root;
+    wave_fence();
+    for (uint32_t l = A.levels; l >= S.first && l >= 2; l--) {
+        const uint32_t e = S.off[l] + lane;
+        if (e < S.off[l + 1]) {
+            const uint32_t p = S.old[e - b0], k = S.kids[e - b0];
+            DNode in;
+            if (p >= kMat) in = load_node(A.nodes, p);
+            else
+                for (uint32_t& x : in.c) x = p;
+            const uint32_t cb = (k & 0x3ffffffu) + S.off[S.first - 1];
+            for (uint32_t j = cb; j <= cb + (k >> 29); j++) {
+                const uint32_t id = l > S.first ? (S.kids[j - b0] >> 26) & 7u : key_octant(A.keys[j]);
+                uint32_t x = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++) x = c == id ? in.c[c] : x;
+                if (l > S.first) S.old[j - b0] = x;
+                else A.old[j] = x;
+            }
+        }
+        wave_fence();
+    }
+}
+
+// The small levels bottom up; `base` is the store's size.
+__device__ void top_small_up(const TopArgs& A, SmallTop& S, uint32_t base, uint32_t lane)
+{
+    const uint32_t b0 = S.off[S.first], c0 = S.off[S.first - 1];
+    const auto old_node = [&](uint32_t l, uint32_t& old, DNode& n) {
+        const uint32_t e = S.off[l] + lane;
+        old = l <= A.levels && e < S.off[l + 1] ? S.old[e - b0] : 0u;
+        if (old >= kMat) n = load_node(A.nodes, old);
+        else
+            for (uint32_t& x : n.c) x = old;
+    };
+    uint32_t old, top = 0;
+    DNode out;
+    old_node(S.first, old, out);
+    for (uint32_t l = S.first; l <= A.levels; l++) {
+        const uint32_t e = S.off[l] + lane;
+        const bool have = e < S.off[l + 1];
+        uint32_t next_old;
+        DNode next;
+        old_node(l + 1, next_old, next);
+        uint32_t r = old;
+        bool fresh = false, changed = false;
+        if (have) {
+            const uint32_t k = S.kids[e - b0], cb = (k & 0x3ffffffu) + c0;
+            for (uint32_t j = cb; j <= cb + (k >> 29); j++) {
+                const uint32_t id = l > S.first ? (S.kids[j - b0] >> 26) & 7u : key_octant(A.keys[j]);
+                const uint32_t x = l > S.first ? S.below[j - S.off[l - 1]] : A.res[j];
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++)
+                    if (c == id && out.c[c] != x) {
+                        out.c[c] = x;
+                        changed = true;
+                    }
+            }
+        }
+        if (changed) { // Interner::intern: collapse, else the store's node, else new
+            bool uniform = out.c[0] < kMat;
+#pragma unroll
+            for (int c = 1; c < 8; c++) uniform = uniform && out.c[c] == out.c[0];
+            r = uniform ? out.c[0] : index_find(A.nodes, A.index, A.index_mask, out);
+            fresh = r == kEmptySlot;
+        }
+        // new nodes appended in entry order, equal ones once
+        uint64_t todo = __ballot(fresh);
+        while (todo) {
+            const int g = __ffsll((unsigned long long)todo) - 1;
+            bool eq = fresh;
+#pragma unroll
+            for (int c = 0; c < 8; c++) eq = eq && out.c[c] == uint32_t(__builtin_amdgcn_readlane(int(out.c[c]), g));
+            todo &= ~__ballot(eq);
+            if (eq) r = base;
+            if (int(lane) == g) store_node(A.nodes, base, out);
+            else if (eq) fresh = false; // the first of the equal ones inserts it
+            base++;
+        }
+        wave_fence();
+        if (fresh) index_insert<true>(A.nodes, A.index, A.index_mask, r, out);
+        if (have) S.below[lane] = r;
+        wave_fence();
+        top = r;
+        old = next_old;
+        out = next;
+    }
+    if (lane == 0) {
+        *A.out_count = base;
+        *A.out_root = top; // the top level has one entry
+    }
+}
+
+// One workgroup, so its barriers order its memory operations: all of them go through one L1 and one L2.
 __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
 {
     __shared__ uint32_t wave_kept[kTopBlock / 64];
+    __shared__ SmallTop small;
     __shared__ uint32_t count_s;
     const uint32_t t = threadIdx.x, T = blockDim.x;
     if (t == 0) count_s = *A.out_count;
     for (uint32_t i = A.lvl_off[0] + t; i < A.lvl_off[1]; i += T) A.res[i] = A.results[A.morton_regions[i]];
+    top_stage(A, small, t, T);
     // The nodes the entries held before the edits, top down: the top entry (height 32, one key)
     // holds the root, and an entry's children hold the children of its node (node_at of every
     // entry, with one read per entry instead of one per level above it).
-    if (t == 0) A.old[A.lvl_off[A.levels]] = A.root;
-    __threadfence();
+    if (t < 64) top_small_down(A, small, t);
     __syncthreads();
-    for (uint32_t l = A.levels; l >= 2; l--) {
-        for (uint32_t i = A.lvl_off[l] + t; i < A.lvl_off[l + 1]; i += T) {
-            const uint32_t p = __hip_atomic_load(A.old + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for (uint32_t j = A.cbeg[i]; j < A.cend[i]; j++) {
-                const DRegionKey k = A.keys[j];
-                const uint32_t id = (k.x & 1u) | (k.y & 1u) << 1 | (k.z & 1u) << 2;
-                A.old[j] = p < kMat ? p : A.nodes[uint64_t(p) * 8 + id];
-            }
+    for (uint32_t l = small.first - 1; l >= 2; l--) {
+        for (uint32_t i = small.off[l] + t; i < small.off[l + 1]; i += T) {
+            const uint32_t p = A.old[i];
+            const uint32_t ce = A.cend[i];
+            for (uint32_t j = A.cbeg[i]; j < ce; j++) A.old[j] = p < kMat ? p : A.nodes[uint64_t(p) * 8 + key_octant(A.keys[j])];
         }
-        __threadfence();
         __syncthreads();
     }
-    for (uint32_t l = 1; l <= A.levels; l++) {
-        const uint32_t b = A.lvl_off[l], e = A.lvl_off[l + 1];
+    for (uint32_t l = 1; l < small.first; l++) {
+        const uint32_t b = small.off[l], e = small.off[l + 1];
         for (uint32_t i = b + t; i < e; i += T) {
-            const uint32_t old = __hip_atomic_load(A.old + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t old = A.old[i];
             DNode out;
-            for (int c = 0; c < 8; c++) out.c[c] = old < kMat ? old : A.nodes[uint64_t(old) * 8 + c];
+            if (old >= kMat) out = load_node(A.nodes, old);
+            else
+                for (uint32_t& x : out.c) x = old;
             bool changed = false;
-            for (uint32_t j = A.cbeg[i]; j < A.cend[i]; j++) {
-                const DRegionKey k = A.keys[j];
-                const uint32_t id = (k.x & 1u) | (k.y & 1u) << 1 | (k.z & 1u) << 2;
-                if (A.res[j] != out.c[id]) {
-                    out.c[id] = A.res[j];
-                    changed = true;
-                }
+            const uint32_t ce = A.cend[i];
+            for (uint32_t j = A.cbeg[i]; j < ce; j++) {
+                const uint32_t id = key_octant(A.keys[j]), x = A.res[j];
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++)
+                    if (c == id && out.c[c] != x) {
+                        out.c[c] = x;
+                        changed = true;
+                    }
             }
             uint32_t r = old, cand = 0;
             if (changed) { // Interner::intern: collapse, else the store's node, else new
@@ -829,7 +972,7 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
                 for (int c = 1; c < 8; c++) uniform = uniform && out.c[c] == out.c[0];
                 if (uniform) r = out.c[0];
                 else {
-                    r = index_find<true>(A.nodes, A.index, A.index_mask, out);
+                    r = index_find(A.nodes, A.index, A.index_mask, out);
                     if (r == kEmptySlot) {
                         cand = 1;
                         store_node(A.ckey, i, out);
@@ -839,7 +982,6 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
             A.res[i] = r;
             A.cand[i] = cand;
         }
-        __threadfence();
         __syncthreads();
         // equal new nodes of this level: the first in Morton order is kept
         const uint64_t tmask = (A.tab_off[l + 1] - A.tab_off[l]) - 1;
@@ -856,11 +998,9 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
                 }
             }
         }
-        __threadfence();
         __syncthreads();
         for (uint32_t i = b + t; i < e; i += T)
             if (A.cand[i]) A.crep[i] = __hip_atomic_load(tab + A.cslot[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __threadfence();
         __syncthreads();
         // the kept ones appended in order: a scan over the level in chunks of T entries (each wave
         // ranks its lanes by ballot, then adds the counts of the waves before it)
@@ -885,7 +1025,6 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
             base += all;
             __syncthreads();
         }
-        __threadfence();
         __syncthreads();
         for (uint32_t i = b + t; i < e; i += T)
             if (A.cand[i]) {
@@ -893,13 +1032,9 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
                 else index_insert<true>(A.nodes, A.index, A.index_mask, A.res[i], load_node_coherent(A.ckey, i));
             }
         if (t == 0) count_s = base;
-        __threadfence();
         __syncthreads();
     }
-    if (t == 0) {
-        *A.out_count = count_s;
-        *A.out_root = A.res[A.lvl_off[A.levels]];
-    }
+    if (t < 64) top_small_up(A, small, count_s, t);
 }
 
 // findSubDAG (raytracing.cpp:43-87) of every root child, as cqx::find_subdags, one thread each, with

@@ -38,3 +38,22 @@ def test_device_walk_equals_host(cq, gpu_ctx, monkeypatch, log2, radius, n, kind
         eq = (dv.download() == hv.nodes).all(axis=1)
         assert eq.all(), f"frame {frame}: {(~eq).sum()} of {len(eq)} nodes differ, first at {np.nonzero(~eq)[0][:5]}"
     dv.free()
+
+
+@pytest.mark.parametrize("n", [17, 64, 65, 130])
+def test_levels_above_equal_regions(cq, gpu_ctx, n):
+    """n equal spheres in n parents of regions, in a row through empty space and (every third) one that
+    differs: levels of 64 entries and around, whose new nodes are equal in sets."""
+    hv = cq.HostVolume.generate(cq.gen_default_params(6, 3, n_materials=16))
+    dv = gpu_ctx.upload(hv)
+    for frame in range(2):
+        e = np.zeros((n, 5))
+        e[:, 0] = 64.0 * np.arange(n) + 16.0
+        e[:, 1] = -64.0 * (np.arange(n) % 4) + 16.0 + 4096.0 * frame
+        e[:, 2] = 1024.0 + 16.0
+        e[:, 3] = 6.0
+        e[:, 4] = np.where(np.arange(n) % 3 == 2, 9, 5)
+        assert dv.edit_spheres(e) == hv.edit_spheres(e, threads=8)
+        assert (dv.node_count, dv.root) == (hv.node_count, hv.root)
+        assert (dv.download() == hv.nodes).all()
+    dv.free()
