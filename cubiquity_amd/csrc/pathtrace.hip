@@ -25,7 +25,7 @@
 // a sweep kernel rebuilds each path's throughputs in the forward's FP32 order and runs backwards,
 //   G_K = sky if escaped else 0;  G_j = E_j + A_j G_{j+1};
 //   dV/dE_j = beta_j,  dV/dA_j = beta_j G_{j+1},
-// scaled by dL/dpixel / spp; per-block partial sums in LDS, reduced over blocks in FP64.
+// scaled by dL/dpixel / spp; partial sums in LDS, reduced over blocks in FP64.
 #include "device_internal.h"
 
 #include <algorithm>
@@ -343,31 +343,143 @@ __global__ void __launch_bounds__(256) k_pt_megakernel(const PtDevParams* __rest
 // segment only), then its vertices are swept from last to first.
 //
 // The gradient sums have a fixed order, so the result is the same bit for bit on every run: each
-// wave takes 64 consecutive paths at a time. With at most kAccMaterials materials (kAcc), each
-// lane adds its paths' contributions, vertex by vertex in order, into its own registers, one row per
-// material, and after its last path the wave sums each row by a fixed butterfly into its row of
-// per-material totals in LDS. With more materials, vertex slot by vertex slot, the wave groups its
-// lanes by material (the first remaining lane's material, then the next); a group's six
-// contributions are summed over the wave by a fixed butterfly (lanes outside the group add 0) and
-// lane 0 adds the sums to the wave's row. No atomics are involved; the block adds its waves' rows
-// in wave order.
+// wave takes 64 consecutive paths at a time, and no atomics are involved.
 constexpr uint32_t kAdjointBlock = 256;
 constexpr int kSegment = 4; // vertices per segment: a path of up to 3 bounces is one
 constexpr uint32_t kAdjointWaves = kAdjointBlock / 64;
-constexpr int kAccMaterials = 16;
+constexpr uint32_t kAccMaterials = 16;
 
-template <bool kAcc>
+// Up to kAccMaterials materials: each lane adds its paths' contributions, vertex by vertex in order,
+// into its own column of sums in LDS (one row per material and component), and after its last path
+// the wave sums each row in a fixed order (the tree of a butterfly over the lanes), a row per lane.
+// One wave per workgroup, so that as many as the rows leave room for (6 per CU with 16 materials)
+// share a CU. The sums lived in 96 registers before, each contribution added to all of them through
+// selects, 192 instructions per vertex: 113 us for 2^21 paths of up to 4 vertices and 16 materials,
+// 57 us so (and k_pt_reduce 10 us for 5, over four times the rows). The next paths' records are read while the current ones are swept.
+struct SweepIn {
+    uint32_t stat;
+    uint32_t vm[kSegment]; // the first segment's materials; entries past the path's end are not used
+    float delta[3];
+};
+
+__global__ void __launch_bounds__(64) k_pt_adjoint_lds(const PtDevParams* __restrict__ dp, uint64_t P,
+                                                       const uint8_t* __restrict__ vmat,
+                                                       const uint8_t* __restrict__ vstat,
+                                                       const float* __restrict__ dimage, uint32_t M,
+                                                       float* __restrict__ partials)
+{
+    extern __shared__ float acc[]; // [M * 6 rows: dA rgb, dE rgb per material][64 lanes]
+    __shared__ float table[kAccMaterials + 1][6]; // albedo, emission by material; row 0 for ids not listed (zeros)
+    const PtDevParams& d = *dp;
+    const uint32_t lane = threadIdx.x, rows = M * 6, last = d.bounces;
+    for (uint32_t k = lane; k < (M + 1) * 6; k += 64) {
+        const uint32_t m = k / 6, c = k % 6;
+        table[m][c] = m == 0 ? 0.0f : c < 3 ? d.albedo[m * 3 + c] : d.emission[m * 3 + (c - 3)];
+    }
+    for (uint32_t r = 0; r < rows; r++) acc[r * 64 + lane] = 0.0f;
+    __syncthreads();
+    const float inv_spp = 1.0f / float(d.spp);
+    const uint64_t stride_all = uint64_t(gridDim.x) * 64;
+    const auto load = [&](uint64_t p, SweepIn& in) {
+        const bool valid = p < P;
+        in.stat = valid ? vstat[p] : 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < uint32_t(kSegment); i++) in.vm[i] = valid && i <= last ? vmat[uint64_t(i) * P + p] : 0u;
+        const uint32_t pixel = valid ? uint32_t(p) / d.spp : 0u; // P < 2^32
+#pragma unroll
+        for (int a = 0; a < 3; a++) in.delta[a] = valid ? dimage[uint64_t(pixel) * 3 + a] * inv_spp : 0.0f;
+    };
+    // `base` is the same for the 64 lanes, so every lane runs every iteration
+    uint64_t base = uint64_t(blockIdx.x) * 64;
+    SweepIn cur;
+    load(base + lane, cur);
+    for (; base < P; base += stride_all) {
+        const uint64_t p = base + lane;
+        SweepIn ahead;
+        load(p + stride_all, ahead);
+        const int K = int(cur.stat & ~kEscaped);
+        const bool escaped = (cur.stat & kEscaped) != 0;
+        float G[3];
+        for (int a = 0; a < 3; a++) G[a] = escaped ? d.sky[a] : 0.0f;
+        // the wave's most vertices (a wave-uniform segment count)
+        int kw = 0;
+        while (__any(K > kw)) kw += kSegment;
+        for (int j0 = kw - kSegment; j0 >= 0; j0 -= kSegment) {
+            float b[3] = { 1.0f, 1.0f, 1.0f };
+            for (int j = 0; j < j0 && j < K; j++) {
+                const uint32_t m = vmat[uint64_t(j) * P + p];
+                for (int a = 0; a < 3; a++) b[a] = b[a] * d.albedo[m * 3 + a];
+            }
+            uint32_t vm[kSegment];
+            float vb[kSegment][3], va[kSegment][3];
+#pragma unroll
+            for (int i = 0; i < kSegment; i++) {
+                const bool live = j0 + i < K;
+                const uint32_t m = !live ? 0u : j0 == 0 ? cur.vm[i] : vmat[uint64_t(j0 + i) * P + p];
+                vm[i] = m <= M ? m : 0u;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    va[i][a] = table[vm[i]][a];
+                    vb[i][a] = b[a];
+                    b[a] = b[a] * va[i][a];
+                }
+            }
+#pragma unroll
+            for (int i = kSegment - 1; i >= 0; i--) {
+                if (j0 + i >= K) continue;
+                const uint32_t m = vm[i];
+                float* const row = acc + (m - 1) * 6 * 64 + lane;
+                float c[6];
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const float w = cur.delta[a] * vb[i][a];
+                    c[a] = w * G[a];
+                    c[3 + a] = w;
+                    G[a] = table[m][3 + a] + va[i][a] * G[a];
+                }
+                if (m)
+#pragma unroll
+                    for (int k = 0; k < 6; k++) row[k * 64] += c[k];
+            }
+        }
+        cur = ahead;
+    }
+    __syncthreads();
+    // Row r on lane r & 63: column j ^ lane at step j, so that the 64 lanes read 64 banks; the tree over
+    // the columns (j and j ^ 32 first, then ^ 16, ..) is the same for every lane.
+    for (uint32_t r = lane; r < rows; r += 64) {
+        const float* const v = acc + r * 64;
+        float t[6] = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f }; // partial sums waiting for their other half, by level
+        float sum = 0.0f;
+#pragma unroll
+        for (uint32_t n = 0; n < 64; n++) {
+            uint32_t j = 0; // n with its 6 bits reversed
+#pragma unroll
+            for (uint32_t k = 0; k < 6; k++) j |= ((n >> k) & 1u) << (5 - k);
+            sum = v[j ^ lane];
+#pragma unroll
+            for (uint32_t k = 0; k < 6; k++) {
+                if (!((n >> k) & 1u)) {
+                    t[k] = sum;
+                    break;
+                }
+                sum = t[k] + sum;
+            }
+        }
+        partials[uint64_t(blockIdx.x) * rows + r] = sum;
+    }
+}
+
+// More materials: vertex slot by vertex slot, the wave groups its lanes by material (the first
+// remaining lane's material, then the next); a group's six contributions are summed over the wave by a
+// fixed butterfly (lanes outside the group add 0) and lane 0 adds the sums to the wave's row of
+// per-material totals in LDS; the block adds its waves' rows in wave order.
 __global__ void __launch_bounds__(kAdjointBlock) k_pt_adjoint(const PtDevParams* __restrict__ dp, uint64_t P,
                                                               const uint8_t* __restrict__ vmat,
                                                               const uint8_t* __restrict__ vstat,
                                                               const float* __restrict__ dimage, uint32_t M,
                                                               float* __restrict__ partials)
 {
-    float acc[kAcc ? kAccMaterials : 1][6]; // kAcc: this lane's sums, row m - 1 for material m
-#pragma unroll
-    for (int mm = 0; mm < (kAcc ? kAccMaterials : 1); mm++)
-#pragma unroll
-        for (int k = 0; k < 6; k++) acc[mm][k] = 0.0f;
     __shared__ float g[kAdjointWaves][256 * 6]; // per wave: [material][dA rgb, dE rgb]
     for (uint32_t k = threadIdx.x; k < kAdjointWaves * 256 * 6; k += blockDim.x) (&g[0][0])[k] = 0.0f;
     __syncthreads();
@@ -429,17 +541,6 @@ __global__ void __launch_bounds__(kAdjointBlock) k_pt_adjoint(const PtDevParams*
                         G[a] = d.emission[m * 3 + a] + d.albedo[m * 3 + a] * G[a];
                     }
                 }
-                if constexpr (kAcc) {
-                    if (live) {
-#pragma unroll
-                        for (int mm = 0; mm < kAccMaterials; mm++) {
-                            const bool hit = m == uint32_t(mm + 1);
-#pragma unroll
-                            for (int k = 0; k < 6; k++) acc[mm][k] += hit ? c[k] : 0.0f;
-                        }
-                    }
-                    continue;
-                }
                 uint64_t todo = __ballot(live);
                 while (todo) {
                     const uint32_t m0 = uint32_t(__shfl(int(m), __ffsll((unsigned long long)todo) - 1));
@@ -456,17 +557,6 @@ __global__ void __launch_bounds__(kAdjointBlock) k_pt_adjoint(const PtDevParams*
             }
         }
     }
-    if constexpr (kAcc) {
-#pragma unroll
-        for (int mm = 0; mm < kAccMaterials; mm++)
-#pragma unroll
-            for (int k = 0; k < 6; k++) {
-                float v = acc[mm][k];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-                if (lane == 0) gw[(mm + 1) * 6 + k] = v;
-            }
-    }
     __syncthreads();
     for (uint32_t k = threadIdx.x; k < M * 6; k += blockDim.x) { // material ids 1..M
         float sum = 0.0f;
@@ -476,14 +566,21 @@ __global__ void __launch_bounds__(kAdjointBlock) k_pt_adjoint(const PtDevParams*
 }
 
 // One workgroup per output value ((material - 1) * 6 + component): strided FP64 sums over the
-// block partials, then a fixed-order tree in LDS (deterministic for a given grid).
+// block partials (kWaves rows each, added in FP32 in order), then a fixed-order tree in LDS
+// (deterministic for a given grid).
+template <uint32_t kWaves>
 __global__ void __launch_bounds__(256) k_pt_reduce(const float* __restrict__ partials, uint32_t blocks, uint32_t M,
                                                    float* __restrict__ d_albedo, float* __restrict__ d_emission)
 {
     __shared__ double acc[256];
     const uint32_t k = blockIdx.x;
     double sum = 0.0;
-    for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) sum += double(partials[uint64_t(b) * M * 6 + k]);
+    for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) {
+        float f = 0.0f;
+#pragma unroll
+        for (uint32_t w = 0; w < kWaves; w++) f += partials[(uint64_t(b) * kWaves + w) * M * 6 + k];
+        sum += double(f);
+    }
     acc[threadIdx.x] = sum;
     __syncthreads();
     for (uint32_t w = blockDim.x / 2; w > 0; w /= 2) {
@@ -809,7 +906,8 @@ cqx_status cqx_pathtrace_adjoint(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx
     const uint32_t block = kAdjointBlock;
     const uint32_t blocks =
         uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(ctx->cu_count) * 8, (p->P + block - 1) / block)));
-    const size_t need = size_t(blocks) * pp->n_materials * 6;
+    const bool in_lds = pp->n_materials <= kAccMaterials;
+    const size_t need = size_t(blocks) * (in_lds ? kAdjointWaves : 1u) * pp->n_materials * 6;
     if (need > p->partial_floats) {
         HIP_TRY(hipDeviceSynchronize());
         release(p->partials);
@@ -828,14 +926,18 @@ cqx_status cqx_pathtrace_adjoint(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx
     }
     {
         const cqx::TraceRange sweep("adjoint: backward sweep and reduction");
-        if (pp->n_materials <= uint32_t(kAccMaterials))
-            hipLaunchKernelGGL(k_pt_adjoint<true>, dim3(blocks), dim3(block), 0, s, p->dparams, p->P, p->vmat, p->vstat,
+        if (in_lds) { // a wave per workgroup, with the paths that the 256-thread blocks' waves would take
+            hipLaunchKernelGGL(k_pt_adjoint_lds, dim3(blocks * kAdjointWaves), dim3(64),
+                               pp->n_materials * 6 * 64 * sizeof(float), s, p->dparams, p->P, p->vmat, p->vstat,
                                d_image, pp->n_materials, p->partials);
-        else
-            hipLaunchKernelGGL(k_pt_adjoint<false>, dim3(blocks), dim3(block), 0, s, p->dparams, p->P, p->vmat, p->vstat,
+            hipLaunchKernelGGL(k_pt_reduce<kAdjointWaves>, dim3(pp->n_materials * 6), dim3(256), 0, s, p->partials,
+                               blocks, pp->n_materials, d_albedo, d_emission);
+        } else {
+            hipLaunchKernelGGL(k_pt_adjoint, dim3(blocks), dim3(block), 0, s, p->dparams, p->P, p->vmat, p->vstat,
                                d_image, pp->n_materials, p->partials);
-        hipLaunchKernelGGL(k_pt_reduce, dim3(pp->n_materials * 6), dim3(256), 0, s, p->partials, blocks,
-                           pp->n_materials, d_albedo, d_emission);
+            hipLaunchKernelGGL(k_pt_reduce<1>, dim3(pp->n_materials * 6), dim3(256), 0, s, p->partials, blocks,
+                               pp->n_materials, d_albedo, d_emission);
+        }
     }
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
