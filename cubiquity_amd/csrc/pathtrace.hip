@@ -14,10 +14,10 @@
 // rounded, so the same arithmetic on the CPU reproduces every path bit for bit.
 //
 // Forward, two forms with identical per-path arithmetic:
-//   wavefront  generate -> (intersect, shade) x (bounces + 1), captured once in a hipGraph per
-//              plan and replayed; ray counts live on the device, the persistent traversal kernel
-//              reads them; surviving rays are compacted by one atomic per
-//              1024-thread block
+//   wavefront  camera pass (rays, walk and first vertex in one kernel), then per bounce (walk, shade)
+//              over compacted lists of the surviving paths, captured once in a hipGraph per plan and
+//              replayed; path counts live on the device. On volumes without a packed copy, or with a
+//              launch shaped by the caller: generate -> (intersect, shade) x (bounces + 1)
 //   megakernel one lane per path, grid-stride
 // Both write per-path radiance; k_pt_resolve sums the samples of a pixel in sample order.
 // Adjoint (path replay): runs the wavefront pass again (each path's PCG stream makes it trace the
@@ -26,7 +26,7 @@
 //   G_K = sky if escaped else 0;  G_j = E_j + A_j G_{j+1};
 //   dV/dE_j = beta_j,  dV/dA_j = beta_j G_{j+1},
 // scaled by dL/dpixel / spp; partial sums in LDS, reduced over blocks in FP64.
-#include "device_internal.h"
+#include "walk_kernel.h"
 
 #include <algorithm>
 #include <cmath>
@@ -82,6 +82,24 @@ __device__ __forceinline__ Pcg pcg_seed(uint64_t initstate, uint64_t initseq)
     r.state += initstate;
     pcg_next(r);
     return r;
+}
+
+// A generator's state after `k` steps from (inc + initstate), where pcg_seed's second step starts:
+// mul * (inc + initstate) + add * inc with mul = M^k, add = 1 + M + ... + M^(k-1). A path that reaches
+// depth d has drawn 2 numbers for its camera ray and 2 per scatter, so its generator at depth d follows
+// from its pixel and sample: no state is stored.
+struct PcgJump {
+    uint64_t mul, add;
+};
+
+inline PcgJump pcg_jump(uint32_t depth)
+{
+    PcgJump j{ 1, 0 };
+    for (uint32_t k = 0; k < 1 + 2 + 2 * depth; k++) {
+        j.add = j.add * 6364136223846793005ULL + 1u;
+        j.mul *= 6364136223846793005ULL;
+    }
+    return j;
 }
 
 // uniform in [0, 1) with 24 random bits (exact conversion and scaling)
@@ -170,10 +188,98 @@ __device__ __forceinline__ void path_start(const PtDevParams& d, uint64_t p, Pcg
 
 // ---- wavefront kernels -----------------------------------------------------------------------
 
-// Camera rays and generator states of all paths. The paths' throughput (1) and radiance (0) are
-// not stored: the shading pass at depth 0, which sees every path, starts from those values.
+// The paths still alive at a depth: ray, path index and throughput per entry, in `parts` parts of `pcap`
+// slots, part k filled from its start up to count[k]. A kernel that writes a list claims its slots with
+// one atomicAdd per wave or block on the part's count. On one counter those claims serialise, at 13 ns
+// each: with 1024-thread blocks they alone were the 189 us of the first shading pass over 14.7 M paths.
+// Over 64 parts, each with its count on a cache line of its own, they overlap. The camera pass, whose
+// waves claim for 64 paths each, has a part per group of paths instead (path_group), so that rays of a
+// neighbourhood stay together in the next walk. Only the packed walk can be dealt such lists (PathRays):
+// other launches take one part.
+//
+// Units of a list are dealt in turn to the 8 XCDs (a unit is a workgroup), and the units past a part's
+// count are empty, so equal rows of the parts must not fall on equal XCDs: with row u % per for unit u,
+// the last of every 16 units empty, the first bounce's walk of 2^21 paths took 219 us, 180 rotated.
+constexpr uint32_t kParts = 64;
+constexpr uint32_t kCountStride = 32; // words: 128 bytes
+struct PathList {
+    cqx_ray* rays;
+    uint32_t* paths;
+    float* beta; // [3][slots]
+    uint32_t* count;
+    uint32_t parts, stride; // stride: words from a part's count to the next
+    uint64_t pcap, slots;   // slots >= parts * pcap
+    // Unit u (of `size` slots) as its part and its first row there. The camera pass's groups one after the
+    // other; kParts parts in turn, since consecutive groups of paths went to consecutive parts.
+    __device__ __forceinline__ void unit(uint32_t u, uint32_t size, uint32_t& part, uint64_t& row) const
+    {
+        if (parts > kParts) {
+            const uint32_t per = uint32_t((pcap + size - 1) / size);
+            part = u / per;
+            row = uint64_t((u + part) % per) * size;
+        } else {
+            part = (u + u / parts) % parts;
+            row = uint64_t(u / parts) * size;
+        }
+    }
+    uint32_t units(uint32_t size) const { return uint32_t(parts * ((pcap + size - 1) / size)); }
+};
+
+// Paths per part of the camera pass's list. Frame times (us) at groups of 256, 1024, 4096, 8192 paths and
+// with the 64 parts of the other lists: 2.1 M paths 512^3 adjoint 809 / 765 / 742 / 745 / 764, 7.4 M at
+// 1024^3 1595 / 1575 / 1553 / 1550 / 1575, 14.7 M at 1024^3 2462 / 2465 / 2398 / 2393 / 2402.
+inline uint32_t path_group(uint64_t P)
+{
+    uint32_t g = 64;
+    while (g < 4096 && uint64_t(g) * kParts < P) g *= 2;
+    return g;
+}
+
+// The bounce rays of a depth for the packed walk, with records of 8 bytes (time, info): the shading pass
+// needs no more. With them, the generators' states recomputed and radiance touched only where a vertex
+// adds to it, a bounce moves 88 bytes per ray between its two kernels instead of 152; shading passes of
+// the 14.7 M path frame at depths 1 to 4: 115, 70, 62, 35 -> 85, 50, 41, 26 us.
+struct PathRays {
+    static constexpr bool kUniform = true;
+    using Out = uint64_t;
+    PackedParams P;
+    PathList list;
+    uint64_t* __restrict__ hits;
+    __device__ __forceinline__ void fetch(uint64_t id, PackedParams&, const float*& ray, Out*& out) const
+    {
+        ray = reinterpret_cast<const float*>(list.rays + id);
+        out = hits + id;
+    }
+    __device__ __forceinline__ void deal(uint64_t w, uint32_t chunk, uint64_t, uint64_t& next, uint64_t& end) const
+    {
+        uint32_t part;
+        uint64_t at;
+        list.unit(uint32_t(w), chunk, part, at);
+        const uint64_t count = list.count[uint64_t(part) * list.stride];
+        const uint64_t first = part * list.pcap;
+        next = first + (at < count ? at : count);
+        end = first + (at + chunk < count ? at + chunk : count);
+    }
+    __device__ __forceinline__ void record(const PackedParams& T, const PackedRay& S, Out* dst) const
+    {
+        PackedHit h;
+        h.t = 0.0f;
+        h.info = S.phase == kAnomaly ? CQX_HIT_ANOMALY : 0u;
+        if (S.phase == kHit) (void)packed_hit(T, S, h);
+        __builtin_nontemporal_store(uint64_t(fbits(h.t)) | uint64_t(h.info) << 32, dst);
+    }
+};
+
+__global__ void __launch_bounds__(256) k_pt_clear(uint32_t* __restrict__ x, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) x[i] = 0u;
+}
+
+// Camera rays of all paths. The paths' throughput (1) and radiance (0) are not stored: the shading pass
+// at depth 0, which sees every path, starts from those values.
 __global__ void k_pt_generate(const PtDevParams* __restrict__ dp, uint64_t P, cqx_ray* __restrict__ rays,
-                              uint64_t* __restrict__ rng_state, uint32_t* __restrict__ count)
+                              uint32_t* __restrict__ count)
 {
     const uint64_t p = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (p == 0) *count = uint32_t(P);
@@ -189,84 +295,177 @@ __global__ void k_pt_generate(const PtDevParams* __restrict__ dp, uint64_t P, cq
         r.d[a] = dir[a];
     }
     rays[p] = r;
-    rng_state[p] = rng.state;
 }
 
-__global__ void k_set_u32(uint32_t* __restrict__ x, uint32_t v)
-{
-    if (threadIdx.x == 0) *x = v;
-}
-
-// kRadiance: the render's shading pass (throughput and radiance kept per path). Without it, the
-// adjoint's replay: the same paths, recording each vertex's material (vmat, vstat) only.
+// A path's vertex at `depth`: its contribution l, whether it goes on, and if so its next ray and its
+// throughput b. kRadiance: the render (throughput and radiance). Without it, the adjoint's replay: the
+// same paths, recording each vertex's material (vmat) and how the path ended (vstat) only.
 template <bool kRadiance>
-__global__ void __launch_bounds__(cqx::kCompactBlock) k_pt_shade(const PtDevParams* __restrict__ dp, uint64_t P, uint32_t depth,
-                                                  const uint32_t* __restrict__ count_cur,
-                                                  const cqx_ray* __restrict__ rays_cur,
-                                                  const uint32_t* __restrict__ paths_cur,
-                                                  const cqx_hit* __restrict__ hits, float* __restrict__ beta,
-                                                  float* __restrict__ L, uint64_t* __restrict__ rng_state,
-                                                  cqx_ray* __restrict__ rays_next, uint32_t* __restrict__ paths_next,
-                                                  uint32_t* __restrict__ count_next, uint8_t* __restrict__ vmat,
-                                                  uint8_t* __restrict__ vstat)
+__device__ __forceinline__ bool shade_vertex(const PtDevParams& d, uint64_t P, uint32_t depth, const PcgJump& jump, uint32_t p,
+                                             float t, uint32_t info, const float* o, const float* dir, float* b, float* l,
+                                             cqx_ray& next, uint8_t* __restrict__ vmat, uint8_t* __restrict__ vstat)
+{
+    for (int a = 0; a < 3; a++) l[a] = 0.0f;
+    if (info & CQX_HIT_ANOMALY) {
+        // traversal gave up on this ray: the path ends without a contribution
+        if (!kRadiance) vstat[p] = uint8_t(depth);
+        return false;
+    }
+    if (!(info & CQX_HIT_FLAG)) {
+        if (kRadiance)
+            for (int a = 0; a < 3; a++) l[a] = b[a] * d.sky[a];
+        else vstat[p] = uint8_t(depth | kEscaped);
+        return false;
+    }
+    const uint32_t m = (info >> 16) & 0xffu;
+    if (!kRadiance) vmat[depth * P + p] = uint8_t(m);
+    if (kRadiance)
+        for (int a = 0; a < 3; a++) l[a] = b[a] * d.emission[m * 3 + a];
+    bool cont = false;
+    if (depth < d.bounces) {
+        float pos[3], nrm[3];
+        for (int a = 0; a < 3; a++) pos[a] = o[a] + dir[a] * t;
+        decode_normal(info, nrm);
+        const uint32_t pixel = p / d.spp;
+        Pcg rng;
+        rng.inc = (uint64_t(p - pixel * d.spp) << 1u) | 1u;
+        rng.state = jump.mul * (rng.inc + ((d.seed << 32) + uint64_t(pixel))) + jump.add * rng.inc;
+        cont = scatter(d, rng, pos, nrm, next.o, next.d);
+        if (kRadiance)
+            for (int a = 0; a < 3; a++) b[a] = b[a] * d.albedo[m * 3 + a];
+    }
+    if (!kRadiance && !cont) vstat[p] = uint8_t(depth + 1);
+    return cont;
+}
+
+template <bool kRadiance>
+__device__ __forceinline__ void store_path(const PathList& list, uint64_t slot, const cqx_ray& next, uint32_t p, const float* b)
+{
+    list.rays[slot] = next;
+    list.paths[slot] = p;
+    if (kRadiance)
+        for (int a = 0; a < 3; a++) list.beta[a * list.slots + slot] = b[a];
+}
+
+// The camera pass on a packed volume: a path's camera ray, its walk (one ray per lane, `ids` per wave)
+// and its first vertex, in registers from one to the next: 14.7 M paths at 1024^3 in 582 us, with VALU
+// issue the bound as in the other walks. As three kernels (rays written once and read twice, 32-byte
+// records, claims on one counter) they took 66 + 573 + 189.
+template <bool kRadiance, bool kLod>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
+k_pt_camera(const PtDevParams* __restrict__ dp, uint64_t P, PackedParams T, uint32_t rows, uint32_t ids, PcgJump jump,
+            PathList next, float* __restrict__ L, uint8_t* __restrict__ vmat, uint8_t* __restrict__ vstat)
+{
+    extern __shared__ char lds_rows[];
+    __shared__ cqx_subdag lds_sub[8];
+    __shared__ float keep[3][64]; // the rays' directions, during the walk
+    const PtDevParams& d = *dp;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t base = lane_stack(lds_rows, rows, T.top);
+    const uint32_t occ = T.sub[0].pad1;
+    if (lane < 8) lds_sub[lane] = T.sub[lane];
+    __syncthreads();
+    const uint64_t first = uint64_t(blockIdx.x) * ids, p = first + lane;
+    const bool valid = lane < ids && p < P;
+    PackedRay S;
+    S.phase = kIdle;
+    if (valid) {
+        Pcg rng;
+        float o[3], dir[3];
+        uint32_t pixel;
+        path_start(d, p, rng, o, dir, pixel);
+        for (int a = 0; a < 3; a++) keep[a][lane] = dir[a];
+        ray_setup_packed(S, o[0], o[1], o[2], dir[0], dir[1], dir[2]);
+    }
+    do {
+        enter_octants_packed(lds_sub, T, S, lds_rows, base, occ);
+        while (__ballot(S.phase == kWalk)) walk_burst<kLod>(T, S, lds_rows, base, 12);
+        resolve_leave(S, occ);
+    } while (__ballot(S.phase == kLeave));
+    bool cont = false;
+    cqx_ray ray;
+    float b[3] = { 1.0f, 1.0f, 1.0f };
+    if (valid) {
+        PackedHit h;
+        h.t = 0.0f;
+        h.info = S.phase == kAnomaly ? CQX_HIT_ANOMALY : 0u;
+        if (S.phase == kHit) (void)packed_hit(T, S, h);
+        float dir[3], l[3];
+        for (int a = 0; a < 3; a++) dir[a] = keep[a][lane];
+        cont = shade_vertex<kRadiance>(d, P, 0u, jump, uint32_t(p), h.t, h.info, d.eye, dir, b, l, ray, vmat, vstat);
+        if (kRadiance)
+            for (int a = 0; a < 3; a++) L[a * P + p] = 0.0f + l[a];
+    }
+    const uint64_t alive = __ballot(cont);
+    if (!alive) return;
+    const uint32_t part = uint32_t(first / next.pcap);
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(next.count + uint64_t(part) * next.stride, uint32_t(__popcll(alive)));
+    at = uint32_t(__builtin_amdgcn_readfirstlane(at));
+    if (cont)
+        store_path<kRadiance>(next, part * next.pcap + at + uint32_t(__popcll(alive & ((1ull << lane) - 1ull))), ray,
+                              uint32_t(p), b);
+}
+
+// Threads of a shading block: claims on one counter need as few as possible, on kParts there is time.
+template <typename Hit>
+constexpr uint32_t kShadeBlock = sizeof(Hit) == sizeof(cqx_hit) ? cqx::kCompactBlock : 256u;
+
+__device__ __forceinline__ void read_hit(const cqx_hit& h, float& t, uint32_t& info)
+{
+    t = h.t;
+    info = h.info;
+}
+__device__ __forceinline__ void read_hit(const uint64_t& h, float& t, uint32_t& info)
+{
+    const uint64_t v = __builtin_nontemporal_load(&h);
+    t = bitsf(uint32_t(v));
+    info = uint32_t(v >> 32);
+}
+
+// The shading pass of a depth: a thread per slot, block b on part b % parts. Radiance is read and written
+// only where the vertex adds to it (a sky ray, an emissive material): adding a zero would keep its bits.
+template <bool kRadiance, typename Hit>
+__global__ void __launch_bounds__(kShadeBlock<Hit>) k_pt_shade(const PtDevParams* __restrict__ dp, uint64_t P, uint32_t depth,
+                                                               PcgJump jump, PathList cur, const Hit* __restrict__ hits,
+                                                               PathList next, float* __restrict__ L,
+                                                               uint8_t* __restrict__ vmat, uint8_t* __restrict__ vstat)
 {
     const PtDevParams& d = *dp;
-    const uint32_t n = *count_cur;
-    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    uint32_t part;
+    uint64_t row;
+    cur.unit(blockIdx.x, kShadeBlock<Hit>, part, row);
+    const uint64_t count = cur.count[uint64_t(part) * cur.stride];
+    if (row >= count) return;
+    const uint64_t i = part * cur.pcap + row + threadIdx.x;
     bool cont = false;
     uint32_t p = 0;
-    cqx_ray next;
-    if (i < n) {
-        // depth 0 holds every path in order, with throughput 1 and radiance 0
-        p = depth == 0 ? uint32_t(i) : paths_cur[i];
-        const cqx_hit h = hits[i];
-        float b[3] = { 1.0f, 1.0f, 1.0f }, l[3] = { 0.0f, 0.0f, 0.0f };
+    cqx_ray ray;
+    float b[3] = { 1.0f, 1.0f, 1.0f };
+    if (row + threadIdx.x < count) {
+        // depth 0 (on one part) holds every path in order, with throughput 1 and radiance 0
+        p = depth == 0 ? uint32_t(i) : cur.paths[i];
+        float t, l[3];
+        uint32_t info;
+        read_hit(hits[i], t, info);
         if (kRadiance && depth > 0)
-            for (int a = 0; a < 3; a++) {
-                b[a] = beta[a * P + p];
-                l[a] = L[a * P + p];
-            }
-        if (h.info & CQX_HIT_ANOMALY) {
-            // traversal gave up on this ray: the path ends without a contribution
-            if (vstat) vstat[p] = uint8_t(depth);
-        } else if (!(h.info & CQX_HIT_FLAG)) {
-            for (int a = 0; a < 3; a++) l[a] += b[a] * d.sky[a];
-            if (vstat) vstat[p] = uint8_t(depth | kEscaped);
-        } else {
-            const uint32_t m = (h.info >> 16) & 0xffu;
-            if (vstat) {
-                vmat[depth * P + p] = uint8_t(m);
-                vstat[p] = uint8_t(depth + 1);
-            }
-            for (int a = 0; a < 3; a++) l[a] += b[a] * d.emission[m * 3 + a];
-            if (depth < d.bounces) {
-                const cqx_ray r = rays_cur[i];
-                float pos[3], nrm[3];
-                for (int a = 0; a < 3; a++) pos[a] = r.o[a] + r.d[a] * h.t;
-                decode_normal(h.info, nrm);
-                Pcg rng;
-                rng.state = rng_state[p];
-                rng.inc = ((uint64_t(p % d.spp)) << 1u) | 1u;
-                if (scatter(d, rng, pos, nrm, next.o, next.d)) {
-                    rng_state[p] = rng.state;
-                    if (kRadiance)
-                        for (int a = 0; a < 3; a++) beta[a * P + p] = b[a] * d.albedo[m * 3 + a];
-                    cont = true;
-                }
-            }
+            for (int a = 0; a < 3; a++) b[a] = cur.beta[a * cur.slots + i];
+        const cqx_ray r = cur.rays[i];
+        cont = shade_vertex<kRadiance>(d, P, depth, jump, p, t, info, r.o, r.d, b, l, ray, vmat, vstat);
+        if (kRadiance) {
+            if (depth == 0)
+                for (int a = 0; a < 3; a++) L[a * P + p] = 0.0f + l[a];
+            else if (l[0] != 0.0f || l[1] != 0.0f || l[2] != 0.0f)
+                for (int a = 0; a < 3; a++) L[a * P + p] += l[a];
         }
-        if (kRadiance)
-            for (int a = 0; a < 3; a++) L[a * P + p] = l[a];
     }
-    // compact the surviving rays
+    if (depth >= d.bounces) return; // no path goes on
     const bool take[1] = { cont };
-    uint32_t* const counts[1] = { count_next };
+    const uint32_t to = part % next.parts;
+    uint32_t* const counts[1] = { next.count + to * next.stride };
     uint32_t slot[1];
-    cqx::block_slots<cqx::kCompactBlock>(take, counts, slot);
-    if (cont) {
-        rays_next[slot[0]] = next;
-        paths_next[slot[0]] = p;
-    }
+    cqx::block_slots<kShadeBlock<Hit>>(take, counts, slot);
+    if (cont) store_path<kRadiance>(next, to * next.pcap + slot[0], ray, p, b);
 }
 
 // Per-pixel mean of the samples, summed in sample order. With `staged`, each block first copies
@@ -606,14 +805,17 @@ struct PtPlan {
     cqx_launch_cfg cfg0{}; // traversal launch of the camera rays (depth 0)
     bool open = false;     // the caller left the launch open
     uint64_t P = 0;
+    uint32_t parts = 1; // shape of the path lists
+    uint64_t pcap = 0;
+    uint32_t groups = 0; // parts of the camera pass's list (packed)
+    size_t count_words(uint32_t depth) const { return groups + size_t(depth) * parts * kCountStride; } // counts before depth's
     PtDevParams* dparams = nullptr;
     cqx_ray* rays[2] = { nullptr, nullptr };
     uint32_t* paths[2] = { nullptr, nullptr };
-    cqx_hit* hits = nullptr;
-    float* beta = nullptr;
+    float* beta[2] = { nullptr, nullptr };
+    void* hits = nullptr; // cqx_hit, or 8-byte records on a packed volume
     float* L = nullptr;
-    uint64_t* rng = nullptr;
-    uint32_t* counts = nullptr;
+    uint32_t* counts = nullptr; // per depth, kCountStride words per part
     uint8_t* vmat = nullptr;  // (bounces + 1) x P vertex materials
     uint8_t* vstat = nullptr; // P path records (vertex count, escaped)
     float* partials = nullptr;
@@ -635,11 +837,10 @@ void destroy_pt_plan(PtPlan* p)
     for (int k = 0; k < 2; k++) {
         release(p->rays[k]);
         release(p->paths[k]);
+        release(p->beta[k]);
     }
     release(p->hits);
-    release(p->beta);
     release(p->L);
-    release(p->rng);
     release(p->counts);
     release(p->vmat);
     release(p->vstat);
@@ -757,53 +958,115 @@ cqx_status get_plan(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_params* p
     return CQX_OK;
 }
 
-// Allocates the wavefront buffers and captures generate -> (reset next count, intersect, shade) x
-// (bounces + 1) once into a graph.
-// The wavefront graph of the render (replay false) or of the adjoint's replay (replay true),
-// captured once per plan; the buffers they share are allocated with the first.
+// The wavefront graph of the render (replay false) or of the adjoint's replay (replay true), captured
+// once per plan; the buffers they share are allocated with the first. On a packed volume whose launch
+// the caller left open: camera pass, then (walk, shade) per bounce over lists in parts. Otherwise
+// generate, then (intersect, shade) per depth.
+template <bool kRadiance>
+cqx_status capture(cqx_ctx* ctx, PtPlan* p, hipStream_t s)
+{
+    const uint64_t P = p->P;
+    const bool packed = p->vol->packed_ok && p->open;
+    uint8_t* const vmat = kRadiance ? nullptr : p->vmat;
+    uint8_t* const vstat = kRadiance ? nullptr : p->vstat;
+    const uint64_t slots = p->parts * p->pcap;
+    const uint32_t group = path_group(P), groups = uint32_t((P + group - 1) / group);
+    const auto list = [&](uint32_t depth) {
+        const int k = int(depth & 1u);
+        if (packed && depth == 1) return PathList{ p->rays[k], p->paths[k], p->beta[k], p->counts, groups, 1u, group, slots };
+        return PathList{ p->rays[k], p->paths[k], p->beta[k], p->counts + p->count_words(depth), p->parts, kCountStride,
+                         p->pcap, slots };
+    };
+    const uint32_t all = uint32_t(p->count_words(p->bounces + 2));
+    hipLaunchKernelGGL(k_pt_clear, dim3((all + 255) / 256), dim3(256), 0, s, p->counts, all);
+    if (!packed) {
+        hipLaunchKernelGGL(k_pt_generate, dim3(uint32_t((P + 255) / 256)), dim3(256), 0, s, p->dparams, P, p->rays[0], p->counts);
+        cqx_hit* const hits = static_cast<cqx_hit*>(p->hits);
+        constexpr uint32_t block = kShadeBlock<cqx_hit>;
+        for (uint32_t depth = 0; depth <= p->bounces; depth++) {
+            const cqx_status st =
+                cqx::launch_intersect(ctx, p->vol, p->rays[depth & 1u], P, list(depth).count, CQX_SURFACE_PROPERTIES,
+                                      p->max_footprint, hits, depth == 0 ? &p->cfg0 : &p->cfg, s);
+            if (st != CQX_OK) return st;
+            hipLaunchKernelGGL((k_pt_shade<kRadiance, cqx_hit>), dim3(uint32_t((P + block - 1) / block)), dim3(block), 0, s,
+                               p->dparams, P, depth, pcg_jump(depth), list(depth), hits, list(depth + 1), p->L, vmat, vstat);
+        }
+        return CQX_OK;
+    }
+    bool lod = false;
+    const PackedParams T = packed_params(p->vol, 1u, p->cfg.max_iters ? p->cfg.max_iters : cqx::kDefaultMaxIters,
+                                         p->max_footprint, lod);
+    const uint32_t rows = T.top + 1u, ids = cqx::lanes_per_wave(P);
+    const size_t lds = size_t(rows) * kRowBytes;
+    const dim3 camera(uint32_t((P + ids - 1) / ids));
+    if (lod)
+        hipLaunchKernelGGL((k_pt_camera<kRadiance, true>), camera, dim3(64), lds, s, p->dparams, P, T, rows, ids,
+                           pcg_jump(0), list(1), p->L, vmat, vstat);
+    else
+        hipLaunchKernelGGL((k_pt_camera<kRadiance, false>), camera, dim3(64), lds, s, p->dparams, P, T, rows, ids,
+                           pcg_jump(0), list(1), p->L, vmat, vstat);
+    uint64_t* const hits = static_cast<uint64_t*>(p->hits);
+    const uint32_t chunk = cqx::dealt_ids(P);
+    constexpr uint32_t block = kShadeBlock<uint64_t>;
+    for (uint32_t depth = 1; depth <= p->bounces; depth++) {
+        const PathRays src{ T, list(depth), hits };
+        const dim3 walk(src.list.units(chunk)), shade(src.list.units(block));
+        const uint32_t refill = chunk > 64 ? 16u : 64u;
+        if (lod)
+            hipLaunchKernelGGL((k_walk<PathRays, true, true>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 12u, refill,
+                               rows, chunk, nullptr, 0u);
+        else
+            hipLaunchKernelGGL((k_walk<PathRays, false, true>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 12u, refill,
+                               rows, chunk, nullptr, 0u);
+        hipLaunchKernelGGL((k_pt_shade<kRadiance, uint64_t>), shade, dim3(block), 0, s, p->dparams, P, depth,
+                           pcg_jump(depth), list(depth), hits, list(depth + 1), p->L, vmat, vstat);
+    }
+    return CQX_OK;
+}
+
 cqx_status ensure_wavefront(cqx_ctx* ctx, PtPlan* p, bool replay)
 {
     if (replay ? p->exec_replay : p->exec) return CQX_OK;
-    const uint64_t P = p->P;
     cqx_status st = CQX_OK;
     if (!p->hits) {
+        const bool packed = p->vol->packed_ok && p->open;
+        const uint64_t group = path_group(p->P), groups = (p->P + group - 1) / group;
+        p->parts = packed ? uint32_t(std::min<uint64_t>(kParts, groups)) : 1u;
+        p->pcap = packed ? (groups + p->parts - 1) / p->parts * group : p->P;
+        const uint64_t slots = p->parts * p->pcap;
         for (int k = 0; k < 2 && st == CQX_OK; k++) {
-            st = alloc(&p->rays[k], P);
-            if (st == CQX_OK) st = alloc(&p->paths[k], P);
+            st = alloc(&p->rays[k], slots);
+            if (st == CQX_OK) st = alloc(&p->paths[k], slots);
+            if (st == CQX_OK) st = alloc(&p->beta[k], 3 * slots);
         }
-        if (st == CQX_OK) st = alloc(&p->hits, P);
-        if (st == CQX_OK) st = alloc(&p->beta, 3 * P);
-        if (st == CQX_OK) st = alloc(&p->rng, P);
-        if (st == CQX_OK) st = alloc(&p->counts, 64);
+        p->groups = packed ? uint32_t(groups) : 0u;
+        if (st == CQX_OK) st = alloc(&p->counts, p->count_words(p->bounces + 2));
+        if (st == CQX_OK) {
+            uint8_t* hits = nullptr;
+            st = alloc(&hits, slots * (packed ? sizeof(uint64_t) : sizeof(cqx_hit)));
+            p->hits = hits;
+        }
+        if (st != CQX_OK) { // all or none, so that a later call starts over
+            for (int k = 0; k < 2; k++) {
+                release(p->rays[k]);
+                release(p->paths[k]);
+                release(p->beta[k]);
+                p->rays[k] = nullptr;
+                p->paths[k] = nullptr;
+                p->beta[k] = nullptr;
+            }
+            release(p->counts);
+            p->counts = nullptr;
+        }
     }
     if (st == CQX_OK && replay && !p->vstat) { // the adjoint's path record
-        st = alloc(&p->vmat, (p->bounces + 1) * P);
-        if (st == CQX_OK) st = alloc(&p->vstat, P);
+        st = alloc(&p->vmat, (p->bounces + 1) * p->P);
+        if (st == CQX_OK) st = alloc(&p->vstat, p->P);
     }
     if (st != CQX_OK) return st;
     hipStream_t s = ctx->capture_stream;
     HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    const uint32_t gb = uint32_t((P + 255) / 256);
-    const uint32_t gc = uint32_t((P + cqx::kCompactBlock - 1) / cqx::kCompactBlock);
-    hipLaunchKernelGGL(k_pt_generate, dim3(gb), dim3(256), 0, s, p->dparams, P, p->rays[0], p->rng, p->counts + 0);
-    cqx_status cst = CQX_OK;
-    for (uint32_t depth = 0; depth <= p->bounces && cst == CQX_OK; depth++) {
-        const int cur = depth & 1, nxt = cur ^ 1;
-        uint32_t* cnt_cur = p->counts + cur * 16;
-        uint32_t* cnt_next = p->counts + nxt * 16;
-        hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, s, cnt_next, 0u);
-        cst = cqx::launch_intersect(ctx, p->vol, p->rays[cur], P, cnt_cur, CQX_SURFACE_PROPERTIES, p->max_footprint,
-                                    p->hits, depth == 0 ? &p->cfg0 : &p->cfg, s, nullptr,
-                                    depth && p->open ? cqx::dealt_ids(p->P) : 0u);
-        if (replay)
-            hipLaunchKernelGGL(k_pt_shade<false>, dim3(gc), dim3(cqx::kCompactBlock), 0, s, p->dparams, P, depth, cnt_cur,
-                               p->rays[cur], p->paths[cur], p->hits, p->beta, p->L, p->rng, p->rays[nxt], p->paths[nxt],
-                               cnt_next, p->vmat, p->vstat);
-        else
-            hipLaunchKernelGGL(k_pt_shade<true>, dim3(gc), dim3(cqx::kCompactBlock), 0, s, p->dparams, P, depth, cnt_cur,
-                               p->rays[cur], p->paths[cur], p->hits, p->beta, p->L, p->rng, p->rays[nxt], p->paths[nxt],
-                               cnt_next, nullptr, nullptr);
-    }
+    const cqx_status cst = replay ? capture<false>(ctx, p, s) : capture<true>(ctx, p, s);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(s, &g);
     (replay ? p->graph_replay : p->graph) = g;

@@ -18,7 +18,7 @@
 //                           into a coarse Morton grid over the origins' bounds, handed out cell
 //                           by cell
 // All keep the traversal stack in LDS (one column per lane, one row per node height).
-#include "device_internal.h"
+#include "walk_kernel.h"
 
 #include <algorithm>
 #include <cmath>
@@ -65,11 +65,6 @@ __global__ void __launch_bounds__(256) k_intersect_lane(TraceParams P, const cqx
 // (blockIdx.x % 8, the order in which workgroups are spread over the XCDs), so waves of one XCD
 // draw from their own counter; a wave whose queue is drained moves on to the next queue. A wave
 // exits when every queue is drained and all its lanes are idle.
-constexpr int kQueues = 8;
-constexpr int kCounterStride = 16; // queue counters 128 bytes apart: one cache line each
-constexpr int kFlagWord = 8;       // the sampled flag of gated launches, in the first counter's line
-static_assert(kFlagWord < kCounterStride && kFlagWord % kCounterStride != 0, "a word no counter uses");
-
 __global__ void k_reset_counters(unsigned long long* counters)
 {
     if (threadIdx.x < kQueues) counters[threadIdx.x * kCounterStride] = 0;
@@ -83,14 +78,6 @@ __device__ __forceinline__ void setup_from(RayState& S, const float* r)
 #pragma unroll
     for (int i = 0; i < 6; i++) v[i] = __builtin_nontemporal_load(r + i);
     ray_setup(S, v[0], v[1], v[2], v[3], v[4], v[5]);
-}
-
-__device__ __forceinline__ void store_record(cqx_hit* dst, const cqx_hit& h)
-{
-    const uint32_t* s = reinterpret_cast<const uint32_t*>(&h);
-    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-#pragma unroll
-    for (int i = 0; i < 8; i++) __builtin_nontemporal_store(s[i], d + i);
 }
 
 // Where a persistent wave's ray ids come from. SingleSource: one volume, one ray array; its
@@ -353,7 +340,7 @@ __global__ void __launch_bounds__(256) k_intersect_pair(SingleSource src, uint64
 // k_walk serves the launches of k_intersect_lane and k_intersect_persistent (variants 1 and 2) on a
 // volume's packed copy (walk_packed.h) with the same records, whenever every volume of the launch has one.
 
-struct PackedSingle {
+struct PackedSingle : OneRange {
     static constexpr bool kUniform = true;
     PackedParams P;
     const cqx_ray* __restrict__ rays;
@@ -391,7 +378,7 @@ struct TableDescs {
 };
 
 template <typename Descs>
-struct PackedBatch {
+struct PackedBatch : OneRange {
     static constexpr bool kUniform = false;
     Descs desc;
     uint32_t n_batches;
@@ -420,153 +407,6 @@ struct PackedBatch {
         out = b.hits + k;
     }
 };
-
-__device__ __forceinline__ const PackedParams& uniform_params(const PackedSingle& s, const PackedParams&) { return s.P; }
-template <typename Descs>
-__device__ __forceinline__ const PackedParams& uniform_params(const PackedBatch<Descs>&, const PackedParams& lane)
-{
-    return lane;
-}
-
-__device__ __forceinline__ void setup_packed(PackedRay& S, const float* r)
-{
-    float v[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) v[i] = __builtin_nontemporal_load(r + i);
-    ray_setup_packed(S, v[0], v[1], v[2], v[3], v[4], v[5]);
-}
-
-// The lane's stack_base(): its wave's `rows` rows of the workgroup's LDS, its own word of each.
-__device__ __forceinline__ uint32_t lane_stack(char* rows_lds, uint32_t rows, uint32_t top)
-{
-    // the low 32 bits of a generic LDS address are the LDS address
-    const uint32_t lds = uint32_t(reinterpret_cast<uintptr_t>(rows_lds));
-    return stack_base(lds + (threadIdx.x >> 6) * rows * kRowBytes + (threadIdx.x & 63u) * 4u, top);
-}
-
-// Up to `steps` steps of the wave's walking lanes: the plain rays' step when every walking lane may
-// take it (its ray plain, its iterations far enough from the cap), the general one otherwise.
-template <bool kLod>
-__device__ __forceinline__ void walk_burst(const PackedParams& P, PackedRay& S, char* lds, uint32_t base, uint32_t steps)
-{
-    const bool walking = S.phase == kWalk;
-    const uint32_t room = P.max_iters >= 2u * steps ? P.max_iters - 2u * steps : 0u;
-    const bool odd = walking && (!S.plain || S.iters > room || P.max_iters < 2u * steps);
-    if (__ballot(odd)) {
-        for (uint32_t k = 0; k < steps; k++)
-            if (S.phase == kWalk) walk_step_packed_any(P, S, lds, base);
-    } else {
-        for (uint32_t k = 0; k < steps; k++)
-            if (S.phase == kWalk) walk_step_packed<kLod>(P, S, lds, base);
-    }
-}
-
-__device__ __forceinline__ uint64_t uniform64(uint64_t v)
-{
-    return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v)))) |
-           uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v >> 32)))) << 32;
-}
-
-// What a wave does is the same in both forms; they differ in where its ray ids come from.
-//   dealt (kDealt)  wave w owns ids [w * chunk, (w + 1) * chunk): no counters, no claims, the hardware's
-//                   dispatcher balances the load. With chunk <= 64 and refill 64 it is one ray per lane.
-//   claimed         persistent waves claim `chunk` ids at a time from the queues' counters
-// `gate`: a launch that runs only when the sampled flag there equals `want` (k_sample_rays).
-// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take it to 6.
-template <typename Source, bool kLod, bool kDealt>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6)))
-k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
-       uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk, const unsigned long long* __restrict__ gate,
-       uint32_t want)
-{
-    extern __shared__ char lds_rows[];
-    if (gate && *gate != want) return;
-    if (n_dev) {
-        const uint64_t nd = *n_dev;
-        n = nd < n ? nd : n;
-    }
-    PackedParams P;
-    cqx_hit* dst = nullptr;
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t base;
-    if constexpr (Source::kUniform) base = lane_stack(lds_rows, rows, src.P.top);
-    else base = lane_stack(lds_rows, rows, src.top);
-
-    PackedRay S;
-    S.phase = kIdle;
-    __shared__ cqx_subdag lds_sub[8];
-    const cqx_subdag* tab = lds_sub;
-    uint32_t occ = 0u; // occupied octants of the launch's (a lane's) volume
-    if constexpr (Source::kUniform) {
-        occ = src.P.sub[0].pad1;
-        if (threadIdx.x < 8) lds_sub[threadIdx.x] = src.P.sub[threadIdx.x];
-        __syncthreads();
-    }
-    const uint64_t per_q = (n + kQueues - 1) / kQueues;
-    uint32_t qc = blockIdx.x % kQueues; // current queue
-    uint32_t drained = 0;               // queues found empty so far
-    uint64_t c_next = 0, c_end = 0;     // ray ids claimed by this wave
-    if constexpr (kDealt) {
-        const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
-        const uint64_t at = (uint64_t(blockIdx.x) * (blockDim.x >> 6) + wave) * chunk;
-        c_next = at < n ? at : n;
-        c_end = at + chunk < n ? at + chunk : n;
-        drained = kQueues;
-    }
-
-    for (;;) {
-        // A service pass runs once `refill` lanes wait, or none walks: misses of lanes that left their
-        // last SubDAG, records of the finished lanes, new rays for the idle ones, then the next SubDAG
-        // of every lane between SubDAGs (one copy of that code, for new and continuing rays; a ray
-        // that turns out to miss there has its record written by the next pass).
-        const uint64_t walking = __ballot(S.phase == kWalk);
-        const uint32_t nwait = 64u - uint32_t(__popcll(walking));
-        if (nwait >= refill || walking == 0) {
-            resolve_leave(S, occ);
-            if (is_finished(S.phase)) {
-                cqx_hit out;
-                emit_packed(uniform_params(src, P), S, out);
-                store_record(dst, out);
-                S.phase = kIdle;
-            }
-            while (c_next == c_end && drained < kQueues) {
-                const uint64_t q_begin = per_q * qc;
-                const uint64_t q_end = q_begin + per_q < n ? q_begin + per_q : n;
-                const uint64_t q_len = q_end > q_begin ? q_end - q_begin : 0;
-                unsigned long long claim = 0;
-                if (lane == 0) claim = atomicAdd(&counters[qc * kCounterStride], (unsigned long long)chunk);
-                claim = uniform64(claim);
-                if (claim < q_len) {
-                    c_next = q_begin + claim;
-                    c_end = q_begin + (claim + chunk < q_len ? claim + chunk : q_len);
-                } else {
-                    qc = (qc + 1) % kQueues;
-                    drained++;
-                }
-            }
-            const uint64_t idle = __ballot(S.phase == kIdle);
-            if (S.phase == kIdle) {
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
-                const uint64_t k = c_next + rank;
-                if (k < c_end) {
-                    const float* r;
-                    src.fetch(k, P, r, dst);
-                    setup_packed(S, r);
-                    if constexpr (!Source::kUniform) {
-                        tab = P.sub;
-                        occ = P.sub[0].pad1;
-                    }
-                }
-            }
-            const uint64_t nidle = uint64_t(__popcll(idle));
-            c_next = c_next + nidle < c_end ? c_next + nidle : c_end;
-            if (drained == kQueues && c_next == c_end && __ballot(S.phase != kIdle) == 0) break;
-            enter_octants_packed(tab, uniform_params(src, P), S, lds_rows, base, occ);
-        }
-        walk_burst<kLod>(uniform_params(src, P), S, lds_rows, base, regroup);
-    }
-}
 
 // Whether a batch's rays are coherent (camera rays, sun shadow rays): of 64 pairs of neighbouring rays
 // spread over the array, at least 56 have nearly equal directions (cosine above 0.97) and origins
@@ -1162,15 +1002,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
     PackedParams PP{};
     bool lod = false;
     if (packed) {
-        PP.packed = vol->packed;
-        PP.sub = vol->sub;
-        PP.surf = P.surf;
-        PP.max_iters = P.max_iters;
-        PP.top = uint32_t(vol->max_height);
-        PP.fp_disabled = P.fp_disabled;
-        PP.max_footprint = max_footprint;
-        lod_thresholds(max_footprint, PP.lod_hi, PP.lod_lo);
-        lod = !std::isinf(PP.lod_hi);
+        PP = packed_params(vol, P.surf, P.max_iters, max_footprint, lod);
     }
 
     const uint32_t bin_bits = cfg ? cfg->bin_bits : 0u;
@@ -1187,7 +1019,7 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
         }
     }
     if (packed) {
-        const PackedSingle src{ PP, rays, hits, order };
+        const PackedSingle src{ {}, PP, rays, hits, order };
         const bool open = launch_open(cfg);
         uint32_t blocks = 0, regroup = 0, refill = 0, chunk = 0;
         if (variant == 2) {
@@ -1636,7 +1468,7 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     const WalkLaunch walk{ lod, cqx::launch_open(cfg) && total <= kDealtBatchRays, uint32_t(max_height), block, blocks,
                            regroup, refill, chunk, counters };
     if (packed && n_batches <= kInlineBatches) {
-        PackedBatch<InlineDescs> src{ {}, n_batches, max_iters, uint32_t(max_height) };
+        PackedBatch<InlineDescs> src{ {}, {}, n_batches, max_iters, uint32_t(max_height) };
         std::copy(pdesc.begin(), pdesc.end(), src.desc.d);
         launch_batch(src, walk, total, s);
         HIP_TRY(hipGetLastError());
@@ -1655,7 +1487,7 @@ cqx_status cqx_intersect_batched(cqx_ctx* ctx, const cqx_batch* batches, uint32_
     HIP_TRY(hipMemcpy(ctx->batch_desc, packed ? static_cast<const void*>(pdesc.data()) : desc.data(), bytes,
                       hipMemcpyHostToDevice));
     if (packed) {
-        launch_batch(PackedBatch<TableDescs>{ { static_cast<const PackedDesc*>(ctx->batch_desc) }, n_batches, max_iters,
+        launch_batch(PackedBatch<TableDescs>{ {}, { static_cast<const PackedDesc*>(ctx->batch_desc) }, n_batches, max_iters,
                                               uint32_t(max_height) }, walk, total, s);
         HIP_TRY(hipGetLastError());
         return CQX_OK;

@@ -510,8 +510,53 @@ __device__ __forceinline__ uint32_t entered_voxel_plain(float o, float d, float 
     return fbits((entry_axis ? lo : c) + kBias) - kBiasBits;
 }
 
-// Record of a finished ray: emit_record of traverse_core.h from the packed walk's state. The
-// nearest material takes the first occupied child from the node's mask: one read per level.
+// The hit of a finished ray (phase kHit): its time and info word (with P.surf the normal and the nearest
+// material, which takes the first occupied child from the node's mask: one read per level), and which
+// axes it entered by. False (info CQX_HIT_ANOMALY) where the material's descent meets an empty node.
+struct PackedHit {
+    float t;
+    uint32_t info;
+    uint32_t entries; // with the material's descent
+    bool ex, ey, ez;
+};
+
+__device__ __forceinline__ bool packed_hit(const PackedParams& P, const PackedRay& S, PackedHit& h)
+{
+    const uint32_t slot = S.cid ^ S.sign_bits;
+    const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
+    const float t0x = (px - S.ox) * S.ix, t0y = (py - S.oy) * S.iy, t0z = (pz - S.oz) * S.iz;
+    h.t = max3f(t0x, t0y, t0z);
+    h.ex = h.t == t0x;
+    h.ey = h.t == t0y;
+    h.ez = h.t == t0z;
+    h.entries = S.entries;
+    const float bsize = S.s > 0.0f ? S.s : 1.0f; // a SubDAG of height 0: the node itself, of side 1
+    h.info = 1u | (slot << 1) | (((fbits(bsize) >> 23) - 127u) << 4);
+    if (!P.surf) return true;
+    uint32_t m = S.word;
+    while (m >= (kMaterialCount << 8)) {
+        h.entries++;
+        const uint32_t mask = m & 0xffu;
+        if (mask == 0) {
+            h.info = CQX_HIT_ANOMALY;
+            return false;
+        }
+        uint32_t ids = (0x76534210u | 0x88888888u) ^ (S.sign_bits * 0x11111111u);
+        while (!((mask >> (ids & 7u)) & 1u)) ids >>= 4;
+        m = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(P.packed) +
+                                               (((m >> 3) & ~31u) | ((ids & 7u) << 2)));
+    }
+    // normal = vec3(equal(tEntry, childT0)) * -rayDirSign, raytracing.cpp:317-318: magnitude 1 on
+    // the entry axes, and the sign bit of -rayDirSign on every axis (0 * -1 = -0)
+    h.info |= (h.ex ? 1u << 9 : 0u) | (h.ey ? 1u << 11 : 0u) | (h.ez ? 1u << 13 : 0u);
+    h.info |= (S.sign_bits & 1u) ? 0u : 1u << 10;
+    h.info |= (S.sign_bits & 2u) ? 0u : 1u << 12;
+    h.info |= (S.sign_bits & 4u) ? 0u : 1u << 14;
+    h.info |= (m >> 8) << 16;
+    return true;
+}
+
+// Record of a finished ray: emit_record of traverse_core.h from the packed walk's state.
 __device__ __forceinline__ void emit_packed(const PackedParams& P, const PackedRay& S, cqx_hit& out)
 {
     result_miss(out);
@@ -519,56 +564,30 @@ __device__ __forceinline__ void emit_packed(const PackedParams& P, const PackedR
     out.iters = S.iters;
     out.info = S.phase == kAnomaly ? CQX_HIT_ANOMALY : 0u;
     if (S.phase != kHit) return;
-    const uint32_t slot = S.cid ^ S.sign_bits;
+    PackedHit h;
+    const bool found = packed_hit(P, S, h);
+    out.entries = h.entries;
+    out.info = h.info;
+    if (!found) return;
     const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
-    const float t0x = (px - S.ox) * S.ix, t0y = (py - S.oy) * S.iy, t0z = (pz - S.oz) * S.iz;
-    const float tce = max3f(t0x, t0y, t0z);
-    const bool ex = tce == t0x, ey = tce == t0y, ez = tce == t0z;
-    const float bsize = S.s > 0.0f ? S.s : 1.0f; // a SubDAG of height 0: the node itself, of side 1
-    uint32_t info = 1u | (slot << 1) | (((fbits(bsize) >> 23) - 127u) << 4);
-    if (P.surf) {
-        uint32_t m = S.word;
-        uint32_t entries = S.entries;
-        while (m >= (kMaterialCount << 8)) {
-            entries++;
-            const uint32_t mask = m & 0xffu;
-            if (mask == 0) {
-                out.entries = entries;
-                out.info = CQX_HIT_ANOMALY;
-                return;
-            }
-            uint32_t ids = (0x76534210u | 0x88888888u) ^ (S.sign_bits * 0x11111111u);
-            while (!((mask >> (ids & 7u)) & 1u)) ids >>= 4;
-            m = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(P.packed) +
-                                                   (((m >> 3) & ~31u) | ((ids & 7u) << 2)));
-        }
-        out.entries = entries;
-        // normal = vec3(equal(tEntry, childT0)) * -rayDirSign, raytracing.cpp:317-318: magnitude 1 on
-        // the entry axes, and the sign bit of -rayDirSign on every axis (0 * -1 = -0)
-        info |= (ex ? 1u << 9 : 0u) | (ey ? 1u << 11 : 0u) | (ez ? 1u << 13 : 0u);
-        info |= (S.sign_bits & 1u) ? 0u : 1u << 10;
-        info |= (S.sign_bits & 2u) ? 0u : 1u << 12;
-        info |= (S.sign_bits & 4u) ? 0u : 1u << 14;
-        info |= (m >> 8) << 16;
-    }
+    const float bsize = S.s > 0.0f ? S.s : 1.0f;
     uint32_t vx, vy, vz;
     if (S.plain) {
         const float ext = bsize - 1.0f;
-        vx = entered_voxel_plain(S.ox, S.dx, tce, px, px + ext, ex);
-        vy = entered_voxel_plain(S.oy, S.dy, tce, py, py + ext, ey);
-        vz = entered_voxel_plain(S.oz, S.dz, tce, pz, pz + ext, ez);
+        vx = entered_voxel_plain(S.ox, S.dx, h.t, px, px + ext, h.ex);
+        vy = entered_voxel_plain(S.oy, S.dy, h.t, py, py + ext, h.ey);
+        vz = entered_voxel_plain(S.oz, S.dz, h.t, pz, pz + ext, h.ez);
     } else {
         const int32_t size = int32_t(bsize);
-        vx = uint32_t(entered_voxel(S.ox, S.dx, tce, int32_t(px), size, ex));
-        vy = uint32_t(entered_voxel(S.oy, S.dy, tce, int32_t(py), size, ey));
-        vz = uint32_t(entered_voxel(S.oz, S.dz, tce, int32_t(pz), size, ez));
+        vx = uint32_t(entered_voxel(S.ox, S.dx, h.t, int32_t(px), size, h.ex));
+        vy = uint32_t(entered_voxel(S.oy, S.dy, h.t, int32_t(py), size, h.ey));
+        vz = uint32_t(entered_voxel(S.oz, S.dz, h.t, int32_t(pz), size, h.ez));
     }
     out.voxel[0] = int32_t(vx ^ (0u - (S.sign_bits & 1u)));
     out.voxel[1] = int32_t(vy ^ (0u - ((S.sign_bits >> 1) & 1u)));
     out.voxel[2] = int32_t(vz ^ (0u - (S.sign_bits >> 2)));
-    out.t = tce;
+    out.t = h.t;
     out.node = S.node >> 8;
-    out.info = info;
 }
 
 } // namespace cqxd
