@@ -246,9 +246,8 @@ __global__ void __launch_bounds__(cqx::kCompactBlock) k_demo_primary(DemoDev d, 
         }
     }
     const bool take[3] = { hit && d.include_sun, hit && d.include_sky, hit };
-    uint32_t* const counts[3] = { sec_count, sec_count, sec_count };
     uint32_t k[3];
-    cqx::block_slots<cqx::kCompactBlock>(take, counts, k);
+    cqx::block_slots<cqx::kCompactBlock>(take, sec_count, k);
     const cqx_ray r[3] = { sun, sky, refl };
     const uint32_t kind[3] = { kSun0, kSky0, kRefl };
 #pragma unroll
@@ -307,9 +306,8 @@ __global__ void __launch_bounds__(cqx::kCompactBlock) k_demo_bounce(DemoDev d, u
         }
     }
     const bool take[2] = { hit && d.include_sun, hit && d.include_sky };
-    uint32_t* const counts[2] = { sh_count, sh_count };
     uint32_t k[2];
-    cqx::block_slots<cqx::kCompactBlock>(take, counts, k);
+    cqx::block_slots<cqx::kCompactBlock>(take, sh_count, k);
     if (take[0]) {
         sh_rays[k[0]] = sun;
         sh_tags[k[0]] = p * 4u + kSun1;

@@ -462,9 +462,8 @@ __global__ void __launch_bounds__(kShadeBlock<Hit>) k_pt_shade(const PtDevParams
     if (depth >= d.bounces) return; // no path goes on
     const bool take[1] = { cont };
     const uint32_t to = part % next.parts;
-    uint32_t* const counts[1] = { next.count + to * next.stride };
     uint32_t slot[1];
-    cqx::block_slots<kShadeBlock<Hit>>(take, counts, slot);
+    cqx::block_slots<kShadeBlock<Hit>>(take, next.count + to * next.stride, slot);
     if (cont) store_path<kRadiance>(next, to * next.pcap + slot[0], ray, p, b);
 }
 
