@@ -30,6 +30,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <new>
 
@@ -55,9 +56,22 @@ struct PtDevParams {
     uint32_t width, height, spp, bounces;
     uint32_t pad;
     uint64_t seed;
+    float* image;            // the render's output
     float albedo[256 * 3];   // by material id
     float emission[256 * 3]; // by material id
 };
+
+// A call's parameters as kernel arguments (at most 4 KiB): all but the material tables, then the
+// materials [first, first + kArgMaterials).
+constexpr uint32_t kArgMaterials = 128;
+constexpr uint32_t kHeadWords = offsetof(PtDevParams, albedo) / 4;
+struct PtArgs {
+    uint32_t head[kHeadWords];
+    uint32_t first;
+    float albedo[kArgMaterials * 3];
+    float emission[kArgMaterials * 3];
+};
+static_assert(sizeof(PtArgs) < 4000 && 2 * kArgMaterials == 256, "two launches hold the tables");
 
 // ---- PCG32 (O'Neill 2014) ---------------------------------------------------------------------
 struct Pcg {
@@ -270,10 +284,18 @@ struct PathRays {
     }
 };
 
-__global__ void __launch_bounds__(256) k_pt_clear(uint32_t* __restrict__ x, uint32_t n)
+// Starts a call: its parameters to the device and the path counts cleared, one launch for a copy from
+// host memory and a clear (a kernel each).
+__global__ void __launch_bounds__(256) k_pt_begin(PtArgs args, PtDevParams* __restrict__ dp, uint32_t* __restrict__ counts,
+                                                  uint32_t n)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) x[i] = 0u;
+    if (i < kHeadWords) reinterpret_cast<uint32_t*>(dp)[i] = args.head[i];
+    if (i < kArgMaterials * 3) {
+        dp->albedo[args.first * 3 + i] = args.albedo[i];
+        dp->emission[args.first * 3 + i] = args.emission[i];
+    }
+    for (uint32_t k = i; k < n; k += gridDim.x * 256) counts[k] = 0u;
 }
 
 // Camera rays of all paths. The paths' throughput (1) and radiance (0) are not stored: the shading pass
@@ -467,33 +489,41 @@ __global__ void __launch_bounds__(kShadeBlock<Hit>) k_pt_shade(const PtDevParams
     if (cont) store_path<kRadiance>(next, to * next.pcap + slot[0], ray, p, b);
 }
 
-// Per-pixel mean of the samples, summed in sample order. With `staged`, each block first copies
-// its pixels' samples of one channel (contiguous in L) to LDS with coalesced reads, then each
-// thread sums its pixel's row there; otherwise threads read L directly (spp too large for LDS).
+// Per-pixel mean of the samples, summed in sample order; channel blockIdx.y of 256 pixels per block.
+// With `staged`, a block first copies its pixels' samples (contiguous in L) to LDS with coalesced reads,
+// then each thread sums its pixel's row there (a word of padding per 32, so that rows of 2^k samples do
+// not share banks); otherwise threads read L directly (spp too large for LDS). 1280x720x16: 75 us with
+// the three channels in turn and without padding, 33 us so (177 MB at 5.3 TB/s, the rate of a copy).
+constexpr uint32_t resolve_words(uint32_t samples) { return samples + (samples >> 5) + 1u; }
+
 __global__ void __launch_bounds__(256) k_pt_resolve(const PtDevParams* __restrict__ dp, uint64_t P,
-                                                    const float* __restrict__ L, float* __restrict__ image,
-                                                    uint32_t staged)
+                                                    const float* __restrict__ L, uint32_t staged)
 {
-    extern __shared__ float tile[]; // blockDim.x x spp floats when staged
+    extern __shared__ float tile[]; // resolve_words(256 * spp) when staged
     const PtDevParams& d = *dp;
-    const uint32_t pixels = d.width * d.height, spp = d.spp;
-    const uint32_t q0 = blockIdx.x * blockDim.x; // < pixels: the grid covers the pixels once
+    const uint32_t pixels = d.width * d.height, spp = d.spp, a = blockIdx.y;
+    const uint32_t q0 = blockIdx.x * 256; // < pixels: the grid covers the pixels once
     const uint32_t q = q0 + threadIdx.x;
-    const uint32_t npix = pixels - q0 < blockDim.x ? pixels - q0 : blockDim.x;
-    for (int a = 0; a < 3; a++) {
-        float sum = 0.0f;
-        if (staged) {
-            const float* src = L + a * P + uint64_t(q0) * spp;
-            for (uint32_t k = threadIdx.x; k < npix * spp; k += blockDim.x) tile[k] = src[k];
-            __syncthreads();
-            if (q < pixels)
-                for (uint32_t s = 0; s < spp; s++) sum += tile[threadIdx.x * spp + s];
-            __syncthreads();
-        } else if (q < pixels) {
-            for (uint32_t s = 0; s < spp; s++) sum += L[a * P + uint64_t(q) * spp + s];
-        }
-        if (q < pixels) image[uint64_t(q) * 3 + a] = sum / float(spp);
+    const uint32_t npix = pixels - q0 < 256 ? pixels - q0 : 256;
+    const float* const src = L + a * P + uint64_t(q0) * spp;
+    float sum = 0.0f;
+    if (staged) {
+#pragma unroll 8
+        for (uint32_t k = threadIdx.x; k < npix * spp; k += 256) tile[k + (k >> 5)] = __builtin_nontemporal_load(src + k);
+        __syncthreads();
+        if (q < pixels)
+            for (uint32_t s = 0, k = threadIdx.x * spp; s < spp; s++, k++) sum += tile[k + (k >> 5)];
+    } else if (q < pixels) {
+        for (uint32_t s = 0; s < spp; s++) sum += src[uint64_t(threadIdx.x) * spp + s];
     }
+    if (q < pixels) d.image[uint64_t(q) * 3 + a] = sum / float(spp);
+}
+
+void launch_resolve(const PtDevParams* dparams, uint32_t pixels, uint32_t spp, uint64_t P, const float* L, hipStream_t s)
+{
+    const bool staged = spp <= 64;
+    hipLaunchKernelGGL(k_pt_resolve, dim3((pixels + 255) / 256, 3), dim3(256),
+                       staged ? resolve_words(256 * spp) * sizeof(float) : 0, s, dparams, P, L, staged ? 1u : 0u);
 }
 
 // ---- megakernel forward ------------------------------------------------------------------------
@@ -809,6 +839,7 @@ struct PtPlan {
     uint32_t groups = 0; // parts of the camera pass's list (packed)
     size_t count_words(uint32_t depth) const { return groups + size_t(depth) * parts * kCountStride; } // counts before depth's
     PtDevParams* dparams = nullptr;
+    bool high = true; // dparams' tables past kArgMaterials are not known to be zero
     cqx_ray* rays[2] = { nullptr, nullptr };
     uint32_t* paths[2] = { nullptr, nullptr };
     float* beta[2] = { nullptr, nullptr };
@@ -957,7 +988,8 @@ cqx_status get_plan(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_params* p
     return CQX_OK;
 }
 
-// The wavefront graph of the render (replay false) or of the adjoint's replay (replay true), captured
+// The wavefront graph of the render (replay false, down to the image) or of the adjoint's replay (replay
+// true), captured
 // once per plan; the buffers they share are allocated with the first. On a packed volume whose launch
 // the caller left open: camera pass, then (walk, shade) per bounce over lists in parts. Otherwise
 // generate, then (intersect, shade) per depth.
@@ -976,8 +1008,6 @@ cqx_status capture(cqx_ctx* ctx, PtPlan* p, hipStream_t s)
         return PathList{ p->rays[k], p->paths[k], p->beta[k], p->counts + p->count_words(depth), p->parts, kCountStride,
                          p->pcap, slots };
     };
-    const uint32_t all = uint32_t(p->count_words(p->bounces + 2));
-    hipLaunchKernelGGL(k_pt_clear, dim3((all + 255) / 256), dim3(256), 0, s, p->counts, all);
     if (!packed) {
         hipLaunchKernelGGL(k_pt_generate, dim3(uint32_t((P + 255) / 256)), dim3(256), 0, s, p->dparams, P, p->rays[0], p->counts);
         cqx_hit* const hits = static_cast<cqx_hit*>(p->hits);
@@ -1066,6 +1096,7 @@ cqx_status ensure_wavefront(cqx_ctx* ctx, PtPlan* p, bool replay)
     hipStream_t s = ctx->capture_stream;
     HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     const cqx_status cst = replay ? capture<false>(ctx, p, s) : capture<true>(ctx, p, s);
+    if (!replay) launch_resolve(p->dparams, p->width * p->height, p->spp, p->P, p->L, s);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(s, &g);
     (replay ? p->graph_replay : p->graph) = g;
@@ -1083,6 +1114,25 @@ cqx_status check(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_params* pp)
     if (P == 0) return fail(CQX_ERR_INVALID_ARG, "empty image");
     if (P >= (uint64_t(1) << 32)) return fail(CQX_ERR_LIMIT, "at most 2^32 - 1 paths per call");
     return CQX_OK;
+}
+
+// Queues the call's parameters and the clearing of the path counts, ahead of its kernels. Material ids
+// past the caller's are black; the upper half of the tables is written where it holds more than that.
+void begin(PtPlan* p, const PtDevParams& host, uint32_t n_materials, hipStream_t s)
+{
+    const uint32_t words = p->counts ? uint32_t(p->count_words(p->bounces + 2)) : 0u;
+    const uint32_t blocks = std::max(2u, std::min(64u, words / 256)); // 2: the material table's 384 words
+    PtArgs args;
+    std::memcpy(args.head, &host, sizeof(args.head));
+    const bool high = n_materials >= kArgMaterials;
+    const uint32_t halves = high || p->high ? 2 : 1;
+    p->high = high;
+    for (uint32_t half = 0; half < halves; half++) {
+        args.first = half * kArgMaterials;
+        std::memcpy(args.albedo, host.albedo + args.first * 3, sizeof(args.albedo));
+        std::memcpy(args.emission, host.emission + args.first * 3, sizeof(args.emission));
+        hipLaunchKernelGGL(k_pt_begin, dim3(blocks), dim3(256), 0, s, args, p->dparams, p->counts, words);
+    }
 }
 
 TraceParams trace_params(const cqx_dvolume* vol, const cqx_pt_params* pp, const cqx_launch_cfg* cfg)
@@ -1121,7 +1171,8 @@ cqx_status cqx_pathtrace(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_para
         if (st != CQX_OK) return st;
     }
     hipStream_t s = hipStream_t(stream_ptr);
-    HIP_TRY(hipMemcpyAsync(p->dparams, &host, sizeof(host), hipMemcpyHostToDevice, s));
+    host.image = image;
+    begin(p, host, pp->n_materials, s);
     if (mode == 0) {
         const cqx::TraceRange bounces("wavefront graph: camera rays, then per bounce traversal and shading");
         HIP_TRY(hipGraphLaunch(p->exec, s));
@@ -1135,14 +1186,9 @@ cqx_status cqx_pathtrace(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_pt_para
         const uint32_t blocks = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, (p->P + block - 1) / block)));
         hipLaunchKernelGGL(k_pt_megakernel, dim3(blocks), dim3(block), lds, s, p->dparams, trace_params(vol, pp, cfg),
                            p->P, p->L);
+        launch_resolve(p->dparams, pp->width * pp->height, pp->spp, p->P, p->L, s);
     }
-    const uint32_t pixels = pp->width * pp->height;
-    const size_t tile = size_t(256) * pp->spp * sizeof(float);
-    const bool staged = tile <= 65536;
-    hipLaunchKernelGGL(k_pt_resolve, dim3((pixels + 255) / 256), dim3(256), staged ? tile : 0, s, p->dparams, p->P,
-                       p->L, image, staged ? 1u : 0u);
     HIP_TRY(hipGetLastError());
-    // the plan's parameter block is read by the kernels just queued; keep `host` alive until then
     HIP_TRY(hipStreamSynchronize(s));
     return CQX_OK;
 }
@@ -1180,7 +1226,7 @@ cqx_status cqx_pathtrace_adjoint(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx
         p->partial_floats = need;
     }
     hipStream_t s = hipStream_t(stream_ptr);
-    HIP_TRY(hipMemcpyAsync(p->dparams, &host, sizeof(host), hipMemcpyHostToDevice, s));
+    begin(p, host, pp->n_materials, s);
     // replay the paths (the replay graph records each path's vertices), then sweep them backwards
     {
         const cqx::TraceRange replay("adjoint: path replay (wavefront graph)");
