@@ -82,7 +82,10 @@ struct EditPlan {
 
 // Smallest region height for these edits (>= 5), or -1 when they must be applied in order.
 int region_height(const cqx_sphere_edit* edits, uint64_t n);
-// The regions each edit touches and the levels above them (hs >= 0).
+// The regions each edit touches and the levels above them (hs >= 0): plan_regions, which makes keys, first
+// and edit_ids, then plan_levels, which makes the rest.
+void plan_regions(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan);
+void plan_levels(EditPlan& plan);
 void plan_edits(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan);
 
 } // namespace cqx

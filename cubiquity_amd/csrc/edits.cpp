@@ -388,10 +388,17 @@ bool morton_less(const RegionKey& a, const RegionKey& b)
 
 void plan_edits(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan)
 {
+    plan_regions(edits, n, hs, plan);
+    plan_levels(plan);
+}
+
+void plan_regions(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan)
+{
     plan = EditPlan{};
     plan.hs = hs;
     // Regions each edit's bounds touch (one voxel of margin), edits kept in order per region.
     std::vector<std::pair<RegionKey, uint32_t>> touch;
+    touch.reserve(size_t(n) * 6);
     for (uint64_t i = 0; i < n; i++) {
         uint32_t lo[3], hi[3];
         for (int a = 0; a < 3; a++) {
@@ -448,13 +455,27 @@ void plan_edits(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan
         }
     }
     plan.first.push_back(touch.size());
+}
+
+void plan_levels(EditPlan& plan)
+{
     const size_t nr = plan.keys.size();
     plan.morton_regions.resize(nr);
-    for (size_t r = 0; r < nr; r++) plan.morton_regions[r] = uint32_t(r);
-    // Morton order: the interleaved code of the keys' 32 bits per axis, z above y above x at each
-    // bit (morton_less's rule: the axis of the most significant differing bit decides), sorted as
-    // 96-bit integers.
-    {
+    // Morton order: the interleaved code of the keys (morton_less's rule: z above y above x at each bit,
+    // the axis of the most significant differing bit decides). Keys lie around that of the origin, c,
+    // which differs from c - 1 in every bit: with every key in [c - 2^m, c + 2^m), k - (c - 2^m) keeps
+    // the order (above bit m a key's bits are the opposite of bit m) and has m + 1 bits. Edits within 2^23
+    // voxels of the origin and regions of at least 2^5 make m <= 18.
+    const uint32_t c = 1u << (31 - plan.hs);
+    uint32_t m = 0;
+    for (const RegionKey& k : plan.keys)
+        for (uint32_t v : { k.x, k.y, k.z })
+            while (v < c - (1u << m) || v - c + (1u << m) >= 2u << m) m++;
+    std::vector<uint32_t>& order = plan.morton_regions;
+    for (size_t r = 0; r < nr; r++) order[r] = uint32_t(r);
+    if (m > 20) {
+        std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return morton_less(plan.keys[a], plan.keys[b]); });
+    } else {
         const auto spread = [](uint32_t v) { // bits 0..20 of v to bits 0, 3, ..., 60
             uint64_t x = v & 0x1fffffu;
             x = (x | (x << 32)) & 0x1f00000000ffffull;
@@ -464,23 +485,25 @@ void plan_edits(const cqx_sphere_edit* edits, uint64_t n, int hs, EditPlan& plan
             x = (x | (x << 2)) & 0x1249249249249249ull;
             return x;
         };
-        struct Coded {
-            uint64_t hi, lo; // bits 21..31 and bits 0..20 of each axis, interleaved
-            uint32_t region;
-            bool operator<(const Coded& o) const { return hi != o.hi ? hi < o.hi : lo < o.lo; }
-        };
-        std::vector<Coded> code(nr);
+        const uint32_t low = c - (1u << m);
+        std::vector<uint64_t> code(nr);
+        std::vector<uint32_t> tmp(nr);
         for (size_t r = 0; r < nr; r++) {
             const RegionKey& k = plan.keys[r];
-            code[r] = { spread(k.x >> 21) | (spread(k.y >> 21) << 1) | (spread(k.z >> 21) << 2),
-                        spread(k.x) | (spread(k.y) << 1) | (spread(k.z) << 2), uint32_t(r) };
+            code[r] = spread(k.x - low) | (spread(k.y - low) << 1) | (spread(k.z - low) << 2);
         }
-        std::sort(code.begin(), code.end());
-        for (size_t r = 0; r < nr; r++) plan.morton_regions[r] = code[r].region;
+        for (uint32_t shift = 0; shift < 3 * (m + 1); shift += 11) { // LSD radix sort
+            uint32_t count[2049] = {};
+            for (uint32_t r : order) count[((code[r] >> shift) & 2047u) + 1]++;
+            for (int d = 0; d < 2048; d++) count[d + 1] += count[d];
+            for (uint32_t r : order) tmp[count[(code[r] >> shift) & 2047u]++] = r;
+            order.swap(tmp);
+        }
     }
-    const int levels = kRootHeight - hs;
+    const int levels = kRootHeight - plan.hs;
     plan.level_keys.assign(size_t(levels) + 1, {});
     plan.level_children.assign(size_t(levels) + 1, {});
+    plan.level_keys[0].reserve(nr);
     for (size_t r = 0; r < nr; r++) plan.level_keys[0].push_back(plan.keys[plan.morton_regions[r]]);
     for (int l = 1; l <= levels; l++) {
         const std::vector<RegionKey>& below = plan.level_keys[size_t(l) - 1];

@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
 #include <new>
@@ -121,6 +122,19 @@ __global__ void __launch_bounds__(256) k_index_insert(const uint32_t* __restrict
 
 struct DRegionKey {
     uint32_t x, y, z;
+};
+
+// What a call's kernels leave for the host, read in one copy where the host needs it.
+struct EditReport {
+    uint64_t listed;    // nodes the regions listed
+    uint64_t kept;      // of them, the distinct ones
+    uint32_t outgrown;  // a region outgrew its slice
+    uint32_t next_run;  // the region walk's work counter
+    uint32_t count;     // store size after the levels above the regions
+    uint32_t root;
+    uint32_t deep;      // k_find_subdags: a single-child chain deeper than the tree
+    uint32_t pad;
+    cqx_subdag sub[8];
 };
 
 // SphereBrush (voxelization.h:91-126) in FP32, as SphereBrushF in edits.cpp.
@@ -563,14 +577,12 @@ struct MergeArgs {
     uint32_t* rep;      // position -> kept position of its node
     uint32_t* table;    // merge table
     uint64_t table_mask;
-    uint32_t* max_level;
 };
 
 __global__ void __launch_bounds__(256) k_merge_flatten(MergeArgs M)
 {
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < M.nr; r += gridDim.x * blockDim.x) {
         const uint64_t o = M.off[r], poff = M.pool_off[r];
-        uint32_t top = 0;
         for (uint32_t l = 0; l < M.counts[r]; l++) { // children before parents
             const DNode n = load_node(M.pool, poff + l);
             uint32_t lv = 0;
@@ -582,9 +594,7 @@ __global__ void __launch_bounds__(256) k_merge_flatten(MergeArgs M)
             M.src[o + l] = uint32_t(poff + l);
             M.region[o + l] = r;
             M.level[o + l] = uint8_t(lv);
-            top = lv > top ? lv : top;
         }
-        if (M.counts[r]) atomicMax(M.max_level, top);
     }
 }
 
@@ -713,9 +723,23 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_tiles(uint64_t* __restrict_
         }
 }
 
-__global__ void __launch_bounds__(256) k_counts_to_u64(const uint32_t* __restrict__ c, uint64_t* __restrict__ o, uint32_t n)
+__global__ void __launch_bounds__(256) k_region_counts(const uint32_t* __restrict__ c, const uint32_t* __restrict__ overflow,
+                                                       uint64_t* __restrict__ o, uint32_t n, EditReport* __restrict__ rep)
 {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) o[i] = c[i];
+    bool over = false;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        o[i] = c[i];
+        over = over || overflow[i];
+    }
+    if (over) rep->outgrown = 1u;
+}
+
+__global__ void __launch_bounds__(64) k_edit_begin(EditReport* __restrict__ rep)
+{
+    if (threadIdx.x == 0) {
+        rep->outgrown = 0u;
+        rep->next_run = 0u;
+    }
 }
 
 __global__ void __launch_bounds__(256) k_merge_kept(MergeArgs M, uint64_t* kept)
@@ -765,8 +789,8 @@ struct TopArgs {
     uint64_t* cslot;
     uint32_t* table;      // per level: 2 x pow2 slots from tab_off[l]
     const uint64_t* tab_off;
-    uint32_t* out_count;  // in: store size after the merge; out: after the top levels
-    uint32_t* out_root;
+    uint32_t count;       // store size after the merge
+    EditReport* rep;
     uint32_t* old;        // per entry of level >= 1: the node it held before the edits
 };
 
@@ -919,8 +943,8 @@ __device__ void top_small_up(const TopArgs& A, SmallTop& S, uint32_t base, uint3
         out = next;
     }
     if (lane == 0) {
-        *A.out_count = base;
-        *A.out_root = top; // the top level has one entry
+        A.rep->count = base;
+        A.rep->root = top; // the top level has one entry
     }
 }
 
@@ -931,7 +955,7 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
     __shared__ SmallTop small;
     __shared__ uint32_t count_s;
     const uint32_t t = threadIdx.x, T = blockDim.x;
-    if (t == 0) count_s = *A.out_count;
+    if (t == 0) count_s = A.count;
     for (uint32_t i = A.lvl_off[0] + t; i < A.lvl_off[1]; i += T) A.res[i] = A.results[A.morton_regions[i]];
     top_stage(A, small, t, T);
     // The nodes the entries held before the edits, top down: the top entry (height 32, one key)
@@ -1040,10 +1064,10 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
 // findSubDAG (raytracing.cpp:43-87) of every root child, as cqx::find_subdags, one thread each, with
 // the packed walk's pads (pad0 the node's packed word, pad1 the mask of the occupied SubDAGs). Each
 // level is one 32-byte read of the node: 27 us on one thread with a read per child.
-__global__ void __launch_bounds__(64) k_find_subdags(const uint32_t* __restrict__ nodes, const uint32_t* __restrict__ root_p,
-                                                     cqx_subdag* __restrict__ out, uint32_t* __restrict__ err)
+__global__ void __launch_bounds__(64) k_find_subdags(const uint32_t* __restrict__ nodes, uint32_t root,
+                                                     cqx_subdag* __restrict__ out, EditReport* __restrict__ rep)
 {
-    const uint32_t root = *root_p;
+    if (root == kEmptySlot) root = rep->root; // the one k_edit_top left there
     const uint32_t c = threadIdx.x;
     bool deep = false;
     cqx_subdag s{};
@@ -1080,8 +1104,8 @@ __global__ void __launch_bounds__(64) k_find_subdags(const uint32_t* __restrict_
     }
     const uint64_t occupied = __ballot(c < 8 && s.node > 0), failed = __ballot(deep);
     s.pad1 = uint32_t(occupied);
-    if (c == 0) *err = failed ? 1u : 0u;
-    if (c < 8 && !failed) out[c] = s;
+    if (c == 0) rep->deep = failed ? 1u : 0u;
+    if (c < 8 && !failed) out[c] = rep->sub[c] = s;
 }
 
 uint32_t grid_for(uint64_t n, const cqx_ctx* ctx, uint32_t block)
@@ -1111,6 +1135,11 @@ struct DeviceEdits {
         size_t bytes = 0;
     };
     Buf bufs[40];
+    struct Staged {
+        Buf dev, host; // host: pinned memory
+    };
+    Staged staged[2]; // the plans of the regions and of the levels above them (Stage)
+    Buf report;       // device: EditReport
     std::vector<uint32_t> roots{ 0 }; // history (checkpoint / undo / redo), as the host volume's
     size_t current = 0;
 };
@@ -1120,6 +1149,11 @@ void destroy_device_edits(DeviceEdits* e)
     if (!e) return;
     release(e->index);
     for (auto& b : e->bufs) release(b.p);
+    for (auto& st : e->staged) {
+        release(st.dev.p);
+        if (st.host.p) (void)hipHostFree(st.host.p);
+    }
+    release(e->report.p);
     delete e;
 }
 
@@ -1129,10 +1163,9 @@ namespace {
 
 // Buffer slots of DeviceEdits::bufs.
 enum : int {
-    kBufEdits, kBufKeys, kBufFirst, kBufEditIds, kBufRun, kBufPoolOff, kBufCap, kBufCounts, kBufResults,
-    kBufOverflow, kBufPool, kBufTable, kBufOff, kBufSrc, kBufRegion, kBufLevel, kBufKey, kBufSlotOf, kBufRep,
-    kBufMergeTable, kBufFin, kBufScalars, kBufLvlOff, kBufTopKeys, kBufCbeg, kBufCend, kBufMorton, kBufRes,
-    kBufCand, kBufCkey, kBufTopTable, kBufRoot, kBufCslot, kBufTabOff, kBufSubRoot, kBufNext, kBufScanSums, kBufOld
+    kBufRun, kBufPoolOff, kBufCap, kBufCounts, kBufResults, kBufOverflow, kBufPool, kBufTable, kBufOff, kBufSrc, kBufRegion,
+    kBufLevel, kBufKey, kBufSlotOf, kBufRep, kBufMergeTable, kBufFin, kBufRes, kBufCand, kBufCkey, kBufTopTable,
+    kBufCslot, kBufScanSums, kBufOld
 };
 
 // Buffer `slot` of the volume's edit state with at least `bytes` (contents not kept when grown).
@@ -1164,10 +1197,81 @@ cqx_status upload(cqx::DeviceEdits* E, int slot, const std::vector<T>& v, T** ou
     return CQX_OK;
 }
 
+// A plan on its way to the device: its arrays put next to each other in pinned memory, and copied in
+// one piece (a copy each was 12 us of the host's time, 16 of them a call).
+struct Stage {
+    size_t used = 0;
+    char* host = nullptr;
+    char* dev = nullptr;
+    std::vector<char> plain; // where pinned memory cannot be had
+
+    cqx_status reserve(cqx::DeviceEdits::Staged& s, size_t bytes)
+    {
+        if (s.dev.bytes < bytes) {
+            const size_t want = std::max(bytes, s.dev.bytes + s.dev.bytes / 2);
+            release(s.dev.p);
+            if (s.host.p) (void)hipHostFree(s.host.p);
+            s = {};
+            if (hipMalloc(&s.dev.p, want) != hipSuccess) {
+                s.dev.p = nullptr;
+                return fail(CQX_ERR_OOM, "edit buffer of %zu bytes failed", want);
+            }
+            s.dev.bytes = want;
+            if (hipHostMalloc(&s.host.p, want, hipHostMallocDefault) != hipSuccess) {
+                s.host.p = nullptr;
+                (void)hipGetLastError();
+            }
+        }
+        if (!s.host.p) plain.resize(bytes);
+        host = s.host.p ? static_cast<char*>(s.host.p) : plain.data();
+        dev = static_cast<char*>(s.dev.p);
+        return CQX_OK;
+    }
+    static size_t room(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    // Space for `count` values: the host's in *h, the device address they will have returned.
+    template <typename T>
+    T* put(size_t count, T** h)
+    {
+        *h = reinterpret_cast<T*>(host + used);
+        T* const d = reinterpret_cast<T*>(dev + used);
+        used += room(count * sizeof(T));
+        return d;
+    }
+    template <typename T>
+    T* put(const std::vector<T>& v)
+    {
+        T* h = nullptr;
+        T* const d = put(v.size(), &h);
+        if (!v.empty()) std::memcpy(h, v.data(), v.size() * sizeof(T));
+        return d;
+    }
+    // Queues the copy of what was put.
+    cqx_status send() const
+    {
+        if (plain.empty()) HIP_TRY(hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, nullptr));
+        else HIP_TRY(hipMemcpy(dev, host, used, hipMemcpyHostToDevice));
+        return CQX_OK;
+    }
+};
+
+cqx_status report_buffer(cqx::DeviceEdits* E, EditReport** out)
+{
+    auto& b = E->report;
+    if (!b.p) {
+        if (hipMalloc(&b.p, sizeof(EditReport)) != hipSuccess) {
+            b.p = nullptr;
+            return fail(CQX_ERR_OOM, "edit buffer of %zu bytes failed", sizeof(EditReport));
+        }
+        b.bytes = sizeof(EditReport);
+    }
+    *out = static_cast<EditReport*>(b.p);
+    return CQX_OK;
+}
+
 cqx_status scan_u64(cqx_ctx*, cqx::DeviceEdits* E, uint64_t* v, uint64_t n, uint64_t* total)
 {
     const uint64_t tiles = (n + kScanTile - 1) / kScanTile;
-    if (tiles <= 1) {
+    if (tiles <= 4) { // a few values per thread: one launch instead of three
         hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(1024), 0, 0, v, n, total);
     } else {
         if (tiles > 0x7fffffffull) return fail(CQX_ERR_LIMIT, "scan of %llu values", (unsigned long long)n);
@@ -1229,36 +1333,40 @@ cqx_status ensure_store(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t count)
     return CQX_OK;
 }
 
-// Sets the volume's root and recomputes its SubDAGs on the device; nodes from first_new on are new.
-cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root, uint64_t first_new)
+// The volume's root and SubDAGs from the report that k_find_subdags left; nodes from first_new on are new.
+cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root, uint64_t first_new, EditReport& rep)
 {
-    uint32_t* d = nullptr;
-    cqx_status st = buf(vol->edits, kBufSubRoot, 2, &d);
-    if (st != CQX_OK) return st;
-    HIP_TRY(hipMemcpy(d, &root, 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_find_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, d, vol->sub, d + 1);
-    HIP_TRY(hipGetLastError());
-    uint32_t err = 0;
-    HIP_TRY(hipMemcpy(&err, d + 1, 4, hipMemcpyDeviceToHost));
-    if (err) return fail(CQX_ERR_INVALID_DAG, "single-child chain deeper than the tree");
-    cqx_subdag s[8];
-    HIP_TRY(hipMemcpy(s, vol->sub, sizeof(s), hipMemcpyDeviceToHost));
+    if (rep.deep) return fail(CQX_ERR_INVALID_DAG, "single-child chain deeper than the tree");
     int max_height = 0;
-    for (int c = 0; c < 8; c++) {
-        if (s[c].node > 0) max_height = std::max(max_height, int(s[c].height));
-        s[c].pad0 = s[c].pad1 = 0; // the packed walk's, on the device copy only
+    for (cqx_subdag& s : rep.sub) {
+        if (s.node > 0) max_height = std::max(max_height, int(s.height));
+        s.pad0 = s.pad1 = 0; // the packed walk's, on the device copy only
     }
     if (ctx->pt_plan && max_height != vol->max_height) { // its graph holds the stack size
         cqx::destroy_pt_plan(ctx->pt_plan);
         ctx->pt_plan = nullptr;
     }
     vol->root = root;
-    std::memcpy(vol->hsub, s, sizeof(s));
+    std::memcpy(vol->hsub, rep.sub, sizeof(rep.sub));
     vol->max_height = max_height;
-    st = cqx::refresh_packed(ctx, vol, first_new);
+    const cqx_status st = cqx::refresh_packed(ctx, vol, first_new);
     if (st != CQX_OK) return st;
-    HIP_TRY(hipStreamSynchronize(nullptr));
+    if (first_new < vol->node_count) HIP_TRY(hipStreamSynchronize(nullptr));
     return CQX_OK;
+}
+
+// Makes `root`, a node of the store, the volume's root.
+cqx_status switch_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root)
+{
+    EditReport* d_rep = nullptr;
+    const cqx_status st = report_buffer(vol->edits, &d_rep);
+    if (st != CQX_OK) return st;
+    HIP_TRY(hipDeviceSynchronize()); // launches in flight may read the SubDAGs
+    hipLaunchKernelGGL(k_find_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, root, vol->sub, d_rep);
+    HIP_TRY(hipGetLastError());
+    EditReport rep;
+    HIP_TRY(hipMemcpy(&rep, d_rep, sizeof(rep), hipMemcpyDeviceToHost));
+    return set_root(ctx, vol, root, vol->node_count, rep);
 }
 
 cqx_status check_args(cqx_ctx* ctx, cqx_dvolume* vol)
@@ -1299,11 +1407,11 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
         return std::chrono::duration<double, std::milli>(clock::now() - t).count();
     };
     clock::time_point t_phase = clock::now();
-    double ms[6] = { 0, 0, 0, 0, 0, 0 }; // plan, index, regions, merge, levels above, SubDAGs
+    double ms[4] = { 0, 0, 0, 0 }; // plan, regions, merge, levels above
     int attempts = 0;
     cqx::EditPlan plan;
     try {
-        cqx::plan_edits(edits, n, hs, plan);
+        cqx::plan_regions(edits, n, hs, plan);
     } catch (const std::bad_alloc&) {
         return fail(CQX_ERR_OOM, "out of host memory while planning edits");
     }
@@ -1311,20 +1419,33 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
     HIP_TRY(hipDeviceSynchronize()); // launches in flight may read the store or the index
     const uint64_t base = vol->node_count;
     const uint32_t nr = uint32_t(plan.keys.size());
-    ms[0] = ms_since(t_phase);
-    t_phase = clock::now();
     st = ensure_index(ctx, vol, base);
     if (st != CQX_OK) return st;
-    HIP_TRY(hipDeviceSynchronize());
-    ms[1] = ms_since(t_phase);
-    t_phase = clock::now();
+    EditReport* d_rep = nullptr;
+    if ((st = report_buffer(E, &d_rep)) != CQX_OK) return st;
 
     // ---- regions ----
-    std::vector<DRegionKey> keys(nr);
-    for (uint32_t r = 0; r < nr; r++) keys[r] = { plan.keys[r].x, plan.keys[r].y, plan.keys[r].z };
+    Stage stage;
+    if ((st = stage.reserve(E->staged[0], Stage::room(n * sizeof(cqx_sphere_edit)) + Stage::room(nr * sizeof(DRegionKey)) +
+                                              Stage::room((size_t(nr) + 1) * 8) + Stage::room(plan.edit_ids.size() * 4) +
+                                              2 * Stage::room(size_t(nr) * 4) + Stage::room(size_t(nr) * 8))) != CQX_OK)
+        return st;
+    cqx_sphere_edit* h_edits;
+    DRegionKey* h_keys;
+    uint32_t *h_run, *h_cap;
+    uint64_t* h_pool_off;
+    const cqx_sphere_edit* const d_edits = stage.put(n, &h_edits);
+    const DRegionKey* const d_keys = stage.put(nr, &h_keys);
+    const uint64_t* const d_first = stage.put(plan.first);
+    const uint32_t* const d_edit_ids = stage.put(plan.edit_ids);
+    uint32_t* d_run = stage.put(nr, &h_run);
+    uint32_t* d_cap = stage.put(nr, &h_cap);
+    uint64_t* d_pool_off = stage.put(nr, &h_pool_off);
+    std::memcpy(h_edits, edits, n * sizeof(cqx_sphere_edit));
+    for (uint32_t r = 0; r < nr; r++) h_keys[r] = { plan.keys[r].x, plan.keys[r].y, plan.keys[r].z };
     std::vector<uint32_t> cap(nr), run(nr);
     std::vector<uint64_t> pool_off(nr);
-    std::vector<double> work(nr);
+    std::vector<float> work(nr);
     uint64_t pool_total = 0;
     // First slice of each region's list: per sphere about twice the voxels of its largest cross
     // section the region can hold (a sphere changes nodes along its surface, a few per voxel
@@ -1334,35 +1455,44 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
     const char* fixed_slice = std::getenv("CQX_EDIT_FIRST_SLICE");
     const double fixed = fixed_slice ? std::atof(fixed_slice) : 0.0;
     const double side = std::ldexp(1.0, hs);
+    float most = 0.0f;
     for (uint32_t r = 0; r < nr; r++) {
         double est = 64.0;
         for (uint64_t j = plan.first[r]; j < plan.first[r + 1]; j++) {
             const double rad = edits[plan.edit_ids[j]].radius;
             est += 2.0 * std::min(3.14159265 * rad * rad, side * side) + 16.0;
         }
-        work[r] = est;
+        work[r] = float(est);
+        most = std::max(most, work[r]);
         if (fixed >= 1.0) est = fixed;
         cap[r] = uint32_t(pow2_at_least(uint64_t(std::min(est, 1048576.0))));
         pool_off[r] = pool_total;
         pool_total += cap[r];
-        run[r] = r;
     }
     // the wave that takes the heaviest region (most sphere surface) early finishes early: the
-    // phase then lasts about as long as its heaviest region or its average load per wave
-    std::stable_sort(run.begin(), run.end(), [&](uint32_t a, uint32_t b) { return work[a] > work[b]; });
-    cqx_sphere_edit* d_edits;
-    DRegionKey* d_keys;
-    uint64_t *d_first, *d_pool_off;
-    uint32_t *d_edit_ids, *d_run, *d_cap, *d_counts, *d_results, *d_overflow, *d_pool, *d_table;
-    std::vector<cqx_sphere_edit> ev(edits, edits + n);
-    if ((st = upload(E, kBufEdits, ev, &d_edits)) != CQX_OK || (st = upload(E, kBufKeys, keys, &d_keys)) != CQX_OK ||
-        (st = upload(E, kBufFirst, plan.first, &d_first)) != CQX_OK ||
-        (st = upload(E, kBufEditIds, plan.edit_ids, &d_edit_ids)) != CQX_OK ||
-        (st = buf(E, kBufCounts, nr, &d_counts)) != CQX_OK || (st = buf(E, kBufResults, nr, &d_results)) != CQX_OK ||
-        (st = buf(E, kBufOverflow, nr, &d_overflow)) != CQX_OK)
+    // phase then lasts about as long as its heaviest region or its average load per wave. Sorted
+    // into 1024 classes of work: the order within one does not matter.
+    {
+        uint32_t at[1025] = {};
+        const auto cls = [&](uint32_t r) { return 1023u - uint32_t(std::min(1023.0f, work[r] * (1023.0f / most))); };
+        for (uint32_t r = 0; r < nr; r++) at[cls(r) + 1]++;
+        for (int k = 0; k < 1024; k++) at[k + 1] += at[k];
+        for (uint32_t r = 0; r < nr; r++) run[at[cls(r)]++] = r;
+    }
+    std::memcpy(h_run, run.data(), nr * 4);
+    std::memcpy(h_cap, cap.data(), nr * 4);
+    std::memcpy(h_pool_off, pool_off.data(), nr * 8);
+    uint32_t *d_counts, *d_results, *d_overflow, *d_pool, *d_table;
+    uint64_t* d_off;
+    if ((st = stage.send()) != CQX_OK || (st = buf(E, kBufCounts, nr, &d_counts)) != CQX_OK ||
+        (st = buf(E, kBufResults, nr, &d_results)) != CQX_OK || (st = buf(E, kBufOverflow, nr, &d_overflow)) != CQX_OK ||
+        (st = buf(E, kBufOff, nr + 1, &d_off)) != CQX_OK)
         return st;
+    ms[0] = ms_since(t_phase);
+    t_phase = clock::now();
     // A region whose list outgrows its slice runs again with a slice 8 times larger, placed after
     // the others; the pool keeps what the finished regions listed.
+    EditReport rep{};
     for (int attempt = 0; !run.empty(); attempt++) {
         if (attempt > 6) return fail(CQX_ERR_LIMIT, "an edit region listed more nodes than the retries allow");
         if (base + uint64_t(*std::max_element(cap.begin(), cap.end())) >= 0xfffffffeull)
@@ -1385,96 +1515,111 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
         }
         d_pool = static_cast<uint32_t*>(pb.p);
         d_table = static_cast<uint32_t*>(tb.p);
-        if ((st = upload(E, kBufRun, run, &d_run)) != CQX_OK || (st = upload(E, kBufPoolOff, pool_off, &d_pool_off)) != CQX_OK ||
-            (st = upload(E, kBufCap, cap, &d_cap)) != CQX_OK)
+        if (attempt > 0 && ((st = upload(E, kBufRun, run, &d_run)) != CQX_OK ||
+                            (st = upload(E, kBufPoolOff, pool_off, &d_pool_off)) != CQX_OK ||
+                            (st = upload(E, kBufCap, cap, &d_cap)) != CQX_OK))
             return st;
-        uint32_t* d_next = nullptr;
-        if ((st = buf(E, kBufNext, 1, &d_next)) != CQX_OK) return st;
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, 0, d_next, uint64_t(1), 0u);
+        hipLaunchKernelGGL(k_edit_begin, dim3(1), dim3(64), 0, 0, d_rep);
         RegionArgs A{ vol->nodes, E->index, E->index_cap - 1, vol->root, hs, uint32_t(base), d_edits, d_keys, d_first,
-                      d_edit_ids, d_run, uint32_t(run.size()), d_next, d_pool_off, d_cap, d_pool, d_table, d_counts,
+                      d_edit_ids, d_run, uint32_t(run.size()), &d_rep->next_run, d_pool_off, d_cap, d_pool, d_table, d_counts,
                       d_results, d_overflow };
         const uint32_t waves = uint32_t(std::min<uint64_t>(run.size(), uint64_t(ctx->cu_count) * 32));
         hipLaunchKernelGGL(k_edit_regions, dim3(waves), dim3(64), sizeof(Frame) * size_t(std::max(hs - 3, 1)), 0, A);
+        hipLaunchKernelGGL(k_region_counts, dim3(grid_for(nr, ctx, 256)), dim3(256), 0, 0, d_counts, d_overflow, d_off, nr,
+                           d_rep);
         HIP_TRY(hipGetLastError());
-        std::vector<uint32_t> over(nr);
-        HIP_TRY(hipMemcpy(over.data(), d_overflow, nr * 4, hipMemcpyDeviceToHost));
-        std::vector<uint32_t> again;
-        for (uint32_t r : run)
-            if (over[r]) {
-                again.push_back(r);
-                cap[r] *= 8;
-                pool_off[r] = pool_total;
-                pool_total += cap[r];
+        if ((st = scan_u64(ctx, E, d_off, uint64_t(nr), &d_rep->listed)) != CQX_OK) return st;
+        if (attempt == 0) { // the levels above are planned while the regions run
+            try {
+                cqx::plan_levels(plan);
+            } catch (const std::bad_alloc&) {
+                return fail(CQX_ERR_OOM, "out of host memory while planning edits");
             }
-        if (!again.empty())
+        }
+        HIP_TRY(hipMemcpy(&rep, d_rep, offsetof(EditReport, next_run), hipMemcpyDeviceToHost));
+        std::vector<uint32_t> again;
+        if (rep.outgrown) {
+            std::vector<uint32_t> over(nr);
+            HIP_TRY(hipMemcpy(over.data(), d_overflow, nr * 4, hipMemcpyDeviceToHost));
+            for (uint32_t r : run)
+                if (over[r]) {
+                    again.push_back(r);
+                    cap[r] *= 8;
+                    pool_off[r] = pool_total;
+                    pool_total += cap[r];
+                }
             cqx::log_debug("device edits: %zu of %zu regions outgrew their node lists; running them again",
                            again.size(), run.size());
+        }
         run.swap(again);
         attempts = attempt + 1;
     }
-    ms[2] = ms_since(t_phase);
+    const uint64_t total = rep.listed;
+    ms[1] = ms_since(t_phase);
     t_phase = clock::now();
 
     // ---- merge ----
-    uint64_t *d_off, *d_slot_of, *d_fin, *d_scalars;
-    uint32_t *d_src, *d_region, *d_key, *d_rep, *d_mtable;
-    uint8_t* d_level;
-    if ((st = buf(E, kBufOff, nr + 1, &d_off)) != CQX_OK || (st = buf(E, kBufScalars, 8, &d_scalars)) != CQX_OK) return st;
-    hipLaunchKernelGGL(k_counts_to_u64, dim3(grid_for(nr, ctx, 256)), dim3(256), 0, 0, d_counts, d_off, nr);
-    if ((st = scan_u64(ctx, E, d_off, uint64_t(nr), d_scalars)) != CQX_OK) return st;
-    uint64_t total = 0;
-    HIP_TRY(hipMemcpy(&total, d_scalars, 8, hipMemcpyDeviceToHost));
     if (base + total >= 0xfffffffeull) return fail(CQX_ERR_LIMIT, "store too large for on-device edits");
-    const uint64_t mcap = pow2_at_least(std::max<uint64_t>(1024, 2 * total));
-    if ((st = buf(E, kBufSrc, total, &d_src)) != CQX_OK || (st = buf(E, kBufRegion, total, &d_region)) != CQX_OK ||
-        (st = buf(E, kBufLevel, total, &d_level)) != CQX_OK || (st = buf(E, kBufKey, total * 8, &d_key)) != CQX_OK ||
-        (st = buf(E, kBufSlotOf, total, &d_slot_of)) != CQX_OK || (st = buf(E, kBufRep, total, &d_rep)) != CQX_OK ||
-        (st = buf(E, kBufMergeTable, mcap, &d_mtable)) != CQX_OK || (st = buf(E, kBufFin, total + 1, &d_fin)) != CQX_OK)
-        return st;
-    uint32_t* d_max_level = reinterpret_cast<uint32_t*>(d_scalars + 1);
-    HIP_TRY(hipMemset(d_max_level, 0, 4));
-    MergeArgs M{ uint32_t(base), nr, d_pool_off, d_pool, d_counts, d_off, total, d_src, d_region, d_level, d_key,
-                 d_slot_of, d_rep, d_mtable, mcap - 1, d_max_level };
-    uint64_t kept_total = 0;
+    uint64_t kept_total = 0, *d_fin = nullptr;
+    MergeArgs M{};
     if (total) {
+        uint64_t* d_slot_of;
+        uint32_t *d_src, *d_region, *d_key, *d_rep_of, *d_mtable;
+        uint8_t* d_level;
+        const uint64_t mcap = pow2_at_least(std::max<uint64_t>(1024, 2 * total));
+        if ((st = buf(E, kBufSrc, total, &d_src)) != CQX_OK || (st = buf(E, kBufRegion, total, &d_region)) != CQX_OK ||
+            (st = buf(E, kBufLevel, total, &d_level)) != CQX_OK || (st = buf(E, kBufKey, total * 8, &d_key)) != CQX_OK ||
+            (st = buf(E, kBufSlotOf, total, &d_slot_of)) != CQX_OK || (st = buf(E, kBufRep, total, &d_rep_of)) != CQX_OK ||
+            (st = buf(E, kBufMergeTable, mcap, &d_mtable)) != CQX_OK || (st = buf(E, kBufFin, total + 1, &d_fin)) != CQX_OK)
+            return st;
+        M = MergeArgs{ uint32_t(base), nr, d_pool_off, d_pool, d_counts, d_off, total, d_src, d_region, d_level, d_key,
+                       d_slot_of, d_rep_of, d_mtable, mcap - 1 };
         hipLaunchKernelGGL(k_merge_flatten, dim3(grid_for(nr, ctx, 256)), dim3(256), 0, 0, M);
         hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(mcap, ctx, 256)), dim3(256), 0, 0, d_mtable, mcap, kEmptySlot);
-        uint32_t max_level = 0;
-        HIP_TRY(hipMemcpy(&max_level, d_max_level, 4, hipMemcpyDeviceToHost));
         const uint32_t g = grid_for(total, ctx, 256);
-        for (uint32_t lv = 0; lv <= max_level; lv++) {
+        for (uint32_t lv = 0; lv < uint32_t(hs); lv++) { // a node of height h has level h - 1 at most
             hipLaunchKernelGGL(k_merge_keys, dim3(g), dim3(256), 0, 0, M, lv);
             hipLaunchKernelGGL(k_merge_insert, dim3(g), dim3(256), 0, 0, M, lv);
             hipLaunchKernelGGL(k_merge_rep, dim3(g), dim3(256), 0, 0, M, lv);
         }
         hipLaunchKernelGGL(k_merge_kept, dim3(g), dim3(256), 0, 0, M, d_fin);
-        if ((st = scan_u64(ctx, E, d_fin, total, d_scalars + 2)) != CQX_OK) return st;
+        if ((st = scan_u64(ctx, E, d_fin, total, &d_rep->kept)) != CQX_OK) return st;
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpy(&kept_total, d_scalars + 2, 8, hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(&kept_total, &d_rep->kept, 8, hipMemcpyDeviceToHost));
     }
     // ---- the levels above the regions: schedule, capacity ----
+    DRegionKey* h_tkeys;
+    uint32_t *h_lvl_off, *h_cbeg, *h_cend;
+    uint64_t* h_tab_off;
+    uint64_t ntop = 0;
     const uint32_t levels = uint32_t(32 - hs);
-    std::vector<uint32_t> lvl_off(levels + 2, 0), morton(plan.morton_regions), cbeg, cend;
-    std::vector<DRegionKey> tkeys;
-    std::vector<uint64_t> tab_off(levels + 2, 0);
+    for (uint32_t l = 0; l <= levels; l++) ntop += plan.level_keys[l].size();
+    Stage above;
+    if ((st = above.reserve(E->staged[1], Stage::room((levels + 2) * 4) + Stage::room((levels + 2) * 8) +
+                                              Stage::room(ntop * sizeof(DRegionKey)) + 2 * Stage::room(ntop * 4) +
+                                              Stage::room(size_t(nr) * 4))) != CQX_OK)
+        return st;
+    const uint32_t* const d_lvl_off = above.put(levels + 2, &h_lvl_off);
+    const uint64_t* const d_tab_off = above.put(levels + 2, &h_tab_off);
+    const DRegionKey* const d_tkeys = above.put(ntop, &h_tkeys);
+    const uint32_t* const d_cbeg = above.put(ntop, &h_cbeg);
+    const uint32_t* const d_cend = above.put(ntop, &h_cend);
+    const uint32_t* const d_morton = above.put(plan.morton_regions);
+    uint32_t at = 0;
+    h_tab_off[0] = 0;
     for (uint32_t l = 0; l <= levels; l++) {
-        lvl_off[l] = uint32_t(tkeys.size());
+        h_lvl_off[l] = at;
         const auto& lk = plan.level_keys[l];
-        for (size_t i = 0; i < lk.size(); i++) {
-            tkeys.push_back({ lk[i].x, lk[i].y, lk[i].z });
-            if (l == 0) {
-                cbeg.push_back(0);
-                cend.push_back(0);
-            } else {
-                cbeg.push_back(lvl_off[l - 1] + plan.level_children[l][i]);
-                cend.push_back(lvl_off[l - 1] + plan.level_children[l][i + 1]);
-            }
+        for (size_t i = 0; i < lk.size(); i++, at++) {
+            h_tkeys[at] = { lk[i].x, lk[i].y, lk[i].z };
+            h_cbeg[at] = l == 0 ? 0 : h_lvl_off[l - 1] + plan.level_children[l][i];
+            h_cend[at] = l == 0 ? 0 : h_lvl_off[l - 1] + plan.level_children[l][i + 1];
         }
-        tab_off[l + 1] = tab_off[l] + (l == 0 ? 0 : pow2_at_least(std::max<uint64_t>(2, 2 * lk.size())));
+        h_tab_off[l + 1] = h_tab_off[l] + (l == 0 ? 0 : pow2_at_least(std::max<uint64_t>(2, 2 * lk.size())));
     }
-    lvl_off[levels + 1] = uint32_t(tkeys.size());
-    const uint64_t ntop = tkeys.size();
+    h_lvl_off[levels + 1] = at;
+    const uint64_t top_slots = h_tab_off[levels + 1];
+    if ((st = above.send()) != CQX_OK) return st;
     st = ensure_store(ctx, vol, base + kept_total + ntop);
     if (st != CQX_OK) return st;
     st = ensure_index(ctx, vol, base + kept_total + ntop);
@@ -1487,54 +1632,38 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
         HIP_TRY(hipGetLastError());
     }
     E->indexed = base + kept_total;
-
-    HIP_TRY(hipDeviceSynchronize());
-    ms[3] = ms_since(t_phase);
+    ms[2] = ms_since(t_phase);
     t_phase = clock::now();
 
-    // ---- the levels above the regions ----
-    uint32_t *d_lvl_off, *d_cbeg, *d_cend, *d_morton, *d_res, *d_cand, *d_ckey, *d_ttable, *d_root;
-    DRegionKey* d_tkeys;
-    uint64_t *d_tab_off, *d_cslot;
-    if ((st = upload(E, kBufLvlOff, lvl_off, &d_lvl_off)) != CQX_OK || (st = upload(E, kBufTopKeys, tkeys, &d_tkeys)) != CQX_OK ||
-        (st = upload(E, kBufCbeg, cbeg, &d_cbeg)) != CQX_OK || (st = upload(E, kBufCend, cend, &d_cend)) != CQX_OK ||
-        (st = upload(E, kBufMorton, morton, &d_morton)) != CQX_OK || (st = buf(E, kBufRes, ntop, &d_res)) != CQX_OK ||
-        (st = buf(E, kBufCand, 2 * ntop, &d_cand)) != CQX_OK || (st = buf(E, kBufCkey, ntop * 8, &d_ckey)) != CQX_OK ||
-        (st = buf(E, kBufTopTable, tab_off[levels + 1], &d_ttable)) != CQX_OK ||
-        (st = upload(E, kBufTabOff, tab_off, &d_tab_off)) != CQX_OK ||
-        (st = buf(E, kBufRoot, 2, &d_root)) != CQX_OK)
+    // ---- the levels above the regions, and the new root's SubDAGs ----
+    uint32_t *d_res, *d_cand, *d_ckey, *d_ttable, *d_old;
+    uint64_t* d_cslot;
+    if ((st = buf(E, kBufRes, ntop, &d_res)) != CQX_OK || (st = buf(E, kBufCand, 2 * ntop, &d_cand)) != CQX_OK ||
+        (st = buf(E, kBufCkey, ntop * 8, &d_ckey)) != CQX_OK || (st = buf(E, kBufTopTable, top_slots, &d_ttable)) != CQX_OK ||
+        (st = buf(E, kBufCslot, ntop, &d_cslot)) != CQX_OK || (st = buf(E, kBufOld, ntop, &d_old)) != CQX_OK)
         return st;
-    if ((st = buf(E, kBufCslot, ntop, &d_cslot)) != CQX_OK) return st;
-    uint32_t* d_old = nullptr;
-    if ((st = buf(E, kBufOld, ntop, &d_old)) != CQX_OK) return st;
-    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(tab_off[levels + 1], ctx, 256)), dim3(256), 0, 0, d_ttable,
-                       tab_off[levels + 1], kEmptySlot);
-    const uint32_t count_after_merge = uint32_t(base + kept_total);
-    HIP_TRY(hipMemcpy(d_root, &count_after_merge, 4, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(top_slots, ctx, 256)), dim3(256), 0, 0, d_ttable, top_slots, kEmptySlot);
     TopArgs T{ vol->nodes, E->index, E->index_cap - 1, vol->root, hs, levels, d_lvl_off, d_tkeys, d_cbeg, d_cend,
-               d_morton, d_results, d_res, d_cand, d_ckey, d_cand + ntop, d_cslot, d_ttable, d_tab_off, d_root,
-               d_root + 1, d_old };
+               d_morton, d_results, d_res, d_cand, d_ckey, d_cand + ntop, d_cslot, d_ttable, d_tab_off,
+               uint32_t(base + kept_total), d_rep, d_old };
     hipLaunchKernelGGL(k_edit_top, dim3(1), dim3(kTopBlock), 0, 0, T);
+    hipLaunchKernelGGL(k_find_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, kEmptySlot, vol->sub, d_rep);
     HIP_TRY(hipGetLastError());
-    uint32_t out[2] = { 0, 0 };
-    HIP_TRY(hipMemcpy(out, d_root, 8, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(&rep, d_rep, sizeof(rep), hipMemcpyDeviceToHost));
     const uint64_t kOffset32Nodes = uint64_t(1) << 27; // the child-offset width the traversal uses
-    if (ctx->pt_plan && (base <= kOffset32Nodes) != (uint64_t(out[0]) <= kOffset32Nodes)) {
+    if (ctx->pt_plan && (base <= kOffset32Nodes) != (uint64_t(rep.count) <= kOffset32Nodes)) {
         cqx::destroy_pt_plan(ctx->pt_plan); // its captured graph holds the old offset width
         ctx->pt_plan = nullptr;
     }
-    vol->node_count = out[0];
-    E->indexed = out[0];
-    ms[4] = ms_since(t_phase);
-    t_phase = clock::now();
-    st = set_root(ctx, vol, out[1], base);
+    vol->node_count = rep.count;
+    E->indexed = rep.count;
+    st = set_root(ctx, vol, rep.root, base, rep);
     if (st != CQX_OK) return st;
-    ms[5] = ms_since(t_phase);
+    ms[3] = ms_since(t_phase);
     cqx::log_debug("device edits: %llu spheres over %u regions of side 2^%d (%d runs); %llu listed, %llu appended, "
-                   "%llu above; plan %.1f ms, index %.1f ms, regions %.1f ms, merge %.1f ms, levels above %.1f ms, "
-                   "SubDAGs %.1f ms", (unsigned long long)n, nr, hs, attempts, (unsigned long long)total,
-                   (unsigned long long)kept_total, (unsigned long long)(out[0] - base - kept_total), ms[0], ms[1],
-                   ms[2], ms[3], ms[4], ms[5]);
+                   "%llu above; plan %.2f ms, regions %.2f ms, merge %.2f ms, levels above %.2f ms",
+                   (unsigned long long)n, nr, hs, attempts, (unsigned long long)total, (unsigned long long)kept_total,
+                   (unsigned long long)(rep.count - base - kept_total), ms[0], ms[1], ms[2], ms[3]);
     E->roots.resize(E->current + 1);
     E->roots[E->current] = vol->root;
     return CQX_OK;
@@ -1559,8 +1688,7 @@ cqx_status cqx_volume_undo(cqx_ctx* ctx, cqx_dvolume* vol)
     cqx::DeviceEdits* E = vol->edits;
     E->roots[E->current] = vol->root;
     if (E->current > 0) E->current--;
-    HIP_TRY(hipDeviceSynchronize());
-    return set_root(ctx, vol, E->roots[E->current], vol->node_count);
+    return switch_root(ctx, vol, E->roots[E->current]);
 }
 
 cqx_status cqx_volume_redo(cqx_ctx* ctx, cqx_dvolume* vol)
@@ -1570,8 +1698,7 @@ cqx_status cqx_volume_redo(cqx_ctx* ctx, cqx_dvolume* vol)
     cqx::DeviceEdits* E = vol->edits;
     E->roots[E->current] = vol->root;
     if (E->current + 1 < E->roots.size()) E->current++;
-    HIP_TRY(hipDeviceSynchronize());
-    return set_root(ctx, vol, E->roots[E->current], vol->node_count);
+    return switch_root(ctx, vol, E->roots[E->current]);
 }
 
 cqx_status cqx_volume_download(cqx_ctx* ctx, const cqx_dvolume* vol, uint64_t first, uint64_t count, uint32_t* nodes)
