@@ -62,7 +62,9 @@ __device__ __forceinline__ uint32_t lane_stack(char* rows_lds, uint32_t rows, ui
 {
     // the low 32 bits of a generic LDS address are the LDS address
     const uint32_t lds = uint32_t(reinterpret_cast<uintptr_t>(rows_lds));
-    return stack_base(lds + (threadIdx.x >> 6) * rows * kRowBytes + (threadIdx.x & 63u) * 4u, top);
+    uint32_t base = stack_base(lds + (threadIdx.x >> 6) * rows * kRowBytes + (threadIdx.x & 63u) * 4u, top);
+    opaque(base); // one register, not its terms added at each use
+    return base;
 }
 
 // Up to `steps` steps of the wave's walking lanes: the plain rays' step when every walking lane may
