@@ -422,12 +422,12 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
 {
     opaque(S.phase);
     float t1x, t1y, t1z;
-    float tcx = packed_exits(S, t1x, t1y, t1z);
     uint32_t slot = S.cid ^ S.sign_bits;
     uint32_t occupied = (S.node >> slot) & 1u;
     if (!occupied) {
         // Advance to the next sibling, raytracing.cpp:328-332: the axes whose exit is the minimum.
         S.iters++;
+        const float tcx = packed_exits(S, t1x, t1y, t1z);
         const uint32_t fx = uint32_t(int32_t(fbits(t1x - tcx) - 1u) >> 31), fy = uint32_t(int32_t(fbits(t1y - tcx) - 1u) >> 31),
                        fz = uint32_t(int32_t(fbits(t1z - tcx) - 1u) >> 31);
         const float obx = S.bx, oby = S.by, obz = S.bz;
@@ -438,13 +438,13 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
         const uint32_t carry = S.cid & flips;
         S.cid ^= flips;
         if (carry) packed_pop(S, lds, base, obx, oby, obz);
-        tcx = packed_exits(S, t1x, t1y, t1z);
         slot = S.cid ^ S.sign_bits;
         occupied = (S.node >> slot) & 1u;
     }
     if (occupied) {
         S.word = packed_fetch(P, S, slot); // the last one read is the hit's
         S.iters++;
+        const float tcx = packed_exits(S, t1x, t1y, t1z);
         const float half = S.s * 0.5f;
         const float px = S.bx - kBias, py = S.by - kBias, pz = S.bz - kBias;
         // entry time of the child; children behind the origin (entry <= 0) compare their centre
