@@ -80,7 +80,8 @@ __device__ __forceinline__ void walk_burst(const PackedParams& P, PackedRay& S, 
             if (S.phase == kWalk) walk_step_packed_any(P, S, lds, base);
     } else {
         for (uint32_t k = 0; k < steps; k++)
-            if (S.phase == kWalk) walk_step_packed<kLod>(P, S, lds, base);
+            if (__builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_ballot_w64(S.phase == kWalk)))
+                walk_step_packed<kLod>(P, S, lds, base);
     }
 }
 

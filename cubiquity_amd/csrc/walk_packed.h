@@ -27,9 +27,10 @@
 // (small batches, the long rays a launch ends with), as the length of one wave's chain: about 170
 // instructions and a read's latency a step. So the child's entry planes are computed while its word is
 // in flight, a walk that left stands on node 0 instead of taking a branch of its own, and phases and the
-// stack base stay in registers the compiler cannot remake in every branch: 144 -> 126 VALU instructions,
-// 1280x720 camera rays with LOD at 1024^3 99 -> 87 us, 65536 camera rays 37.5 -> 32 us, 1021 incoherent
-// rays 51 -> 44 us, 2^24 2.07 -> 2.00 ms.
+// stack base stay in registers the compiler cannot remake in every branch: 144 -> 113 VALU instructions
+// and 60 -> 37 scalar ones. 1280x720 camera rays with LOD at 1024^3 99 -> 80 us, 65536 camera rays 37.5 ->
+// 30 us, 1021 incoherent rays 51 -> 37 us, 2^24 2.07 -> 1.93 ms. (Reading the next word already at the end
+// of a step, with its waits where they belong, took 12 to 20 more instructions and 4 to 12 % longer.)
 // The sign masks and one-instruction minima need values without NaN, -0 and underflow: ray_plain() is true for rays where
 // none can occur. A wave with another ray among its walking lanes takes walk_step_packed_any, which
 // keeps the compare-selects of the reference.
@@ -399,6 +400,7 @@ __device__ __forceinline__ void packed_pop(PackedRay& S, char* lds, uint32_t bas
     const uint32_t z = uint32_t(__builtin_clz(diff)); // the highest bit is 31 - z; the node's height 32 - z
     const bool left = z < S.zstart;
     S.phase = left ? uint32_t(kLeave) : S.phase;
+    opaque(S.phase); // one select
     S.node = 0u;
     if (left) return;
     S.sp = base + z * kRowBytes;
@@ -414,17 +416,27 @@ __device__ __forceinline__ void packed_pop(PackedRay& S, char* lds, uint32_t bas
     S.entries++;
 }
 
+// Whether the current child is occupied.
+__device__ __forceinline__ bool on_occupied(const PackedRay& S) { return (S.node >> (S.cid ^ S.sign_bits)) & 1u; }
+
+// The footprint test of a child of size s and exit time tcx by its thresholds: large when 0 <= tcx <=
+// lod_hi * s, or tcx <= lod_lo * s (which is negative). Where tcx is not -0, tcx >= 0 or tcx <= -q
+// says that the bits of -tcx, as an integer, are at least those of q >= 0: one compare.
+template <bool kLod>
+__device__ __forceinline__ bool large_at(const PackedParams& P, float tcx, float s)
+{
+    const bool large = (fbits(tcx) ^ 0x80000000u) >= fbits(-P.lod_lo * s);
+    return kLod ? large & (tcx <= P.lod_hi * s) : large;
+}
+
 // One step of a plain ray (ray_plain) whose phase is kWalk: an advance if the current child is empty,
 // then the descent into (or hit of) the current child if it is occupied. Counts up to two
 // iterations; the caller keeps iters + 2 <= max_iters.
 template <bool kLod>
 __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRay& S, char* lds, uint32_t base)
 {
-    opaque(S.phase);
     float t1x, t1y, t1z;
-    uint32_t slot = S.cid ^ S.sign_bits;
-    uint32_t occupied = (S.node >> slot) & 1u;
-    if (!occupied) {
+    if (!on_occupied(S)) {
         // Advance to the next sibling, raytracing.cpp:328-332: the axes whose exit is the minimum.
         S.iters++;
         const float tcx = packed_exits(S, t1x, t1y, t1z);
@@ -438,11 +450,10 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
         const uint32_t carry = S.cid & flips;
         S.cid ^= flips;
         if (carry) packed_pop(S, lds, base, obx, oby, obz);
-        slot = S.cid ^ S.sign_bits;
-        occupied = (S.node >> slot) & 1u;
     }
-    if (occupied) {
-        S.word = packed_fetch(P, S, slot); // the last one read is the hit's
+    opaque(S.cid); // tested anew: carrying the outcome past the branch takes more instructions
+    if (on_occupied(S)) {
+        S.word = packed_fetch(P, S, S.cid ^ S.sign_bits); // the last one read is the hit's
         S.iters++;
         const float tcx = packed_exits(S, t1x, t1y, t1z);
         const float half = S.s * 0.5f;
@@ -454,11 +465,11 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
         uint32_t my = less_mask(((py + half) - S.oy) * S.iy, tce);
         uint32_t mz = less_mask(((pz + half) - S.oz) * S.iz, tce);
         in_flight(mx, my, mz);
-        // large: 0 <= tcx <= lod_hi * s, or tcx <= lod_lo * s (which is negative)
-        bool large = (tcx <= P.lod_lo * S.s) | (tcx >= 0.0f);
-        if (kLod) large = large & (tcx <= P.lod_hi * S.s);
-        const bool down = large & (S.word >= (kMaterialCount << 8));
-        if (down & (S.s >= 1.5f)) {
+        // (s >= 1.5: deeper than a valid DAG otherwise; packed_hit tells these from hits)
+        const bool down = large_at<kLod>(P, tcx, S.s) & (S.word >= (kMaterialCount << 8)) & (S.s >= 1.5f);
+        S.phase = down ? S.phase : uint32_t(kHit);
+        opaque(S.phase);
+        if (down) {
             if (tcx < S.last_exit) stack_store(lds, S.sp, S.node);
             S.last_exit = tcx;
             S.sp += kRowBytes;
@@ -469,8 +480,6 @@ __device__ __forceinline__ void walk_step_packed(const PackedParams& P, PackedRa
             S.by += bitsf(fbits(half) & my);
             S.bz += bitsf(fbits(half) & mz);
             S.cid = (mx & 1u) | (my & 2u) | (mz & 4u);
-        } else {
-            S.phase = down ? kAnomaly : kHit; // (deeper than a valid DAG)
         }
     }
 }
@@ -564,6 +573,14 @@ __device__ __forceinline__ bool packed_hit(const PackedParams& P, const PackedRa
     h.ey = h.t == t0y;
     h.ez = h.t == t0z;
     h.entries = S.entries;
+    if (S.plain && S.word >= (kMaterialCount << 8) && S.s < 1.5f) { // a walk that would go deeper than a valid DAG
+        float t1x, t1y, t1z;
+        const float tcx = packed_exits(S, t1x, t1y, t1z);
+        if (large_at<true>(P, tcx, S.s)) {
+            h.info = CQX_HIT_ANOMALY;
+            return false;
+        }
+    }
     const float bsize = S.s > 0.0f ? S.s : 1.0f; // a SubDAG of height 0: the node itself, of side 1
     h.info = 1u | (slot << 1) | (((fbits(bsize) >> 23) - 127u) << 4);
     if (!P.surf) return true;
