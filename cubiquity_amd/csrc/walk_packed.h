@@ -183,6 +183,15 @@ __device__ __forceinline__ void opaque(uint32_t& v)
     (void)v;
 #endif
 }
+// Keeps what is computed of a, b and c in the branch it stands in.
+__device__ __forceinline__ void stay_here(float& a, float& b, float& c)
+{
+#if defined(__AMDGCN__)
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
+#else
+    (void)a, (void)b, (void)c;
+#endif
+}
 // Has a, b and c computed here, while a read issued before is in flight, rather than after its wait in
 // the branch that uses them (where the compiler moves them).
 __device__ __forceinline__ void in_flight(uint32_t& a, uint32_t& b, uint32_t& c)
@@ -217,9 +226,11 @@ struct OctantChain {
 __device__ __forceinline__ OctantChain octant_chain(const PackedRay& S)
 {
     OctantChain c;
-    c.distx = (-S.ox) / S.dx;
-    c.disty = (-S.oy) / S.dy;
-    c.distz = (-S.oz) / S.dz;
+    float ox = S.ox, oy = S.oy, oz = S.oz;
+    stay_here(ox, oy, oz); // (three divisions that few lanes need: hoisted out of enter_octants_packed's loop otherwise)
+    c.distx = (-ox) / S.dx;
+    c.disty = (-oy) / S.dy;
+    c.distz = (-oz) / S.dz;
     c.oct = 0;
     if (c.distx < 0.0f) { c.oct += 1; c.distx += kFltMax; }
     if (c.disty < 0.0f) { c.oct += 2; c.disty += kFltMax; }
@@ -281,6 +292,21 @@ __device__ __forceinline__ uint32_t stack_load(const char* lds, uint32_t off)
 #endif
 }
 
+// Node 0 in `rows` rows from `off` on: ancestors not pushed yet read as node 0, as in the reference's zeroed
+// stack. Four rows at a time (two instructions), the last four overlapping those before.
+__device__ __forceinline__ void stack_clear(char* lds, uint32_t off, uint32_t rows)
+{
+    const auto four = [&](uint32_t at) {
+        for (uint32_t k = 0; k < 4; k++) stack_store(lds, at + k * kRowBytes, 0u);
+    };
+    if (rows < 4u) {
+        for (uint32_t k = 0; k < rows; k++) stack_store(lds, off + k * kRowBytes, 0u);
+        return;
+    }
+    for (uint32_t k = 4; k < rows; k += 4, off += 4u * kRowBytes) four(off);
+    four(off + (((rows - 1u) & 3u) - 3u) * kRowBytes);
+}
+
 // A lane's stack base: row(h) = base + (32 - h) rows, for the column (first row) at `column`.
 __device__ __forceinline__ uint32_t stack_base(uint32_t column, uint32_t top) { return column + (top - 32u) * kRowBytes; }
 
@@ -314,8 +340,7 @@ __device__ __forceinline__ void octant_enter_packed(const cqx_subdag* tab, const
     const float exitt = min3f(((px + nsz) - S.ox) * S.ix, ((py + nsz) - S.oy) * S.iy, ((pz + nsz) - S.oz) * S.iz);
     S.phase = kLeave;
     if (!(entry < exitt)) return;
-    // ancestors not pushed yet read as node 0, as in the reference's zeroed stack
-    for (uint32_t r = 32u - P.top; r <= 32u; r++) stack_store(lds, base + r * kRowBytes, 0u);
+    stack_clear(lds, base + (32u - P.top) * kRowBytes, P.top + 1u);
     S.zstart = 32u - uint32_t(height);
     S.sp = base + S.zstart * kRowBytes;
     S.node = sd.pad0;
