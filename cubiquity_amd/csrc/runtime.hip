@@ -765,15 +765,16 @@ cqx_status bin_rays(cqx_ctx* ctx, const cqx_ray* rays, uint64_t n, const BinBox&
 // `chunk`: ray ids a wave claims per atomic, about a 32nd of a wave's share (64 to 4096). Smaller
 // claims end the launch with less left over in single waves, and with the 8 per-XCD counters on
 // separate cache lines their atomics are cheap: a quarter of the share was 4-9 % slower.
-// Defaults: the best launch of a sweep on the 1024^3 incoherent workload; the packed walk's steps do
-// more, and its service passes cost less, so it regroups every 12 steps (2.03 ms against 2.06 at 8), and
-// up to 2^23 rays runs 24 waves per CU (4.0 M rays at 4096^3: 1.03 ms against 1.09 at 32; 2^24 at 1024^3:
-// 2.14 against 2.04): the fewer waves share a SIMD, the sooner the last rays end.
+// Defaults: the best launch of a sweep on the 1024^3 incoherent workload. The packed walk's steps do
+// more and its service passes cost less, so it regroups every 16 steps, with 28 waves per CU, and 24 up to
+// 2^23 rays: the fewer waves share a SIMD and its L1, the sooner a wave's reads and the last rays end.
+// Measured (us, 24 / 28 / 32 waves): 2^24 rays at 1024^3 1959 / 1855 / 1933 (12 steps: 1927 / 1882 /
+// 1912), 4.0 M at 4096^3 983 / 1040 / 1068 (994 / 1045 / 1054).
 cqx_status persistent_shape(const cqx_ctx* ctx, const cqx_launch_cfg* cfg, uint32_t block, uint64_t n, bool packed,
                             uint32_t& blocks, uint32_t& regroup, uint32_t& refill, uint32_t& chunk)
 {
-    const uint32_t waves_per_cu = (cfg && cfg->waves_per_cu) ? cfg->waves_per_cu : packed && n <= (1u << 23) ? 24u : 32u;
-    regroup = (cfg && cfg->regroup_interval) ? cfg->regroup_interval : packed ? 12u : 8u;
+    const uint32_t waves_per_cu = (cfg && cfg->waves_per_cu) ? cfg->waves_per_cu : !packed ? 32u : n <= (1u << 23) ? 24u : 28u;
+    regroup = (cfg && cfg->regroup_interval) ? cfg->regroup_interval : packed ? 16u : 8u;
     refill = (cfg && cfg->refill_lanes) ? cfg->refill_lanes : 16u;
     if (waves_per_cu > 64 || regroup > 4096 || refill > 64)
         return fail(CQX_ERR_INVALID_ARG, "persistent launch parameters out of range");
@@ -956,7 +957,7 @@ void launch_dealt(const PackedSingle& src, bool lod, uint32_t block, hipStream_t
                   uint32_t chunk, const unsigned long long* gate = nullptr, uint32_t want = 0)
 {
     const uint64_t per_block = uint64_t(block / 64) * chunk;
-    launch_walk<true>(src, lod, (n + per_block - 1) / per_block, block, stream, n, n_dev, nullptr, 12u,
+    launch_walk<true>(src, lod, (n + per_block - 1) / per_block, block, stream, n, n_dev, nullptr, 16u,
                       chunk > 64 ? 16u : 64u, chunk, gate, want);
 }
 
@@ -1143,7 +1144,7 @@ void launch_batch_as(const Batch& src, const WalkLaunch& w, uint64_t total, hipS
     if (w.dealt) {
         const uint32_t ids = cqx::lanes_per_wave(total);
         hipLaunchKernelGGL((k_walk<Batch, kLod, true>), dim3(uint32_t((total + ids - 1) / ids)), dim3(64), size_t(rows) * 256,
-                           s, src, total, no_count, w.counters, 12u, 64u, rows, ids, no_gate, 0u);
+                           s, src, total, no_count, w.counters, 16u, 64u, rows, ids, no_gate, 0u);
     } else {
         hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, w.counters);
         hipLaunchKernelGGL((k_walk<Batch, kLod, false>), dim3(w.blocks), dim3(w.block), size_t(rows) * w.block * 4, s, src,

@@ -308,7 +308,7 @@ cqx_status cqx_volume_info(const cqx_dvolume* vol, const uint32_t** dev_nodes, u
 /* Launch parameters of the traversal kernel. With every field that shapes the launch zero (or no
  * configuration at all) the library picks the launch by the batch's size and, past 2^20 rays, by
  * whether a sample of the rays is coherent; otherwise zero fields take the built-in defaults
- * (variant 2, 256 threads, 32 waves per CU, or 24 up to 2^23 rays, regroup 12, refill 16; stores of
+ * (variant 2, 256 threads, 28 waves per CU, or 24 up to 2^23 rays, regroup 16, refill 16; stores of
  * more than 2^24 nodes or volumes past 2^22 voxels from the origin: 32 waves, regroup 8). */
 typedef struct {
     uint32_t variant;          /* 0 auto (the autotuner's choice), 1 one ray per lane, 2 persistent waves
