@@ -5,8 +5,8 @@
 //     spheres in order, and the levels above the regions in Morton order;
 //   k_edit_regions: one wave per region descends to the region's node and applies its spheres in
 //     order with fillBrush's arithmetic (voxelization.cpp:825-915; EditWalk::fill, here with an
-//     explicit stack, each node's 8 children tested on the wave's 64 lanes at once and a height-2
-//     node's 64 voxels in one step), interning changed nodes into the region's own list with its own
+//     explicit stack, each node's 8 children tested on the wave's 64 lanes at once and the 512 voxels
+//     of a height-3 node in one step), interning changed nodes into the region's own list with its own
 //     hash table; a node without listed children is first looked up in the device index over the
 //     store. A list that outgrows its slice stops its region, which runs again with a larger one;
 //   merge (k_merge_*): the lists laid end to end in region order and merged as merge_regions does:
@@ -208,15 +208,12 @@ struct RegionArgs {
 };
 
 // The walk of one region (one wave): lane l stands for child c = l / 8 of the node it is at and, of
-// that child, corner, child or voxel k = l % 8.
-//
-// EditWalk::fill visits a node per step; here a node of height 2 (its 8 children and their 64 voxels)
-// is one step too (brick): the corners of its height-1 children are their voxels, so the 64 tests of
-// one step decide children and voxels alike, and the children that changed are interned together,
-// 8 lanes probing for each. Above that the walk is depth first with the children's children read
-// as soon as a node is entered, so that entering a child waits for no memory. What is interned, and in
-// which order, is the recursion's. The phase lasts as long as its longest walk, a chain of dependent
-// reads: 1000 spheres in a 2048^3 volume 2.62 ms with a step per node, 0.70 ms now.
+// that child, corner or child k = l % 8; the height-2 children of a node of height 3 are one step together
+// (bricks). Above that the walk is depth first with the children's children read as soon as a node is
+// entered, so that entering a child waits for no memory. What is interned, and in which order, is the
+// recursion's. The phase lasts as long as its longest walk, a chain of dependent reads: 1000 spheres in a
+// 2048^3 volume 2.62 ms with a step per node, 0.69 ms with a step per height-2 node, 0.35 ms now (0.63 ms where
+// most new nodes are in neither the store nor the list, 0.73 before).
 struct Region {
     const RegionArgs& A;
     uint64_t poff;
@@ -290,7 +287,9 @@ __device__ __forceinline__ void probe_groups(const uint32_t* __restrict__ slots,
 // RegionStore::intern of each group's node (`w`: word k of group c's node) whose bit is set in
 // `active`, in group order: 8 equal material children collapse; a node without listed children
 // that is in the store is shared; otherwise the region's list keeps one copy of each node. The
-// group's node index in all its lanes; false when the list outgrew its slice.
+// group's node index in all its lanes; false when the list outgrew its slice. kNew: the nodes are known not to
+// collapse and not to be in the store.
+template <bool kNew = false>
 __device__ bool intern_groups(Region& R, uint32_t w, uint32_t active, uint32_t lane, uint32_t& result)
 {
     const RegionArgs& A = R.A;
@@ -308,7 +307,7 @@ __device__ bool intern_groups(Region& R, uint32_t w, uint32_t active, uint32_t l
     uint32_t r = uniform ? n.c[0] : kEmptySlot;
     const uint64_t hash = hash_node(n);
     uint64_t at = 0;
-    probe_groups(A.index, A.index_mask, A.nodes, n, hash, need && !listed, lane, r, at);
+    if (!kNew) probe_groups(A.index, A.index_mask, A.nodes, n, hash, need && !listed, lane, r, at);
     uint32_t* const tab = A.table + R.poff * 2;
     const uint64_t tmask = uint64_t(R.cap) * 2 - 1;
     uint32_t local = kEmptySlot;
@@ -383,33 +382,99 @@ __device__ __forceinline__ bool test_children(const Brush& b, uint32_t mat, uint
     return true;
 }
 
-// fillBrush on a node of height 2 whose child c is `child` in the lanes of group c: the new node.
-__device__ bool brick(Region& R, const Brush& b, uint32_t mat, uint32_t node, uint32_t child, int32_t lx, int32_t ly,
-                      int32_t lz, uint32_t lane, uint32_t& result)
+// Index of a store node with this content, or kEmptySlot: a lane's own search, two slots' nodes at a time.
+__device__ uint32_t store_find(const RegionArgs& A, const DNode& n)
 {
-    result = node;
-    const uint32_t c = lane >> 3, k = lane & 7u;
-    uint32_t fill, walk;
-    bool inside;
-    if (!test_children(b, mat, child, 2u, lx, ly, lz, lane, fill, walk, inside) || !(fill | walk)) return true;
-    const bool walked = (walk >> c) & 1u;
-    uint32_t out = ((fill >> c) & 1u) ? mat : child;
-    if (walk) {
-        const float x = float(int32_t(uint32_t(lx) + 2u * (c & 1u) + (k & 1u))),
-                    y = float(int32_t(uint32_t(ly) + 2u * ((c >> 1) & 1u) + ((k >> 1) & 1u))),
-                    z = float(int32_t(uint32_t(lz) + 2u * (c >> 2) + (k >> 2)));
-        const uint32_t v = walked ? R.child(child, k) : 0u;
-        const bool ok = !(b.hi[0] < x || b.lo[0] > x) && !(b.hi[1] < y || b.lo[1] > y) && !(b.hi[2] < z || b.lo[2] > z);
-        const bool set = walked && ok && inside && v != mat;
-        const uint32_t changed = bytes_any(__ballot(set));
-        if (changed) {
-            uint32_t r;
-            if (!intern_groups(R, set ? mat : v, changed, lane, r)) return false;
-            if ((changed >> c) & 1u) out = r;
+    for (uint64_t i = hash_node(n) & A.index_mask;; i += 2) {
+        const uint32_t s0 = A.index[i & A.index_mask], s1 = A.index[(i + 1) & A.index_mask];
+        if (s0 == kEmptySlot) return kEmptySlot;
+        const DNode a = load_node(A.nodes, s0), b = load_node(A.nodes, s1 == kEmptySlot ? s0 : s1);
+        if (node_eq(a, n)) return s0;
+        if (s1 == kEmptySlot) return kEmptySlot;
+        if (node_eq(b, n)) return s1;
+    }
+}
+
+// fillBrush on the children in `walk` of a node of height 3 (lower corner lo), height-2 nodes ("bricks"):
+// lane l stands for child c = l % 8 of brick l / 8, `kid`; `out` holds the brick's node in its 8 lanes and
+// receives the new one. A lane tests its child and the child's 8 voxels and searches the store for the
+// new node, for all bricks at once; what is not there goes into the region's list brick by brick, in
+// the recursion's order, and if everything is, the bricks' own nodes are interned together. A step per
+// brick instead (its 8 children by 8 lanes each) was a chain of 5 reads a brick, against 2 to 3 now and, with
+// nothing new, 5 for all 8.
+__device__ bool bricks(Region& R, const Brush& b, uint32_t mat, uint32_t walk, uint32_t kid, int32_t lx, int32_t ly,
+                       int32_t lz, uint32_t lane, uint32_t& out, uint32_t& changed)
+{
+    const RegionArgs& A = R.A;
+    const uint32_t g = lane >> 3, c = lane & 7u;
+    const uint32_t x0 = uint32_t(lx) + 4u * (g & 1u) + 2u * (c & 1u), y0 = uint32_t(ly) + 4u * ((g >> 1) & 1u) + 2u * ((c >> 1) & 1u),
+                   z0 = uint32_t(lz) + 4u * (g >> 2) + 2u * (c >> 2);
+    const float fx[2] = { float(int32_t(x0)), float(int32_t(x0 + 1u)) }, fy[2] = { float(int32_t(y0)), float(int32_t(y0 + 1u)) },
+                fz[2] = { float(int32_t(z0)), float(int32_t(z0 + 1u)) };
+    uint32_t next = kid;   // the child's new node
+    bool fresh = false;    // not settled: in neither the store nor, yet, the list
+    DNode n;
+    const bool ok = ((walk >> g) & 1u) && kid != mat && !(b.hi[0] < fx[0] || b.lo[0] > fx[1]) &&
+                    !(b.hi[1] < fy[0] || b.lo[1] > fy[1]) && !(b.hi[2] < fz[0] || b.lo[2] > fz[1]);
+    if (ok) {
+        uint32_t inside = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) inside |= (b.contains(fx[k & 1u], fy[(k >> 1) & 1u], fz[k >> 2]) ? 1u : 0u) << k;
+        if (inside == 0xffu) next = mat;
+        else if (!b.box_outside(fx[0], fy[0], fz[0], fx[1], fy[1], fz[1])) {
+            if (kid < kMat)
+                for (uint32_t& w : n.c) w = kid;
+            else n = kid >= A.base ? load_node(A.pool, R.poff + (kid - A.base)) : load_node(A.nodes, kid);
+            bool differs = false, uniform = true, listed = false;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) {
+                const float x = fx[k & 1u], y = fy[(k >> 1) & 1u], z = fz[k >> 2];
+                const bool in = !(b.hi[0] < x || b.lo[0] > x) && !(b.hi[1] < y || b.lo[1] > y) && !(b.hi[2] < z || b.lo[2] > z);
+                if (in && ((inside >> k) & 1u) && n.c[k] != mat) {
+                    n.c[k] = mat;
+                    differs = true;
+                }
+                uniform = uniform && n.c[k] == n.c[0];
+                listed = listed || n.c[k] >= A.base;
+            }
+            if (differs) {
+                next = uniform && n.c[0] < kMat ? n.c[0] : listed ? kEmptySlot : store_find(A, n);
+                fresh = next == kEmptySlot;
+            }
         }
     }
-    if (__ballot(out != child) == 0) return true;
-    return intern_one(R, out, lane, result);
+    if (__ballot(fresh) == 0) { // word c of brick g's node is `next`
+        const uint32_t differ = bytes_any(__ballot(next != kid && ((walk >> g) & 1u)));
+        if (!differ) return true;
+        uint32_t r;
+        if (!intern_groups(R, next, differ, lane, r)) return false;
+        if ((differ >> g) & 1u) out = r; // (a brick that changed is another node)
+        changed = 1u;
+        return true;
+    }
+    for (; walk; walk &= walk - 1u) {
+        const uint32_t at = uint32_t(__builtin_ctz(walk));
+        const uint32_t add = uint32_t(__ballot(fresh) >> (8u * at)) & 0xffu; // children of brick `at`
+        if (add) { // to lane (group c', word k) from lane 8 at + c'
+            uint32_t w = 0, r;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) {
+                const uint32_t v = uint32_t(__shfl(int(n.c[k]), int(8u * at + g)));
+                w = k == c ? v : w;
+            }
+            if (!intern_groups<true>(R, w, add, lane, r)) return false;
+            const uint32_t mine = uint32_t(__shfl(int(r), int(8u * c)));
+            if (g == at && fresh) next = mine;
+        }
+        if ((__ballot(next != kid) >> (8u * at) & 0xffu) == 0) continue;
+        uint32_t r;
+        const uint32_t w = uint32_t(__shfl(int(next), int(8u * at + c)));
+        if (!intern_groups(R, w, 1u, lane, r)) return false;
+        r = uni(r); // of group 0
+        if (g == at) out = r;
+        changed = 1u;
+    }
+    return true;
 }
 
 // A node of height 3 or more on the way down, saved while a child of it is walked.
@@ -464,6 +529,11 @@ __device__ bool fill(Region& R, const Brush& b, uint32_t mat, uint32_t node, uin
             changed |= differs ? 1u : 0u;
             continue;
         }
+        if (height == 3) {
+            if (!bricks(R, b, mat, walk, kid, lx, ly, lz, lane, out, changed)) return false;
+            walk = 0;
+            continue;
+        }
         const uint32_t at = uint32_t(__builtin_ctz(walk));
         walk &= walk - 1u;
         const uint32_t side = 1u << (height - 1);
@@ -471,15 +541,6 @@ __device__ bool fill(Region& R, const Brush& b, uint32_t mat, uint32_t node, uin
         const uint32_t grand = uint32_t(__shfl(int(kid), int(8 * at + c))); // the child's child c
         const int32_t cx = int32_t(uint32_t(lx) + side * (at & 1u)), cy = int32_t(uint32_t(ly) + side * ((at >> 1) & 1u)),
                       cz = int32_t(uint32_t(lz) + side * (at >> 2));
-        if (height == 3) {
-            uint32_t res;
-            if (!brick(R, b, mat, child, grand, cx, cy, cz, lane, res)) return false;
-            if (res != child) {
-                changed = 1u;
-                if (c == at) out = res;
-            }
-            continue;
-        }
         uint32_t cset, cwalk;
         if (!test_children(b, mat, grand, side >> 1, cx, cy, cz, lane, cset, cwalk, corner)) continue;
         Frame& f = st[sp++];
