@@ -97,9 +97,10 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 //                   ray per lane.
 //   claimed         persistent waves claim `chunk` ids at a time from the queues' counters
 // `gate`: a launch that runs only when the sampled flag there equals `want` (k_sample_rays).
-// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take it to 6.
+// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take 72 and 7 waves (24 volumes
+// 193 us with 6 waves, 189 with 7, 194 with 8 and 8 to 13 registers spilled).
 template <typename Source, bool kLod, bool kDealt>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 6)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 7)))
 k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
        uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk, const unsigned long long* __restrict__ gate,
        uint32_t want)
