@@ -12,8 +12,8 @@
 //   merge (k_merge_*): the lists laid end to end in region order and merged as merge_regions does:
 //     level by level, the lowest list position among equal nodes is kept, the kept ones are
 //     appended in list order;
-//   k_edit_top: one workgroup rebuilds the levels above the regions bottom-up, each level's changed
-//     nodes interned in Morton order (rebuild_levels);
+//   k_top_*: the levels above the regions rebuilt bottom-up, each level's changed nodes interned in Morton
+//     order (rebuild_levels);
 //   k_find_subdags: the new root's SubDAGs (findSubDAG, raytracing.cpp:43-87).
 // The index over the store (open addressing on the node hash; among equal nodes the lowest index)
 // is built on a volume's first edit and extended with every appended node. Appended nodes only
@@ -133,7 +133,7 @@ struct EditReport {
     uint32_t count;     // store size after the levels above the regions
     uint32_t root;
     uint32_t deep;      // k_find_subdags: a single-child chain deeper than the tree
-    uint32_t pad;
+    uint32_t fresh[29]; // per level above the regions: whether it has new nodes
     cqx_subdag sub[8];
 };
 
@@ -801,6 +801,7 @@ __global__ void __launch_bounds__(64) k_edit_begin(EditReport* __restrict__ rep)
         rep->outgrown = 0u;
         rep->next_run = 0u;
     }
+    if (threadIdx.x < sizeof(rep->fresh) / 4) rep->fresh[threadIdx.x] = 0u;
 }
 
 __global__ void __launch_bounds__(256) k_merge_kept(MergeArgs M, uint64_t* kept)
@@ -853,6 +854,9 @@ struct TopArgs {
     uint32_t count;       // store size after the merge
     EditReport* rep;
     uint32_t* old;        // per entry of level >= 1: the node it held before the edits
+
+    // The new node of entry j of level l.
+    __device__ uint32_t result(uint32_t l, uint32_t j) const { return l == 0 ? results[morton_regions[j]] : res[j]; }
 };
 
 // Index of a store node with this content, or kEmptySlot, while nodes are appended and inserted: 4
@@ -877,7 +881,7 @@ __device__ uint32_t index_find(const uint32_t* nodes, const uint32_t* slots, uin
 // lanes. Above a volume's own height a level holds an entry or a few and depends on the one below, so
 // the time is a chain of memory latencies: per level one read going down, and going up the index slots,
 // a node and the insertion, the old node's words being read a level ahead. At 2048^3, 1000 spheres of
-// radius 2 to 16 (4700 regions, 24 of the 27 levels small): k_edit_top 780 us with every level on the
+// radius 2 to 16 (4700 regions, 24 of the 27 levels small): 780 us with every level on the
 // workgroup (5 barriers and as many passes through memory each, fences at device scope), 200 us so.
 constexpr uint32_t kTopLevels = 28; // 32 - hs for hs >= 5, and level 0
 struct SmallTop {
@@ -966,7 +970,7 @@ __device__ void top_small_up(const TopArgs& A, SmallTop& S, uint32_t base, uint3
             const uint32_t k = S.kids[e - b0], cb = (k & 0x3ffffffu) + c0;
             for (uint32_t j = cb; j <= cb + (k >> 29); j++) {
                 const uint32_t id = l > S.first ? (S.kids[j - b0] >> 26) & 7u : key_octant(A.keys[j]);
-                const uint32_t x = l > S.first ? S.below[j - S.off[l - 1]] : A.res[j];
+                const uint32_t x = l > S.first ? S.below[j - S.off[l - 1]] : A.result(l - 1, j);
 #pragma unroll
                 for (uint32_t c = 0; c < 8; c++)
                     if (c == id && out.c[c] != x) {
@@ -1009,117 +1013,148 @@ __device__ void top_small_up(const TopArgs& A, SmallTop& S, uint32_t base, uint3
     }
 }
 
-// One workgroup, so its barriers order its memory operations: all of them go through one L1 and one L2.
-__global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
+// The levels of more than 64 entries ("large", the lowest ones) are spread over the chip, a launch per step
+// and level, and the new nodes of a level, if any, appended by one workgroup. At 2048^3, 1000 spheres, with
+// four large levels: 130 us for the whole, against 200 us with every level on one workgroup, whose threads
+// took 5 entries of a level one after the other; where the nodes are new, 290 us against 436.
+
+// Old nodes of the small levels and of the level below them, for the launches of the large ones.
+__global__ void __launch_bounds__(kTopBlock) k_top_begin(TopArgs A)
 {
-    __shared__ uint32_t wave_kept[kTopBlock / 64];
     __shared__ SmallTop small;
-    __shared__ uint32_t count_s;
-    const uint32_t t = threadIdx.x, T = blockDim.x;
-    if (t == 0) count_s = A.count;
-    for (uint32_t i = A.lvl_off[0] + t; i < A.lvl_off[1]; i += T) A.res[i] = A.results[A.morton_regions[i]];
-    top_stage(A, small, t, T);
-    // The nodes the entries held before the edits, top down: the top entry (height 32, one key)
-    // holds the root, and an entry's children hold the children of its node (node_at of every
-    // entry, with one read per entry instead of one per level above it).
+    const uint32_t t = threadIdx.x;
+    if (t == 0) A.rep->count = A.count;
+    top_stage(A, small, t, blockDim.x);
     if (t < 64) top_small_down(A, small, t);
     __syncthreads();
-    for (uint32_t l = small.first - 1; l >= 2; l--) {
-        for (uint32_t i = small.off[l] + t; i < small.off[l + 1]; i += T) {
-            const uint32_t p = A.old[i];
-            const uint32_t ce = A.cend[i];
-            for (uint32_t j = A.cbeg[i]; j < ce; j++) A.old[j] = p < kMat ? p : A.nodes[uint64_t(p) * 8 + key_octant(A.keys[j])];
-        }
-        __syncthreads();
-    }
-    for (uint32_t l = 1; l < small.first; l++) {
-        const uint32_t b = small.off[l], e = small.off[l + 1];
-        for (uint32_t i = b + t; i < e; i += T) {
-            const uint32_t old = A.old[i];
-            DNode out;
-            if (old >= kMat) out = load_node(A.nodes, old);
-            else
-                for (uint32_t& x : out.c) x = old;
-            bool changed = false;
-            const uint32_t ce = A.cend[i];
-            for (uint32_t j = A.cbeg[i]; j < ce; j++) {
-                const uint32_t id = key_octant(A.keys[j]), x = A.res[j];
+    const uint32_t b = small.off[small.first], n = small.off[A.levels + 1] - b;
+    for (uint32_t i = t; i < n; i += blockDim.x) A.old[b + i] = small.old[i];
+}
+
+// Old nodes of level l - 1, from those of level l.
+__global__ void __launch_bounds__(256) k_top_old(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    const uint32_t i = begin + blockIdx.x * 256u + threadIdx.x;
+    if (i >= end) return;
+    const uint32_t p = A.old[i], ce = A.cend[i];
+    for (uint32_t j = A.cbeg[i]; j < ce; j++) A.old[j] = p < kMat ? p : A.nodes[uint64_t(p) * 8 + key_octant(A.keys[j])];
+}
+
+// The nodes of level l after the edits, where the store has them; the others as candidates.
+__global__ void __launch_bounds__(64) k_top_build(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    const uint32_t i = begin + blockIdx.x * 64u + threadIdx.x;
+    if (i >= end) return;
+    const uint32_t old = A.old[i];
+    DNode out;
+    if (old >= kMat) out = load_node(A.nodes, old);
+    else
+        for (uint32_t& x : out.c) x = old;
+    bool changed = false;
+    const uint32_t ce = A.cend[i];
+    for (uint32_t j = A.cbeg[i]; j < ce; j++) {
+        const uint32_t id = key_octant(A.keys[j]), x = A.result(l - 1, j);
 #pragma unroll
-                for (uint32_t c = 0; c < 8; c++)
-                    if (c == id && out.c[c] != x) {
-                        out.c[c] = x;
-                        changed = true;
-                    }
+        for (uint32_t c = 0; c < 8; c++)
+            if (c == id && out.c[c] != x) {
+                out.c[c] = x;
+                changed = true;
             }
-            uint32_t r = old, cand = 0;
-            if (changed) { // Interner::intern: collapse, else the store's node, else new
-                bool uniform = out.c[0] < kMat;
-                for (int c = 1; c < 8; c++) uniform = uniform && out.c[c] == out.c[0];
-                if (uniform) r = out.c[0];
-                else {
-                    r = index_find(A.nodes, A.index, A.index_mask, out);
-                    if (r == kEmptySlot) {
-                        cand = 1;
-                        store_node(A.ckey, i, out);
-                    }
-                }
-            }
-            A.res[i] = r;
-            A.cand[i] = cand;
-        }
-        __syncthreads();
-        // equal new nodes of this level: the first in Morton order is kept
-        const uint64_t tmask = (A.tab_off[l + 1] - A.tab_off[l]) - 1;
-        uint32_t* const tab = A.table + A.tab_off[l];
-        for (uint32_t i = b + t; i < e; i += T) {
-            if (!A.cand[i]) continue;
-            const DNode k = load_node_coherent(A.ckey, i);
-            for (uint64_t s = hash_node(k) & tmask;; s = (s + 1) & tmask) {
-                const uint32_t cur = atomicCAS(&tab[s], kEmptySlot, i);
-                if (cur == kEmptySlot || node_eq(load_node_coherent(A.ckey, cur), k)) {
-                    if (cur != kEmptySlot) atomicMin(&tab[s], i);
-                    A.cslot[i] = s;
-                    break;
-                }
+    }
+    uint32_t r = old, cand = 0;
+    if (changed) { // Interner::intern: collapse, else the store's node, else new
+        bool uniform = out.c[0] < kMat;
+        for (int c = 1; c < 8; c++) uniform = uniform && out.c[c] == out.c[0];
+        if (uniform) r = out.c[0];
+        else {
+            r = index_find(A.nodes, A.index, A.index_mask, out);
+            if (r == kEmptySlot) {
+                cand = 1;
+                store_node(A.ckey, i, out);
+                A.rep->fresh[l] = 1u;
             }
         }
-        __syncthreads();
-        for (uint32_t i = b + t; i < e; i += T)
-            if (A.cand[i]) A.crep[i] = __hip_atomic_load(tab + A.cslot[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        // the kept ones appended in order: a scan over the level in chunks of T entries (each wave
-        // ranks its lanes by ballot, then adds the counts of the waves before it)
-        uint32_t base = count_s;
-        for (uint32_t c0 = b; c0 < e; c0 += T) {
-            const uint32_t i = c0 + t;
-            const bool keep = i < e && A.cand[i] && A.crep[i] == i;
-            const uint64_t bal = __ballot(keep);
-            const uint32_t lane = t & 63u, w = t >> 6;
-            if (lane == 0) wave_kept[w] = uint32_t(__popcll(bal));
-            __syncthreads();
-            uint32_t before = 0, all = 0;
-            for (uint32_t v = 0; v < T / 64; v++) {
-                before += v < w ? wave_kept[v] : 0u;
-                all += wave_kept[v];
-            }
-            if (keep) {
-                const uint32_t at = base + before + uint32_t(__popcll(bal & ((1ull << lane) - 1ull)));
-                store_node(A.nodes, at, load_node_coherent(A.ckey, i));
-                A.res[i] = at; // a kept entry's node; the others copy theirs below
-            }
-            base += all;
-            __syncthreads();
+    }
+    A.res[i] = r;
+    A.cand[i] = cand;
+}
+
+// Equal new nodes of level l: the first in Morton order is kept.
+__global__ void __launch_bounds__(64) k_top_unique(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    if (!A.rep->fresh[l]) return;
+    const uint32_t i = begin + blockIdx.x * 64u + threadIdx.x;
+    if (i >= end || !A.cand[i]) return;
+    const uint64_t tmask = (A.tab_off[l + 1] - A.tab_off[l]) - 1;
+    uint32_t* const tab = A.table + A.tab_off[l];
+    const DNode k = load_node(A.ckey, i);
+    for (uint64_t s = hash_node(k) & tmask;; s = (s + 1) & tmask) {
+        const uint32_t cur = atomicCAS(&tab[s], kEmptySlot, i);
+        if (cur == kEmptySlot || node_eq(load_node(A.ckey, cur), k)) {
+            if (cur != kEmptySlot) atomicMin(&tab[s], i);
+            A.cslot[i] = s;
+            break;
         }
+    }
+}
+
+// The kept nodes of level l appended in order: one workgroup, a scan over the level in chunks of its size
+// (each wave ranks its lanes by ballot, then adds the counts of the waves before it).
+__global__ void __launch_bounds__(kTopBlock) k_top_append(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    if (!A.rep->fresh[l]) return;
+    __shared__ uint32_t wave_kept[kTopBlock / 64];
+    const uint32_t t = threadIdx.x, T = blockDim.x, lane = t & 63u, w = t >> 6;
+    const uint32_t* const tab = A.table + A.tab_off[l];
+    uint32_t base = A.rep->count;
+    for (uint32_t c0 = begin; c0 < end; c0 += T) {
+        const uint32_t i = c0 + t;
+        uint32_t first = kEmptySlot;
+        if (i < end && A.cand[i]) A.crep[i] = first = tab[A.cslot[i]];
+        const bool keep = first == i;
+        const uint64_t bal = __ballot(keep);
+        if (lane == 0) wave_kept[w] = uint32_t(__popcll(bal));
         __syncthreads();
-        for (uint32_t i = b + t; i < e; i += T)
-            if (A.cand[i]) {
-                if (A.crep[i] != i) A.res[i] = A.res[A.crep[i]];
-                else index_insert<true>(A.nodes, A.index, A.index_mask, A.res[i], load_node_coherent(A.ckey, i));
-            }
-        if (t == 0) count_s = base;
+        uint32_t before = 0, all = 0;
+        for (uint32_t v = 0; v < T / 64; v++) {
+            before += v < w ? wave_kept[v] : 0u;
+            all += wave_kept[v];
+        }
+        if (keep) A.res[i] = base + before + uint32_t(__popcll(bal & ((1ull << lane) - 1ull)));
+        base += all;
         __syncthreads();
     }
-    if (t < 64) top_small_up(A, small, count_s, t);
+    if (t == 0) A.rep->count = base;
+}
+
+// The kept nodes into the store and its index; the others take the index of theirs.
+__global__ void __launch_bounds__(64) k_top_write(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    if (!A.rep->fresh[l]) return;
+    const uint32_t i = begin + blockIdx.x * 64u + threadIdx.x;
+    if (i >= end || !A.cand[i]) return;
+    if (A.crep[i] == i) store_node(A.nodes, A.res[i], load_node(A.ckey, i));
+    else A.res[i] = A.res[A.crep[i]];
+}
+__global__ void __launch_bounds__(64) k_top_index(TopArgs A, uint32_t l, uint32_t begin, uint32_t end)
+{
+    if (!A.rep->fresh[l]) return;
+    const uint32_t i = begin + blockIdx.x * 64u + threadIdx.x;
+    if (i < end && A.cand[i] && A.crep[i] == i) index_insert(A.nodes, A.index, A.index_mask, A.res[i], load_node(A.ckey, i));
+}
+
+// The small levels; `begun`: k_top_begin and the large levels' launches came before.
+__global__ void __launch_bounds__(kTopBlock) k_top_small(TopArgs A, uint32_t begun)
+{
+    __shared__ SmallTop small;
+    const uint32_t t = threadIdx.x;
+    top_stage(A, small, t, blockDim.x);
+    if (begun) {
+        const uint32_t b = small.off[small.first], n = small.off[A.levels + 1] - b;
+        for (uint32_t i = t; i < n; i += blockDim.x) small.old[i] = A.old[b + i];
+        __syncthreads();
+    } else if (t < 64) top_small_down(A, small, t);
+    if (t < 64) top_small_up(A, small, begun ? A.rep->count : A.count, t);
 }
 
 // findSubDAG (raytracing.cpp:43-87) of every root child, as cqx::find_subdags, one thread each, with
@@ -1128,7 +1163,7 @@ __global__ void __launch_bounds__(kTopBlock) k_edit_top(TopArgs A)
 __global__ void __launch_bounds__(64) k_find_subdags(const uint32_t* __restrict__ nodes, uint32_t root,
                                                      cqx_subdag* __restrict__ out, EditReport* __restrict__ rep)
 {
-    if (root == kEmptySlot) root = rep->root; // the one k_edit_top left there
+    if (root == kEmptySlot) root = rep->root; // the one k_top_small left there
     const uint32_t c = threadIdx.x;
     bool deep = false;
     cqx_subdag s{};
@@ -1707,7 +1742,25 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
     TopArgs T{ vol->nodes, E->index, E->index_cap - 1, vol->root, hs, levels, d_lvl_off, d_tkeys, d_cbeg, d_cend,
                d_morton, d_results, d_res, d_cand, d_ckey, d_cand + ntop, d_cslot, d_ttable, d_tab_off,
                uint32_t(base + kept_total), d_rep, d_old };
-    hipLaunchKernelGGL(k_edit_top, dim3(1), dim3(kTopBlock), 0, 0, T);
+    uint32_t first_small = 1;
+    while (h_lvl_off[first_small + 1] - h_lvl_off[first_small] > 64) first_small++;
+    if (first_small > 1) {
+        hipLaunchKernelGGL(k_top_begin, dim3(1), dim3(kTopBlock), 0, 0, T);
+        for (uint32_t l = first_small - 1; l >= 2; l--) {
+            const uint32_t lb = h_lvl_off[l], le = h_lvl_off[l + 1];
+            hipLaunchKernelGGL(k_top_old, dim3((le - lb + 255) / 256), dim3(256), 0, 0, T, l, lb, le);
+        }
+        for (uint32_t l = 1; l < first_small; l++) {
+            const uint32_t lb = h_lvl_off[l], le = h_lvl_off[l + 1];
+            const dim3 waves((le - lb + 63) / 64);
+            hipLaunchKernelGGL(k_top_build, waves, dim3(64), 0, 0, T, l, lb, le);
+            hipLaunchKernelGGL(k_top_unique, waves, dim3(64), 0, 0, T, l, lb, le);
+            hipLaunchKernelGGL(k_top_append, dim3(1), dim3(kTopBlock), 0, 0, T, l, lb, le);
+            hipLaunchKernelGGL(k_top_write, waves, dim3(64), 0, 0, T, l, lb, le);
+            hipLaunchKernelGGL(k_top_index, waves, dim3(64), 0, 0, T, l, lb, le);
+        }
+    }
+    hipLaunchKernelGGL(k_top_small, dim3(1), dim3(kTopBlock), 0, 0, T, first_small > 1 ? 1u : 0u);
     hipLaunchKernelGGL(k_find_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, kEmptySlot, vol->sub, d_rep);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(&rep, d_rep, sizeof(rep), hipMemcpyDeviceToHost));
