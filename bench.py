@@ -717,9 +717,9 @@ def main():
             "l2_hit_rate": l2_hit_rate,
             "traffic_profile": profile,
             "timed_launch": timed_launch,
-            "limiter": ("measured at 1024^3: cache-resident (the 20 MB store sits in the MALL; L2 hits ~91 %, "
-                        "HBM traffic ~0.3x the algorithmic bytes), bound by dependent child-read latency and "
-                        "divergent VALU work (lane utilisation ~38 %), not by HBM bandwidth; 'hbm' names the "
+            "limiter": ("measured at 1024^3: cache-resident (the store sits in the MALL; L2 hits ~86 %, HBM traffic "
+                        "~0.22x the algorithmic bytes), bound by the issue of divergent VALU work (one instruction "
+                        "per 2.5 cycles and SIMD, ~46 % of lanes active), not by HBM bandwidth; 'hbm' names the "
                         "roofline the algorithmic bytes are priced against" if headline else
                         "measured at 16384^3 (tuned launch): ~1.6x the algorithmic bytes fetched (a 128-B line "
                         "per 32-B node read, L2 hits ~52 %), at ~0.75 of HBM peak on that traffic: bound by HBM "
