@@ -1042,10 +1042,10 @@ cqx_status capture(cqx_ctx* ctx, PtPlan* p, hipStream_t s)
         const dim3 walk(src.list.units(chunk)), shade(src.list.units(block));
         const uint32_t refill = chunk > 64 ? 16u : 64u;
         if (lod)
-            hipLaunchKernelGGL((k_walk<PathRays, true, true>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 16u, refill,
+            hipLaunchKernelGGL((k_walk<PathRays, true, kDealt>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 16u, refill,
                                rows, chunk, nullptr, 0u);
         else
-            hipLaunchKernelGGL((k_walk<PathRays, false, true>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 16u, refill,
+            hipLaunchKernelGGL((k_walk<PathRays, false, kDealt>), walk, dim3(64), lds, s, src, P, nullptr, nullptr, 16u, refill,
                                rows, chunk, nullptr, 0u);
         hipLaunchKernelGGL((k_pt_shade<kRadiance, uint64_t>), shade, dim3(block), 0, s, p->dparams, P, depth,
                            pcg_jump(depth), list(depth), hits, list(depth + 1), p->L, vmat, vstat);

@@ -900,7 +900,8 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
 // Up to kLaneRays one ray per lane: close to the best for either kind. Beyond, the kinds part: a sample
 // of the rays decides on the device between one ray per lane for coherent ones and, for the others,
 // dealt runs of 4 x 64 up to kDealtRays, claims by persistent waves past it (whose tail no longer
-// matters there). The sample and the launch that returns at once take about 10 us.
+// matters there). The sample takes 3 us; up to kDealtRays one of two launches returns at once (2 us), past
+// it one launch is either.
 constexpr uint64_t kLaneRays = 1u << 20;
 constexpr uint64_t kDealtRays = 5u << 19; // 2.6 M
 constexpr uint64_t kGateRays = uint64_t(1) << 31; // the lane launch's grid stays below 2^32 threads
@@ -936,8 +937,8 @@ bool launch_open(const cqx_launch_cfg* c)
 
 namespace {
 
-// k_walk over one volume, dealt (chunk ids per wave) or claimed.
-template <bool kDealt>
+// k_walk over one volume (`chunk`: ids per wave, or per claim).
+template <WalkForm kForm>
 void launch_walk(const PackedSingle& src, bool lod, uint64_t blocks, uint32_t block, hipStream_t stream, uint64_t n,
                  const uint32_t* n_dev, unsigned long long* counters, uint32_t regroup, uint32_t refill, uint32_t chunk,
                  const unsigned long long* gate = nullptr, uint32_t want = 0)
@@ -945,10 +946,10 @@ void launch_walk(const PackedSingle& src, bool lod, uint64_t blocks, uint32_t bl
     const uint32_t rows = src.P.top + 1u;
     const size_t lds = size_t(rows) * block * sizeof(uint32_t);
     if (lod)
-        hipLaunchKernelGGL((k_walk<PackedSingle, true, kDealt>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
+        hipLaunchKernelGGL((k_walk<PackedSingle, true, kForm>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
                            n_dev, counters, regroup, refill, rows, chunk, gate, want);
     else
-        hipLaunchKernelGGL((k_walk<PackedSingle, false, kDealt>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
+        hipLaunchKernelGGL((k_walk<PackedSingle, false, kForm>), dim3(uint32_t(blocks)), dim3(block), lds, stream, src, n,
                            n_dev, counters, regroup, refill, rows, chunk, gate, want);
 }
 
@@ -957,7 +958,7 @@ void launch_dealt(const PackedSingle& src, bool lod, uint32_t block, hipStream_t
                   uint32_t chunk, const unsigned long long* gate = nullptr, uint32_t want = 0)
 {
     const uint64_t per_block = uint64_t(block / 64) * chunk;
-    launch_walk<true>(src, lod, (n + per_block - 1) / per_block, block, stream, n, n_dev, nullptr, 16u,
+    launch_walk<kDealt>(src, lod, (n + per_block - 1) / per_block, block, stream, n, n_dev, nullptr, 16u,
                       chunk > 64 ? 16u : 64u, chunk, gate, want);
 }
 
@@ -1034,12 +1035,16 @@ cqx_status launch_intersect(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray*
         else if (open && !n_dev && n < kGateRays) {
             const unsigned long long* const flag = counters + kFlagWord;
             hipLaunchKernelGGL(k_sample_rays, dim3(1), dim3(64), 0, stream, counters, rays, n, PP.top);
-            launch_dealt(src, lod, 256u, stream, n, nullptr, 64u, flag, 1u);
-            if (n <= kDealtRays) launch_dealt(src, lod, 64u, stream, n, nullptr, 256u, flag, 0u);
-            else launch_walk<false>(src, lod, blocks, block, stream, n, nullptr, counters, regroup, refill, chunk, flag, 0u);
+            if (n <= kDealtRays) {
+                launch_dealt(src, lod, 256u, stream, n, nullptr, 64u, flag, 1u);
+                launch_dealt(src, lod, 64u, stream, n, nullptr, 256u, flag, 0u);
+            } else {
+                launch_walk<kSampled>(src, lod, (n + block - 1) / block, block, stream, n, nullptr, counters, regroup, refill,
+                                      chunk, flag, blocks);
+            }
         } else {
             hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, stream, counters);
-            launch_walk<false>(src, lod, blocks, block, stream, n, n_dev, counters, regroup, refill, chunk);
+            launch_walk<kClaimed>(src, lod, blocks, block, stream, n, n_dev, counters, regroup, refill, chunk);
         }
     } else if (variant == 1) {
         const uint64_t blocks = (n + block - 1) / block;
@@ -1143,11 +1148,11 @@ void launch_batch_as(const Batch& src, const WalkLaunch& w, uint64_t total, hipS
     const unsigned long long* const no_gate = nullptr;
     if (w.dealt) {
         const uint32_t ids = cqx::lanes_per_wave(total);
-        hipLaunchKernelGGL((k_walk<Batch, kLod, true>), dim3(uint32_t((total + ids - 1) / ids)), dim3(64), size_t(rows) * 256,
+        hipLaunchKernelGGL((k_walk<Batch, kLod, kDealt>), dim3(uint32_t((total + ids - 1) / ids)), dim3(64), size_t(rows) * 256,
                            s, src, total, no_count, w.counters, 16u, 64u, rows, ids, no_gate, 0u);
     } else {
         hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, w.counters);
-        hipLaunchKernelGGL((k_walk<Batch, kLod, false>), dim3(w.blocks), dim3(w.block), size_t(rows) * w.block * 4, s, src,
+        hipLaunchKernelGGL((k_walk<Batch, kLod, kClaimed>), dim3(w.blocks), dim3(w.block), size_t(rows) * w.block * 4, s, src,
                            total, no_count, w.counters, w.regroup, w.refill, rows, w.chunk, no_gate, 0u);
     }
 }

@@ -91,22 +91,34 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v)
            uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(v >> 32)))) << 32;
 }
 
-// What a wave does is the same in both forms; they differ in where its ray ids come from.
-//   dealt (kDealt)  wave w owns `chunk` ids or fewer (Source::deal): no counters, no claims, the
+// What a wave does is the same in all forms; they differ in where its ray ids come from.
+//   kDealt          wave w owns `chunk` ids or fewer (Source::deal): no counters, no claims, the
 //                   hardware's dispatcher balances the load. With chunk <= 64 and refill 64 it is one
 //                   ray per lane.
-//   claimed         persistent waves claim `chunk` ids at a time from the queues' counters
-// `gate`: a launch that runs only when the sampled flag there equals `want` (k_sample_rays).
+//   kClaimed        persistent waves claim `chunk` ids at a time from the queues' counters
+//   kSampled        dealt, one ray per lane, where the sampled flag at `gate` is set (k_sample_rays), and
+//                   otherwise claimed by the first `want` workgroups; the rest end at once, in the slots
+//                   that those leave free (as a launch of its own they took 17 us of 1.87 ms at 2^24 rays)
+// With `gate`, kDealt and kClaimed launches run only when the flag equals `want`.
 // At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take 72 and 7 waves (24 volumes
 // 193 us with 6 waves, 189 with 7, 194 with 8 and 8 to 13 registers spilled).
-template <typename Source, bool kLod, bool kDealt>
+enum WalkForm { kClaimed, kDealt, kSampled };
+
+template <typename Source, bool kLod, WalkForm kForm>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Source::kUniform ? 8 : 7)))
 k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long long* __restrict__ counters,
        uint32_t regroup, uint32_t refill, uint32_t rows, uint32_t chunk, const unsigned long long* __restrict__ gate,
        uint32_t want)
 {
     extern __shared__ char lds_rows[];
-    if (gate && *gate != want) return;
+    bool dealt = kForm == kDealt;
+    if constexpr (kForm == kSampled) {
+        dealt = *gate != 0;
+        if (dealt) refill = chunk = 64u;
+        else if (blockIdx.x >= want) return;
+    } else {
+        if (gate && *gate != want) return;
+    }
     if (n_dev) {
         const uint64_t nd = *n_dev;
         n = nd < n ? nd : n;
@@ -132,7 +144,7 @@ k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long
     uint32_t qc = blockIdx.x % kQueues; // current queue
     uint32_t drained = 0;               // queues found empty so far
     uint64_t c_next = 0, c_end = 0;     // ray ids claimed by this wave
-    if constexpr (kDealt) {
+    if (kForm != kClaimed && dealt) {
         const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
         src.deal(uint64_t(blockIdx.x) * (blockDim.x >> 6) + wave, chunk, n, c_next, c_end);
         drained = kQueues;
