@@ -574,7 +574,11 @@ __device__ __forceinline__ void walk_step_packed_any(const PackedParams& P, Pack
 __device__ __forceinline__ uint32_t entered_voxel_plain(float o, float d, float t, float lo, float hi, bool entry_axis)
 {
     const float q = floorf(o + d * t);
+#if defined(__AMDGCN__)
+    const float c = __builtin_amdgcn_fmed3f(q, lo, hi);
+#else
     const float c = smin(smax(q, lo), hi);
+#endif
     return fbits((entry_axis ? lo : c) + kBias) - kBiasBits;
 }
 
