@@ -79,28 +79,32 @@ def build(verbose=False):
     _run([HIPCC, "-shared", "--offload-arch=gfx950", "-o", tmp] + objs +
          ["-pthread", "-L/opt/rocm/lib", "-lrocprofiler-sdk-roctx", "-Wl,-rpath,/opt/rocm/lib"], verbose)
     os.replace(tmp, LIB)
-    build_cpp_checks(verbose)
     return LIB
 
 
-def build_cpp_checks(verbose=False):
+def build_cpp_checks(verbose=False, strict=True):
     """Test programs: the C++ drop-in example run by the GPU tests (links libcqx.so through its
-    rpath) and the host compilation of the device traversal core used by the CPU tests."""
+    rpath) and the host compilations of the device traversal cores used by the CPU tests. Not part of
+    build(): the library does not depend on them. With strict False a program that does not compile is
+    reported and left out, so that no test program fails the caller's build; the tests that run it then do."""
     cpp = os.path.join(ROOT, "tests", "cpp")
-    src = os.path.join(cpp, "dropin_check.cpp")
-    if not os.path.exists(src):
-        return None
-    out = os.path.join(cpp, "dropin_check")
-    _run([CXX, "-std=c++17", "-O2", f"-I{INCLUDE}", src, "-o", out, f"-L{HERE}", "-lcqx",
-          "-Wl,-rpath,$ORIGIN/../../cubiquity_amd"], verbose)
-    for name in ("core_emulation", "packed_emulation"):
-        emu = os.path.join(cpp, name + ".cpp")
-        if os.path.exists(emu):
-            _run([CXX, "-std=c++17", "-O2", "-ffp-contract=off", "-fno-fast-math",
-                  f"-I{os.path.join(cpp, 'host_shim')}", f"-I{INCLUDE}", f"-I{CSRC}", emu, "-o",
-                  os.path.join(cpp, name)], verbose)
-    return out
+    emulation = ["-ffp-contract=off", "-fno-fast-math", f"-I{os.path.join(cpp, 'host_shim')}", f"-I{INCLUDE}", f"-I{CSRC}"]
+    programs = {"dropin_check": [f"-I{INCLUDE}", f"-L{HERE}", "-lcqx", "-Wl,-rpath,$ORIGIN/../../cubiquity_amd"],
+                "core_emulation": emulation, "packed_emulation": emulation}
+    for name, flags in programs.items():
+        src, out = os.path.join(cpp, name + ".cpp"), os.path.join(cpp, name)
+        if os.path.exists(out):
+            os.remove(out)  # a test never runs the program of an older source
+        if not os.path.exists(src):
+            continue
+        try:
+            _run([CXX, "-std=c++17", "-O2", src, "-o", out] + flags, verbose)
+        except (RuntimeError, OSError) as e:
+            if strict:
+                raise
+            print(f"test program {name} not built: {e}", file=sys.stderr, flush=True)
 
 
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
+    build_cpp_checks(verbose="-v" in sys.argv, strict=False)

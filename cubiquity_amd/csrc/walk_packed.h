@@ -124,8 +124,26 @@ struct PackedRay {
     uint32_t plain;   // ray_plain()
 };
 
-__device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); }
-__device__ __forceinline__ float bitsf(uint32_t u) { return __uint_as_float(u); }
+__device__ __forceinline__ uint32_t fbits(float f)
+{
+#if defined(__AMDGCN__)
+    return __float_as_uint(f);
+#else
+    uint32_t u;
+    std::memcpy(&u, &f, 4);
+    return u;
+#endif
+}
+__device__ __forceinline__ float bitsf(uint32_t u)
+{
+#if defined(__AMDGCN__)
+    return __uint_as_float(u);
+#else
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+#endif
+}
 
 // Minimum and maximum of values that are neither NaN nor -0, in one instruction.
 __device__ __forceinline__ float plain_min3(float a, float b, float c)
