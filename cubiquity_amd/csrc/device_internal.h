@@ -96,17 +96,6 @@ cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
 // fits. A copy that cannot be allocated is left out.
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);
 
-// The packed word of a child: its index and the occupancy mask of its node.
-__device__ __forceinline__ uint32_t pack_child(const uint32_t* __restrict__ nodes, uint32_t child)
-{
-    if (child == 0) return 0u;
-    const uint4* q = reinterpret_cast<const uint4*>(nodes) + uint64_t(child) * 2;
-    const uint4 a = q[0], b = q[1];
-    const uint32_t mask = (a.x ? 1u : 0u) | (a.y ? 2u : 0u) | (a.z ? 4u : 0u) | (a.w ? 8u : 0u) | (b.x ? 16u : 0u) |
-                          (b.y ? 32u : 0u) | (b.z ? 64u : 0u) | (b.w ? 128u : 0u);
-    return cqxd::packed_word(child, mask);
-}
-
 // Rays per wave of a one-ray-per-lane launch of n rays (at most 64).
 uint32_t lanes_per_wave(uint64_t n);
 

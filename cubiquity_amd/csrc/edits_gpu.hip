@@ -1220,7 +1220,7 @@ __global__ void __launch_bounds__(64) k_find_subdags(const uint32_t* __restrict_
         s.lower[2] = int32_t(lower[2]);
         s.height = height;
         s.node = node;
-        s.pad0 = cqx::pack_child(nodes, node);
+        s.pad0 = cqxd::pack_child(nodes, kEmptySlot, node); // a node of the store: reached from its root
     }
     const uint64_t occupied = __ballot(c < 8 && s.node > 0), failed = __ballot(deep);
     s.pad1 = uint32_t(occupied);

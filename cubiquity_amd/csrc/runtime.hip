@@ -437,18 +437,19 @@ __global__ void __launch_bounds__(64) k_sample_rays(unsigned long long* counters
 // Packed words of store words [first, first + count): each child's index and the occupancy mask of
 // its node. One thread per word; the mask is one 32-byte read of the child's node.
 __global__ void __launch_bounds__(256) k_pack_nodes(const uint32_t* __restrict__ nodes, uint32_t* __restrict__ packed,
-                                                    uint64_t first, uint64_t count)
+                                                    uint64_t first, uint64_t count, uint64_t node_count)
 {
     const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < count) packed[first + i] = cqx::pack_child(nodes, nodes[first + i]);
+    if (i < count) packed[first + i] = pack_child(nodes, node_count, nodes[first + i]);
 }
 
-__global__ void __launch_bounds__(64) k_pack_subdags(const uint32_t* __restrict__ nodes, cqx_subdag* __restrict__ sub)
+__global__ void __launch_bounds__(64) k_pack_subdags(const uint32_t* __restrict__ nodes, uint64_t node_count,
+                                                     cqx_subdag* __restrict__ sub)
 {
     const uint32_t node = threadIdx.x < 8 ? sub[threadIdx.x].node : 0u;
     const uint32_t occ = uint32_t(__ballot(node > 0));
     if (threadIdx.x >= 8) return;
-    sub[threadIdx.x].pad0 = cqx::pack_child(nodes, node);
+    sub[threadIdx.x].pad0 = pack_child(nodes, node_count, node);
     sub[threadIdx.x].pad1 = occ;
 }
 
@@ -876,7 +877,7 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
         const uint64_t words = (vol->node_count - first) * 8;
         if (words)
             hipLaunchKernelGGL(k_pack_nodes, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, 0, vol->nodes, vol->packed,
-                               first * 8, words);
+                               first * 8, words, vol->node_count);
         HIP_TRY(hipGetLastError());
     }
     vol->packed_ok = vol->packed && packed_eligible(vol->node_count, vol->hsub);
@@ -1324,7 +1325,7 @@ cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nod
         HIP_TRY(hipMemcpy(vol->nodes + first * 8, nodes + first * 8, size_t(node_count - first) * 32,
                           hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(vol->sub, s, sizeof(s), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_pack_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, vol->sub);
+    hipLaunchKernelGGL(k_pack_subdags, dim3(1), dim3(64), 0, 0, vol->nodes, node_count, vol->sub);
     const uint64_t kOffset32Nodes = uint64_t(1) << 27; // the child-offset width the traversal uses
     if (ctx->pt_plan && (old_nodes != vol->nodes || max_height != vol->max_height ||
                          (vol->node_count <= kOffset32Nodes) != (node_count <= kOffset32Nodes))) {

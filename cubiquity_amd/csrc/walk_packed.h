@@ -64,6 +64,18 @@ struct PackedParams {
 // Word for a child with index `index` whose occupancy mask is `mask` (0 for an empty child).
 __host__ __device__ inline uint32_t packed_word(uint32_t index, uint32_t mask) { return index ? (index << 8) | mask : 0u; }
 
+// The packed word of a child: its index and the occupancy mask of its node. Nodes that no root reaches are
+// packed too, and their words are unchecked: one past the store's `node_count` nodes is packed as empty.
+__device__ __forceinline__ uint32_t pack_child(const uint32_t* __restrict__ nodes, uint64_t node_count, uint32_t child)
+{
+    if (child == 0 || child >= node_count) return 0u;
+    const uint4* q = reinterpret_cast<const uint4*>(nodes) + uint64_t(child) * 2;
+    const uint4 a = q[0], b = q[1];
+    const uint32_t mask = (a.x ? 1u : 0u) | (a.y ? 2u : 0u) | (a.z ? 4u : 0u) | (a.w ? 8u : 0u) | (b.x ? 16u : 0u) |
+                          (b.y ? 32u : 0u) | (b.z ? 64u : 0u) | (b.w ? 128u : 0u);
+    return packed_word(child, mask);
+}
+
 // The footprint test size / t > F (one correctly rounded division; size a power of two) as thresholds
 // on t / size, which is exact: with u = t / size, RN(1 / u) > F holds for 0 <= u <= hi and for
 // u <= lo < 0 (RN(1 / u) is monotonic on either side of 0). hi = infinity: for every u >= 0.
