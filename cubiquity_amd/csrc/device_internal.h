@@ -64,6 +64,7 @@ struct cqx_dvolume {
     cqx_subdag* sub = nullptr;
     uint64_t node_count = 0;
     uint64_t capacity = 0; // nodes the device buffer holds (headroom for appended edits)
+    uint64_t uploaded = 0; // nodes of the upload: these may have later ones as children, appended ones may not
     // The packed copy of the store (walk_packed.h): present for stores of at most 2^24 nodes, used
     // when packed_ok (the SubDAGs lie within its coordinate limit).
     uint32_t* packed = nullptr;
@@ -93,7 +94,9 @@ struct ScratchView {
 cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
 // Brings the packed copy up to date after nodes [first, node_count), the SubDAGs or the buffers
 // changed (work queued on the null stream), and drops the path tracer's plan if its graph no longer
-// fits. A copy that cannot be allocated is left out.
+// fits. A copy that cannot be allocated is left out. Words hold their children's masks: where the change
+// reaches into the upload, whose nodes may have changed ones as children, all are made anew, and a
+// store cut short of its upload is walked raw.
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);
 
 // Rays per wave of a one-ray-per-lane launch of n rays (at most 64).

@@ -873,6 +873,7 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
             (void)hipGetLastError();
         }
     }
+    if (first < vol->uploaded) first = 0;
     if (vol->packed) {
         const uint64_t words = (vol->node_count - first) * 8;
         if (words)
@@ -880,7 +881,7 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
                                first * 8, words, vol->node_count);
         HIP_TRY(hipGetLastError());
     }
-    vol->packed_ok = vol->packed && packed_eligible(vol->node_count, vol->hsub);
+    vol->packed_ok = vol->packed && vol->node_count >= vol->uploaded && packed_eligible(vol->node_count, vol->hsub);
     if (ctx->pt_plan && (vol->packed != old || vol->packed_ok != old_ok)) {
         HIP_TRY(hipDeviceSynchronize());
         destroy_pt_plan(ctx->pt_plan); // its captured graph holds the old copy or the other walk
@@ -1244,6 +1245,7 @@ cqx_status cqx_volume_upload(cqx_ctx* ctx, const uint32_t* nodes, uint64_t node_
     if (!v) return fail(CQX_ERR_OOM, "out of host memory");
     v->node_count = node_count;
     v->capacity = node_count;
+    v->uploaded = node_count;
     v->root = root;
     std::memcpy(v->hsub, s, sizeof(s));
     v->max_height = 0;

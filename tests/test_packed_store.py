@@ -45,3 +45,44 @@ def test_gpu_store_with_unreached_nodes(cq, oracle, gpu_ctx, vol128, rays128):
     got = cq.intersectVolume(gpu_ctx, dv, rays).cpu().numpy().view(cq.HIT_DTYPE).reshape(-1)
     assert records_equal(got, ref).all()
     dv.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("keep", [0.02, 0.5, 0.9])
+def test_gpu_update_that_replaces_uploaded_nodes(cq, oracle, gpu_ctx, vol128, rays128, keep):
+    """An update may replace the tail of the uploaded store, whose earlier nodes have children there
+    (a baked store holds parents first): the masks kept with those nodes' words follow. Then the store is
+    cut short of its upload, and extended again."""
+    import torch
+
+    nodes, n = vol128.nodes.copy(), len(vol128.nodes)
+    first = 256 + int(keep * (n - 256))
+    assert (nodes[256:first] >= first).any() and vol128.root < first
+    dv = gpu_ctx.upload(vol128)
+    rays = torch.from_numpy(rays128["incoherent"]).cuda()
+
+    def check(stored):
+        ref = oracle.intersect(stored, oracle.find_subdags(stored, vol128.root), rays128["incoherent"], True, threads=8)
+        got = cq.intersectVolume(gpu_ctx, dv, rays).cpu().numpy().view(cq.HIT_DTYPE).reshape(-1)
+        eq = records_equal(got, ref)
+        assert eq.all(), int((~eq).sum())
+
+    check(nodes)
+    rng = np.random.Generator(np.random.PCG64(int(100 * keep)))
+    fresh = rng.integers(1, 256, (n - first, 8)).astype(np.uint32)  # materials: any node may have them as children
+    fresh[rng.random(fresh.shape) < 0.6] = 0
+    fresh[:, 0] = np.maximum(fresh[:, 0], 1)
+    nodes[first:] = fresh
+    dv.update(cq.HostVolume.from_nodes(nodes, vol128.root), first)
+    check(nodes)
+    tail = nodes[first:].copy()
+    tail[:, 3] = 7
+    nodes[first:] = tail
+    nodes = np.concatenate([nodes, tail[:50]])
+    dv.update(cq.HostVolume.from_nodes(nodes, vol128.root), first)
+    check(nodes)
+    dv.update(cq.HostVolume.from_nodes(nodes[:first], 3), first)  # the whole space material 3
+    assert (cq.intersectVolume(gpu_ctx, dv, rays).cpu().numpy().view(cq.HIT_DTYPE)["info"] >> 16 == 3).all()
+    dv.update(cq.HostVolume.from_nodes(nodes, vol128.root), first)
+    check(nodes)
+    dv.free()
