@@ -93,8 +93,9 @@ struct ScratchView {
 // Grows the context's staging buffer (host-buffer entry points) to at least `bytes`.
 cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
 // Brings the packed copy up to date after nodes [first, node_count), the SubDAGs or the buffers
-// changed (work queued on the null stream), and drops the path tracer's plan if its graph no longer
-// fits. A copy that cannot be allocated is left out. Words hold their children's masks: where the change
+// changed, waiting for what it packs (a copy that could not be had before may be packed whole, whatever
+// `first` says, and launches on any stream read it), and drops the path tracer's plan if its graph no
+// longer fits. A copy that cannot be allocated is left out. Words hold their children's masks: where the change
 // reaches into the upload, whose nodes may have changed ones as children, all are made anew, and a
 // store cut short of its upload is walked raw.
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);

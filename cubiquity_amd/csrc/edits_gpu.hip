@@ -1469,10 +1469,7 @@ cqx_status set_root(cqx_ctx* ctx, cqx_dvolume* vol, uint32_t root, uint64_t firs
     vol->root = root;
     std::memcpy(vol->hsub, rep.sub, sizeof(rep.sub));
     vol->max_height = max_height;
-    const cqx_status st = cqx::refresh_packed(ctx, vol, first_new);
-    if (st != CQX_OK) return st;
-    if (first_new < vol->node_count) HIP_TRY(hipStreamSynchronize(nullptr));
-    return CQX_OK;
+    return cqx::refresh_packed(ctx, vol, first_new);
 }
 
 // Makes `root`, a node of the store, the volume's root.

@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -852,7 +853,10 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
 {
     uint32_t* const old = vol->packed;
     const bool old_ok = vol->packed_ok;
-    if (vol->node_count > kPackedNodes) {
+    // CQX_PACKED_NODES=<nodes>: stores of more nodes keep no packed copy (the tests use it for a copy that
+    // cannot be had).
+    const char* const most = std::getenv("CQX_PACKED_NODES");
+    if (vol->node_count > (most ? std::min<uint64_t>(std::strtoull(most, nullptr, 10), kPackedNodes) : kPackedNodes)) {
         if (old) {
             HIP_TRY(hipDeviceSynchronize()); // launches in flight may read it
             release(old);
@@ -880,6 +884,7 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
             hipLaunchKernelGGL(k_pack_nodes, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, 0, vol->nodes, vol->packed,
                                first * 8, words, vol->node_count);
         HIP_TRY(hipGetLastError());
+        if (words) HIP_TRY(hipStreamSynchronize(nullptr));
     }
     vol->packed_ok = vol->packed && vol->node_count >= vol->uploaded && packed_eligible(vol->node_count, vol->hsub);
     if (ctx->pt_plan && (vol->packed != old || vol->packed_ok != old_ok)) {
@@ -1261,7 +1266,6 @@ cqx_status cqx_volume_upload(cqx_ctx* ctx, const uint32_t* nodes, uint64_t node_
     device_subdags(nodes, s, ds);
     st = hipMemcpy(v->nodes, nodes, bytes, hipMemcpyHostToDevice) == hipSuccess ? cqx::refresh_packed(ctx, v, 0)
                                                                               : fail(CQX_ERR_HIP, "upload of the node store failed");
-    // (the copy is queued behind the packing: both are done when it returns)
     if (st == CQX_OK && (hipMemcpy(v->sub, ds, sizeof(ds), hipMemcpyHostToDevice) != hipSuccess ||
                          hipStreamSynchronize(nullptr) != hipSuccess))
         st = fail(CQX_ERR_HIP, "upload of the SubDAGs failed");

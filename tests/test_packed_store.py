@@ -86,3 +86,35 @@ def test_gpu_update_that_replaces_uploaded_nodes(cq, oracle, gpu_ctx, vol128, ra
     dv.update(cq.HostVolume.from_nodes(nodes, vol128.root), first)
     check(nodes)
     dv.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("back", ["undo", "redo", "update", "edit"])
+def test_gpu_copy_that_returns_is_whole(cq, oracle, gpu_ctx, rays128, monkeypatch, back):
+    """A copy that cannot be had is left out, and made whole by whichever later call can have it: what
+    other streams launch right after that call reads no word still to be packed."""
+    import torch
+
+    hv = cq.HostVolume.generate(cq.gen_default_params(9, 3))
+    rays = cq.incoherent_rays(hv, 9, 11, 20000)
+    side = torch.cuda.Stream()  # does not wait for the null stream
+    r, hits = torch.from_numpy(rays).cuda(), torch.zeros((len(rays), 32), dtype=torch.uint8, device="cuda")
+    spheres = [[20.0 * i, 250.0, 9.0 * i, 6.0, 1 + i % 5] for i in range(20)]
+    monkeypatch.setenv("CQX_PACKED_NODES", "0")
+    dv = gpu_ctx.upload(hv)
+    dv.checkpoint()
+    dv.edit_spheres(spheres)
+    if back == "redo":
+        dv.undo()
+    elif back == "update":
+        hv = cq.HostVolume.from_nodes(dv.download(), dv.root)
+    torch.cuda.synchronize()
+    monkeypatch.delenv("CQX_PACKED_NODES")
+    {"undo": dv.undo, "redo": dv.redo, "update": lambda: dv.update(hv, dv.node_count),
+     "edit": lambda: dv.edit_spheres(spheres)}[back]()
+    cq.intersectVolume(gpu_ctx, dv, r, out=hits, stream=side.cuda_stream)
+    side.synchronize()
+    nodes = dv.download()
+    ref = oracle.intersect(nodes, oracle.find_subdags(nodes, dv.root), rays, True, threads=8)
+    assert records_equal(hits.cpu().numpy().view(cq.HIT_DTYPE).reshape(-1), ref).all()
+    dv.free()
