@@ -69,6 +69,7 @@ struct cqx_dvolume {
     // when packed_ok (the SubDAGs lie within its coordinate limit).
     uint32_t* packed = nullptr;
     uint64_t packed_capacity = 0;
+    uint64_t packed_count = 0; // nodes [0, packed_count) of the copy are as the store's
     bool packed_ok = false;
     uint32_t root = 0;
     cqx_subdag hsub[8];

@@ -851,48 +851,51 @@ cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes)
 
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
 {
-    uint32_t* const old = vol->packed;
     const bool old_ok = vol->packed_ok;
+    vol->packed_ok = false; // whatever ends this early: no walk over a copy that is not in step
+    const auto drop_plan = [&]() -> cqx_status { // its captured graph holds the copy, or the other walk
+        if (!ctx->pt_plan) return CQX_OK;
+        HIP_TRY(hipDeviceSynchronize());
+        destroy_pt_plan(ctx->pt_plan);
+        ctx->pt_plan = nullptr;
+        return CQX_OK;
+    };
     // CQX_PACKED_NODES=<nodes>: stores of more nodes keep no packed copy (the tests use it for a copy that
     // cannot be had).
-    const char* const most = std::getenv("CQX_PACKED_NODES");
-    if (vol->node_count > (most ? std::min<uint64_t>(std::strtoull(most, nullptr, 10), kPackedNodes) : kPackedNodes)) {
-        if (old) {
-            HIP_TRY(hipDeviceSynchronize()); // launches in flight may read it
-            release(old);
-            vol->packed = nullptr;
-            vol->packed_capacity = 0;
-        }
-    } else if (vol->node_count > vol->packed_capacity) {
-        const uint64_t cap = std::min<uint64_t>(std::max(vol->capacity, vol->node_count), kPackedNodes);
-        HIP_TRY(hipDeviceSynchronize());
-        release(old);
+    const char* const env = std::getenv("CQX_PACKED_NODES");
+    const uint64_t most = env ? std::min<uint64_t>(std::strtoull(env, nullptr, 10), kPackedNodes) : kPackedNodes;
+    if (vol->packed && (vol->node_count > most || vol->node_count > vol->packed_capacity)) {
+        const cqx_status st = drop_plan();
+        if (st != CQX_OK) return st;
+        HIP_TRY(hipDeviceSynchronize()); // launches in flight may read it
+        release(vol->packed);
         vol->packed = nullptr;
-        vol->packed_capacity = 0;
+        vol->packed_capacity = vol->packed_count = 0;
+    }
+    if (!vol->packed && vol->node_count <= most) {
+        const uint64_t cap = std::min<uint64_t>(std::max(vol->capacity, vol->node_count), kPackedNodes);
         if (hipMalloc(&vol->packed, size_t(cap) * 32) == hipSuccess) {
             vol->packed_capacity = cap;
-            first = 0;
         } else {
             vol->packed = nullptr; // traversal then runs on the raw store
             (void)hipGetLastError();
         }
     }
-    if (first < vol->uploaded) first = 0;
     if (vol->packed) {
+        // (an error return after the store grew may have left nodes before `first` unpacked)
+        first = first < vol->uploaded ? 0 : std::min(first, vol->packed_count);
+        vol->packed_count = first;
         const uint64_t words = (vol->node_count - first) * 8;
-        if (words)
+        if (words) {
             hipLaunchKernelGGL(k_pack_nodes, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, 0, vol->nodes, vol->packed,
                                first * 8, words, vol->node_count);
-        HIP_TRY(hipGetLastError());
-        if (words) HIP_TRY(hipStreamSynchronize(nullptr));
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipStreamSynchronize(nullptr));
+        }
+        vol->packed_count = vol->node_count;
     }
     vol->packed_ok = vol->packed && vol->node_count >= vol->uploaded && packed_eligible(vol->node_count, vol->hsub);
-    if (ctx->pt_plan && (vol->packed != old || vol->packed_ok != old_ok)) {
-        HIP_TRY(hipDeviceSynchronize());
-        destroy_pt_plan(ctx->pt_plan); // its captured graph holds the old copy or the other walk
-        ctx->pt_plan = nullptr;
-    }
-    return CQX_OK;
+    return vol->packed_ok == old_ok ? CQX_OK : drop_plan();
 }
 
 // The shape of an open launch on a packed volume, by its size. What each line rests on (MI355X, us,

@@ -118,3 +118,43 @@ def test_gpu_copy_that_returns_is_whole(cq, oracle, gpu_ctx, rays128, monkeypatc
     ref = oracle.intersect(nodes, oracle.find_subdags(nodes, dv.root), rays, True, threads=8)
     assert records_equal(hits.cpu().numpy().view(cq.HIT_DTYPE).reshape(-1), ref).all()
     dv.free()
+
+
+@pytest.mark.gpu
+def test_gpu_copy_after_an_edit_that_fails_late(cq, oracle, gpu_ctx, vol128, rays128):
+    """An edit of a store whose root is on a chain deeper than the tree (accepted by an update that
+    brings its SubDAGs) fails once its nodes are in the store and the index. Later edits share those
+    nodes: the copy has them."""
+    import ctypes
+
+    import torch
+
+    nodes = vol128.nodes
+    n, chain = len(nodes), np.zeros((40, 8), np.uint32)
+    chain[0, 0] = 9
+    chain[1:, 0] = np.arange(n, n + 39)  # the octant of the lowest coordinates, far from the edits
+    deep = np.ascontiguousarray(np.concatenate([nodes, chain]))
+    sub = np.ascontiguousarray(oracle.find_subdags(nodes, vol128.root))
+    dv = gpu_ctx.upload(vol128)
+    cq.cabi.check(cq.cabi.lib().cqx_volume_update(
+        gpu_ctx._h, dv._h, deep.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), ctypes.c_uint64(len(deep)),
+        ctypes.c_uint64(n), ctypes.c_uint32(len(deep) - 1), sub.ctypes.data_as(ctypes.c_void_p)))
+    spheres = [[300.0 + 3 * i, 300.0 + i, 300.0, 3.0, 3] for i in range(16)]  # in empty space under either root
+    with pytest.raises(cq.CqxError):
+        dv.edit_spheres(spheres)
+    dv._refresh()
+    held = dv.node_count
+    assert held > len(deep)
+    dv.update(cq.HostVolume.from_nodes(dv.download(), vol128.root), held)
+    rays = rays128["incoherent"].copy()
+    aim = np.array(spheres, np.float32)[np.arange(8000) % 16, :3] - rays[:8000, :3]
+    rays[:8000, 3:] = aim / np.linalg.norm(aim, axis=1, keepdims=True)
+    r = torch.from_numpy(rays).cuda()
+    for hit in (False, True):
+        stored = dv.download()
+        ref = oracle.intersect(stored, oracle.find_subdags(stored, dv.root), rays, True, threads=8)
+        got = cq.intersectVolume(gpu_ctx, dv, r).cpu().numpy().view(cq.HIT_DTYPE).reshape(-1)
+        assert records_equal(got, ref).all() and (got["voxel"][:8000, 0] > 290).any() == hit
+        dv.edit_spheres(spheres)
+        assert ((dv.download(held) >= len(deep)) & (dv.download(held) < held)).any()
+    dv.free()
