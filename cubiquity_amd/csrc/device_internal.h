@@ -21,6 +21,7 @@ namespace cqx {
 
 struct PtPlan; // path-tracer buffers and captured graph (pathtrace.hip)
 void destroy_pt_plan(PtPlan* plan);
+bool plan_holds(const PtPlan* plan, const cqx_dvolume* vol); // whether the plan's graphs walk this volume
 struct DemoPlan; // buffers of the reference-shading mode (demo.hip)
 void destroy_demo_plan(DemoPlan* plan);
 struct DeviceEdits; // a volume's on-device edit state (edits_gpu.hip)
@@ -95,10 +96,10 @@ struct ScratchView {
 cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
 // Brings the packed copy up to date after nodes [first, node_count), the SubDAGs or the buffers
 // changed, waiting for what it packs (a copy that could not be had before may be packed whole, whatever
-// `first` says, and launches on any stream read it), and drops the path tracer's plan if its graph no
-// longer fits. A copy that cannot be allocated is left out. Words hold their children's masks: where the change
-// reaches into the upload, whose nodes may have changed ones as children, all are made anew, and a
-// store cut short of its upload is walked raw.
+// `first` says, and launches on any stream read it), and drops the path tracer's plan if it is this
+// volume's and its graph no longer fits. A copy that cannot be allocated is left out. Words hold their
+// children's masks: where the change reaches into the upload, whose nodes may have changed ones as
+// children, all are made anew, and a store cut short of its upload is walked raw.
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);
 
 // Rays per wave of a one-ray-per-lane launch of n rays (at most 64).

@@ -856,6 +856,8 @@ struct PtPlan {
     hipGraphExec_t exec_replay = nullptr;
 };
 
+bool plan_holds(const PtPlan* p, const cqx_dvolume* vol) { return p && p->vol == vol; }
+
 void destroy_pt_plan(PtPlan* p)
 {
     if (!p) return;

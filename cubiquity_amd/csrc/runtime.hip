@@ -854,7 +854,7 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
     const bool old_ok = vol->packed_ok;
     vol->packed_ok = false; // whatever ends this early: no walk over a copy that is not in step
     const auto drop_plan = [&]() -> cqx_status { // its captured graph holds the copy, or the other walk
-        if (!ctx->pt_plan) return CQX_OK;
+        if (!plan_holds(ctx->pt_plan, vol)) return CQX_OK;
         HIP_TRY(hipDeviceSynchronize());
         destroy_pt_plan(ctx->pt_plan);
         ctx->pt_plan = nullptr;

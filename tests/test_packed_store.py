@@ -158,3 +158,22 @@ def test_gpu_copy_after_an_edit_that_fails_late(cq, oracle, gpu_ctx, vol128, ray
         dv.edit_spheres(spheres)
         assert ((dv.download(held) >= len(deep)) & (dv.download(held) < held)).any()
     dv.free()
+
+
+@pytest.mark.gpu
+def test_gpu_upload_keeps_the_path_tracers_plan(cq, gpu_ctx, vol128):
+    """Uploading one volume while another is rendered: the renderer's plan (buffers and graph, a third of a
+    gigabyte here) is not made again for the next frame."""
+    import torch
+
+    from cubiquity_amd import workloads as W
+
+    dv = gpu_ctx.upload(vol128)
+    setup = cq.PathTraceSetup(W.RAYCAST_128.camera, 640, 480, 8, 2, *cq.material_table(9, 11))
+    image = cq.pathtrace(gpu_ctx, dv, setup)
+    free = torch.cuda.mem_get_info()[0]
+    other = gpu_ctx.upload(cq.HostVolume.from_dense(np.ones((4, 4, 4), np.uint8)))
+    assert torch.cuda.mem_get_info()[0] <= free
+    assert torch.equal(cq.pathtrace(gpu_ctx, dv, setup), image)
+    other.free()
+    dv.free()
