@@ -192,7 +192,7 @@ __device__ __forceinline__ float at_least_denorm(float x)
 // 1 / d correctly rounded for d in [1e-18, 1e18] (a normal result): the hardware's reciprocal (within
 // 1 ulp) and two Newton corrections by fused multiply-adds, the last one Markstein's correctly
 // rounding step; 24 issue cycles against 38 for the general division's scaling and fix-up. Equal to
-// the division for every float of that range (all 1.0e9 compared on the GPU).
+// the division for every float of that range (test_plain_reciprocal.py compares all 1.0e9 on the GPU).
 __device__ __forceinline__ float plain_rcp(float d)
 {
 #if defined(__AMDGCN__)

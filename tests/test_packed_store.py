@@ -177,3 +177,52 @@ def test_gpu_upload_keeps_the_path_tracers_plan(cq, gpu_ctx, vol128):
     assert torch.equal(cq.pathtrace(gpu_ctx, dv, setup), image)
     other.free()
     dv.free()
+
+
+@pytest.mark.gpu
+def test_gpu_path_tracer_follows_the_copy(cq, gpu_ctx, monkeypatch):
+    """One image shape rendered, and its adjoint taken, while the volume's copy grows, is given up past the
+    coordinate limit, cannot be had, and returns: each frame equals the megakernel's (which walks the raw
+    store), each gradient that of a fresh context."""
+    import torch
+
+    from cubiquity_amd import workloads as W
+
+    cam = W.Camera((60.0, 90.0, -120.0), (150.0, 0.0, 40.0), 70.0, 96, 64)
+    setup = cq.PathTraceSetup(cam, 96, 64, 4, 3, *cq.material_table(5, 11))
+    d_image = torch.rand((64, 96, 3), device="cuda")
+    hv = cq.HostVolume.from_dense(np.ones((4, 4, 4), np.uint8), (0, 0, 0))
+    dv = gpu_ctx.upload(hv)
+    near = [[20.0 * i, 3.0, 5.0 * i, 8.0, 1 + i % 5] for i in range(16)]
+
+    def check():
+        image = cq.pathtrace(gpu_ctx, dv, setup)
+        got = cq.pathtrace_adjoint(gpu_ctx, dv, setup, d_image)
+        assert torch.equal(image, cq.pathtrace(gpu_ctx, dv, setup, mode=1))
+        ctx = cq.Context(0)
+        fresh = ctx.upload(cq.HostVolume.from_nodes(dv.download(), dv.root))
+        ref = cq.pathtrace_adjoint(ctx, fresh, setup, d_image)
+        fresh.free()
+        ctx.close()
+        assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+        return image
+
+    images = [check()]
+    dv.edit_spheres(near)  # grows the store past its copy
+    images.append(check())
+    dv.checkpoint()
+    dv.edit_spheres([[float(1 << 22) + 50.0, 3.0, 3.0, 4.0, 2]] + near[1:])
+    check()
+    monkeypatch.setenv("CQX_PACKED_NODES", "0")
+    dv.undo()
+    images.append(check())
+    monkeypatch.delenv("CQX_PACKED_NODES")
+    dv.redo()
+    dv.undo()
+    images.append(check())
+    grown = [[20.0 * i, 40.0, 4.0 * i, 5.0 + 0.1 * i, 1 + i % 5] for i in range(40)]
+    dv.edit_spheres(grown)
+    images.append(check())
+    assert torch.equal(images[1], images[2]) and torch.equal(images[1], images[3])
+    assert not torch.equal(images[0], images[1]) and not torch.equal(images[1], images[4])
+    dv.free()
