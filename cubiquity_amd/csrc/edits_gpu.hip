@@ -356,10 +356,9 @@ __device__ bool intern_one(Region& R, uint32_t out, uint32_t lane, uint32_t& res
 
 // The children of a node (lower corner lo, children of side `side`) against the brush, as masks over
 // the children: those to be filled and those to be walked. False when no child's float box overlaps
-// the brush bounds (geometry.h:346-357): the node stays. `corner`: contains() at corner k of child c.
+// the brush bounds (geometry.h:346-357): the node stays.
 __device__ __forceinline__ bool test_children(const Brush& b, uint32_t mat, uint32_t child, uint32_t side, int32_t lx,
-                                              int32_t ly, int32_t lz, uint32_t lane, uint32_t& fill, uint32_t& walk,
-                                              bool& corner)
+                                              int32_t ly, int32_t lz, uint32_t lane, uint32_t& fill, uint32_t& walk)
 {
     const uint32_t c = lane >> 3, k = lane & 7u;
     const int32_t x0 = int32_t(uint32_t(lx) + side * (c & 1u)), y0 = int32_t(uint32_t(ly) + side * ((c >> 1) & 1u)),
@@ -372,7 +371,7 @@ __device__ __forceinline__ bool test_children(const Brush& b, uint32_t mat, uint
     fill = walk = 0;
     const uint64_t okb = __ballot(ok);
     if (okb == 0) return false;
-    corner = b.contains((k & 1u) ? fx1 : fx0, (k & 2u) ? fy1 : fy0, (k & 4u) ? fz1 : fz0);
+    const bool corner = b.contains((k & 1u) ? fx1 : fx0, (k & 2u) ? fy1 : fy0, (k & 4u) ? fz1 : fz0);
     const uint32_t all = bytes_all(__ballot(corner));
     const uint32_t live = byte_bits(__ballot(ok && child != mat));
     fill = live & all;
@@ -495,9 +494,8 @@ __device__ bool fill(Region& R, const Brush& b, uint32_t mat, uint32_t node, uin
 {
     const uint32_t c = lane >> 3, k = lane & 7u;
     uint32_t out = R.child(node, c), walk, set, kid = 0, changed;
-    bool corner;
     result = node;
-    if (!test_children(b, mat, out, 1u << (height - 1), lx, ly, lz, lane, set, walk, corner)) return true;
+    if (!test_children(b, mat, out, 1u << (height - 1), lx, ly, lz, lane, set, walk)) return true;
     uint32_t sp = 0;
     const auto enter = [&] { // the node's children tested: what is filled, and the next level's reads
         changed = set ? 1u : 0u;
@@ -542,7 +540,7 @@ __device__ bool fill(Region& R, const Brush& b, uint32_t mat, uint32_t node, uin
         const int32_t cx = int32_t(uint32_t(lx) + side * (at & 1u)), cy = int32_t(uint32_t(ly) + side * ((at >> 1) & 1u)),
                       cz = int32_t(uint32_t(lz) + side * (at >> 2));
         uint32_t cset, cwalk;
-        if (!test_children(b, mat, grand, side >> 1, cx, cy, cz, lane, cset, cwalk, corner)) continue;
+        if (!test_children(b, mat, grand, side >> 1, cx, cy, cz, lane, cset, cwalk)) continue;
         Frame& f = st[sp++];
         f.kid[lane] = kid;
         if (k == 0) f.out[c] = out;

@@ -151,8 +151,7 @@ __device__ __forceinline__ void result_miss(cqx_hit& out)
 }
 
 // Ray setup, raytracing.cpp:415-434.
-template <typename Ray>
-__device__ __forceinline__ void ray_setup(Ray& S, float rox, float roy, float roz, float rdx, float rdy, float rdz)
+__device__ __forceinline__ void ray_setup(RayState& S, float rox, float roy, float roz, float rdx, float rdy, float rdz)
 {
     const uint32_t sbx = rdx < 0.0f, sby = rdy < 0.0f, sbz = rdz < 0.0f;
     S.sign_bits = sbx | (sby << 1) | (sbz << 2);

@@ -99,7 +99,7 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 //   kSampled        dealt, one ray per lane, where the sampled flag at `gate` is set (k_sample_rays), and
 //                   otherwise claimed by the first `want` workgroups; the rest end at once, in the slots
 //                   that those leave free (as a launch of its own they took 17 us of 1.87 ms at 2^24 rays)
-// With `gate`, kDealt and kClaimed launches run only when the flag equals `want`.
+// With `gate`, a kDealt launch runs only when the flag equals `want`.
 // At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take 72 and 7 waves (24 volumes
 // 193 us with 6 waves, 189 with 7, 194 with 8 and 8 to 13 registers spilled).
 enum WalkForm { kClaimed, kDealt, kSampled };
@@ -116,7 +116,7 @@ k_walk(Source src, uint64_t n, const uint32_t* __restrict__ n_dev, unsigned long
         dealt = *gate != 0;
         if (dealt) refill = chunk = 64u;
         else if (blockIdx.x >= want) return;
-    } else {
+    } else if constexpr (kForm == kDealt) {
         if (gate && *gate != want) return;
     }
     if (n_dev) {
