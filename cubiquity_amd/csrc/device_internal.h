@@ -26,6 +26,7 @@ struct DemoPlan; // buffers of the reference-shading mode (demo.hip)
 void destroy_demo_plan(DemoPlan* plan);
 struct DeviceEdits; // a volume's on-device edit state (edits_gpu.hip)
 void destroy_device_edits(DeviceEdits* e);
+void forget_nodes(DeviceEdits* e, uint64_t first); // nodes from `first` on are replaced (the device is idle)
 
 // Best-effort release paths: an error here has nowhere useful to go.
 inline void release(void* p) { (void)hipFree(p); }

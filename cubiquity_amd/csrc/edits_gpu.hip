@@ -1262,6 +1262,16 @@ struct DeviceEdits {
     size_t current = 0;
 };
 
+// The index names nodes by what they held: with one of them replaced or cut off it is made anew by the
+// next edit, which would otherwise take a node past the store's end for one of its own.
+void forget_nodes(DeviceEdits* e, uint64_t first)
+{
+    if (!e || first >= e->indexed) return;
+    release(e->index);
+    e->index = nullptr;
+    e->index_cap = e->indexed = 0;
+}
+
 void destroy_device_edits(DeviceEdits* e)
 {
     if (!e) return;

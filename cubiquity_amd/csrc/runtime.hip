@@ -1317,6 +1317,7 @@ cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nod
     for (int c = 0; c < 8; c++)
         if (s[c].node > 0) max_height = std::max(max_height, int(s[c].height));
     HIP_TRY(hipDeviceSynchronize()); // launches in flight may read the store
+    cqx::forget_nodes(vol->edits, first);
     const uint32_t* old_nodes = vol->nodes;
     if (node_count > vol->capacity) {
         const uint64_t cap = std::max<uint64_t>(node_count, vol->capacity + vol->capacity / 2);
