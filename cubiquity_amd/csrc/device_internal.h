@@ -100,7 +100,8 @@ cqx_status ensure_scratch(cqx_ctx* ctx, size_t bytes);
 // `first` says, and launches on any stream read it), and drops the path tracer's plan if it is this
 // volume's and its graph no longer fits. A copy that cannot be allocated is left out. Words hold their
 // children's masks: where the change reaches into the upload, whose nodes may have changed ones as
-// children, all are made anew, and a store cut short of its upload is walked raw.
+// children, all are made anew, and a store cut short of its upload, or of the root that an undo went back
+// to, is walked raw.
 cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first);
 
 // Rays per wave of a one-ray-per-lane launch of n rays (at most 64).

@@ -1540,6 +1540,9 @@ cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sph
     } catch (const std::bad_alloc&) {
         return fail(CQX_ERR_OOM, "out of host memory while planning edits");
     }
+    if (vol->root >= vol->node_count) // an undo past an update that cut the store
+        return fail(CQX_ERR_INVALID_DAG, "root %u is not in the store of %llu nodes", vol->root,
+                    (unsigned long long)vol->node_count);
     cqx::DeviceEdits* E = vol->edits;
     HIP_TRY(hipDeviceSynchronize()); // launches in flight may read the store or the index
     const uint64_t base = vol->node_count;

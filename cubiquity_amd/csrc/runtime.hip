@@ -894,7 +894,8 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
         }
         vol->packed_count = vol->node_count;
     }
-    vol->packed_ok = vol->packed && vol->node_count >= vol->uploaded && packed_eligible(vol->node_count, vol->hsub);
+    vol->packed_ok = vol->packed && vol->root < vol->node_count && vol->node_count >= vol->uploaded &&
+                     packed_eligible(vol->node_count, vol->hsub);
     return vol->packed_ok == old_ok ? CQX_OK : drop_plan();
 }
 
