@@ -24,6 +24,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+# Vector instructions a second: 1024 SIMDs at 2.4 GHz, each one wave instruction per 2 cycles at best
+# (walk_packed.h says which take 2 and which 4).
+VALU_PEAK_GINST = 1024 * 2.4 / 2
 
 
 def log(*a):
@@ -89,6 +92,35 @@ def traffic_from_profiles(launch):
         if p.get("launch") == launch:
             return p.get("hbm_bytes_per_launch"), p.get("l2_hit_rate"), os.path.relpath(path, ROOT)
     return None, None, None
+
+
+def valu_from_profiles(launch):
+    """Vector instructions (per wave) of one launch of the headline traversal, from the same profile."""
+    path = os.path.join(ROOT, "profiles", "traffic_intersect_incoherent_1024.json")
+    if not os.path.exists(path) or launch is None:
+        return None
+    with open(path) as f:
+        return next((p.get("sq_insts_valu_per_launch") for p in json.load(f).get("launches", [])
+                     if p.get("launch") == launch), None)
+
+
+def roofline(ms, alg_bytes, traffic, valu):
+    """What a launch of `ms` reaches of the peak that bounds it: vector issue where the launch's instructions
+    are on record, else HBM on the algorithmic bytes (no fraction where those come from the caches faster than
+    HBM could bring them). Beside it the HBM rate on measured traffic."""
+    hbm = None
+    if traffic:
+        rate = traffic / (ms * 1e-3) / 1e9
+        hbm = {"achieved": round(rate, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(rate / HBM_PEAK_GBS, 4)}
+    alg = alg_bytes / (ms * 1e-3) / 1e9
+    if valu:
+        rate = valu / (ms * 1e-3) / 1e9
+        r = {"bound": "valu_issue", "achieved": round(rate, 2), "peak": VALU_PEAK_GINST, "unit": "Ginst/s",
+             "frac": round(rate / VALU_PEAK_GINST, 4)}
+    else:
+        r = {"bound": "hbm", "achieved": round(alg, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+             "frac": round(alg / HBM_PEAK_GBS, 4) if alg <= HBM_PEAK_GBS else None}
+    return {**r, "hbm": hbm, "algorithmic_gbs": round(alg, 2)}
 
 
 def profiled_launches():
@@ -673,7 +705,6 @@ def main():
     iters = int(hits["iters"].astype(np.int64).sum())
     anomalies = int(((hits["info"] >> 15) & 1).sum())
     alg_bytes = args.rays * (24 + 32) + 32 * entries
-    achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
     timed_launch = None
     if tuned and "timed_instead" in tuned:
         timed_launch = tuned["timed_instead"]["launch"]
@@ -708,19 +739,14 @@ def main():
                       "explicit variant" if args.variant else "built-in defaults",
         },
         "roofline": {
-            "bound": "hbm",
-            "achieved": round(achieved, 2),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            **roofline(avg_ms, alg_bytes, traffic, valu_from_profiles(timed_launch) if headline else None),
             "traffic": traffic,
             "l2_hit_rate": l2_hit_rate,
             "traffic_profile": profile,
             "timed_launch": timed_launch,
             "limiter": ("measured at 1024^3: cache-resident (the store sits in the MALL; L2 hits ~86 %, HBM traffic "
                         "~0.22x the algorithmic bytes), bound by the issue of divergent VALU work (one instruction "
-                        "per 2.5 cycles and SIMD, ~46 % of lanes active), not by HBM bandwidth; 'hbm' names the "
-                        "roofline the algorithmic bytes are priced against" if headline else
+                        "per 2.5 cycles and SIMD, ~46 % of lanes active), not by HBM bandwidth" if headline else
                         "measured at 16384^3 (tuned launch): ~1.6x the algorithmic bytes fetched (a 128-B line "
                         "per 32-B node read, L2 hits ~52 %), at ~0.75 of HBM peak on that traffic: bound by HBM "
                         "bandwidth on whole lines" if w is W.LARGE_16384 else
