@@ -495,8 +495,8 @@ cqx_status cqx_demo_trace(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray* r
     // "auto" (cfg null or variant 0): the primaries (coherent camera rays) one per lane, 64 per
     // workgroup; the secondary lists dealt to the waves (dealt_ids), or, over a raw store or when the
     // caller shaped the launch, on a light persistent grid of 16 waves per CU: the frame's batches
-    // are too small for the persistent default (32 waves per CU) to pay. Dealt: 0.60 -> 0.54 ms on the
-    // 1280x720 frame at 1024^3.
+    // are too small for the persistent default to pay. Dealt: 0.506 -> 0.446 ms on the 1280x720
+    // frame at 1024^3 (claimed by 24 waves per CU 0.558).
     // Only the fields the caller left at zero take these values.
     const uint32_t dealt2 = cqx::launch_open(cfg) ? cqx::dealt_ids(3 * n) : 0u;
     const uint32_t dealt3 = cqx::launch_open(cfg) ? cqx::dealt_ids(2 * n) : 0u;

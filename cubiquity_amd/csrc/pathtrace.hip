@@ -213,7 +213,8 @@ __device__ __forceinline__ void path_start(const PtDevParams& d, uint64_t p, Pcg
 //
 // Units of a list are dealt in turn to the 8 XCDs (a unit is a workgroup), and the units past a part's
 // count are empty, so equal rows of the parts must not fall on equal XCDs: with row u % per for unit u,
-// the last of every 16 units empty, the first bounce's walk of 2^21 paths took 219 us, 180 rotated.
+// the last of every 16 units empty, frames take 5 % longer (2.1 M paths 512^3 adjoint 675 us, 644 rotated;
+// 14.7 M at 1024^3 2249, 2135).
 constexpr uint32_t kParts = 64;
 constexpr uint32_t kCountStride = 32; // words: 128 bytes
 struct PathList {
@@ -239,9 +240,9 @@ struct PathList {
     uint32_t units(uint32_t size) const { return uint32_t(parts * ((pcap + size - 1) / size)); }
 };
 
-// Paths per part of the camera pass's list. Frame times (us) at groups of 256, 1024, 4096, 8192 paths and
-// with the 64 parts of the other lists: 2.1 M paths 512^3 adjoint 809 / 765 / 742 / 745 / 764, 7.4 M at
-// 1024^3 1595 / 1575 / 1553 / 1550 / 1575, 14.7 M at 1024^3 2462 / 2465 / 2398 / 2393 / 2402.
+// Paths per part of the camera pass's list. Frame times (us) at groups of 256, 1024, 4096, 8192
+// paths: 2.1 M paths 512^3 adjoint 721 / 674 / 646 / 653, 7.4 M at 1024^3 1420 / 1397 / 1392 / 1385, 14.7 M
+// at 1024^3 2208 / 2209 / 2138 / 2150.
 inline uint32_t path_group(uint64_t P)
 {
     uint32_t g = 64;
@@ -372,7 +373,8 @@ __device__ __forceinline__ void store_path(const PathList& list, uint64_t slot, 
 // The camera pass on a packed volume: a path's camera ray, its walk (one ray per lane, `ids` per wave)
 // and its first vertex, in registers from one to the next: 14.7 M paths at 1024^3 in 582 us, with VALU
 // issue the bound as in the other walks. As three kernels (rays written once and read twice, 32-byte
-// records, claims on one counter) they took 66 + 573 + 189.
+// records, claims on one counter) they took 66 + 573 + 189. A burst of 8, 12, 16 or 24 steps is the same to
+// 0.5 %: no lane waits for a service pass here.
 template <bool kRadiance, bool kLod>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
 k_pt_camera(const PtDevParams* __restrict__ dp, uint64_t P, PackedParams T, uint32_t rows, uint32_t ids, PcgJump jump,

@@ -770,8 +770,8 @@ cqx_status bin_rays(cqx_ctx* ctx, const cqx_ray* rays, uint64_t n, const BinBox&
 // Defaults: the best launch of a sweep on the 1024^3 incoherent workload. The packed walk's steps do
 // more and its service passes cost less, so it regroups every 16 steps, with 28 waves per CU, and 24 up to
 // 2^23 rays: the fewer waves share a SIMD and its L1, the sooner a wave's reads and the last rays end.
-// Measured (us, 24 / 28 / 32 waves): 2^24 rays at 1024^3 1959 / 1855 / 1933 (12 steps: 1927 / 1882 /
-// 1912), 4.0 M at 4096^3 983 / 1040 / 1068 (994 / 1045 / 1054).
+// Measured (us, 24 / 28 / 32 waves): 2^24 rays at 1024^3 1919 / 1866 / 1914 (12 steps: 1932 / 1886 /
+// 1907), 6.0 M there 804 / 793 / 791, 4.0 M at 4096^3 982 / 1019 / 1052 (990 / 1028 / 1060).
 cqx_status persistent_shape(const cqx_ctx* ctx, const cqx_launch_cfg* cfg, uint32_t block, uint64_t n, bool packed,
                             uint32_t& blocks, uint32_t& regroup, uint32_t& refill, uint32_t& chunk)
 {
@@ -903,12 +903,13 @@ cqx_status refresh_packed(cqx_ctx* ctx, cqx_dvolume* vol, uint64_t first)
 // incoherent / camera rays at 1024^3 unless stated; K: ids per wave in 64s with refill 16, lane: 64 per
 // wave without refill, p: claimed by persistent waves):
 //   n                lane          K = 2         K = 4         p
-//   921600           272 / 138     256 / 173     268 / 275     278 / 224
-//   2.0 M            504 / 196     440 / 219     396 / 299     419 / 306
-//   4.0 M (4096^3)   1496          1259          1157          1037
-//   8.0 M            / 439         / 468         / 494         / 717
-//   2^24             3615          2918          2393          2035
-// Up to kLaneRays one ray per lane: close to the best for either kind. Beyond, the kinds part: a sample
+//   921600           251 / 109     227 / 147     223 / 220     247 / 209
+//   2.0 M            457 / 164     384 / 174     353 / 234     367 / 277
+//   4.0 M (4096^3)   1378          1117          1083          979
+//   8.0 M            1639 / 403    1278 / 390    1080 / 418    1021 / 638
+//   2^24             3358          2584          2134          1852
+// Up to kLaneRays one ray per lane: within 13 % of the best for incoherent rays, where K = 4 takes twice as
+// long for camera rays. Beyond, the kinds part: a sample
 // of the rays decides on the device between one ray per lane for coherent ones and, for the others,
 // dealt runs of 4 x 64 up to kDealtRays, claims by persistent waves past it (whose tail no longer
 // matters there). The sample takes 3 us; up to kDealtRays one of two launches returns at once (2 us), past
@@ -920,8 +921,8 @@ constexpr uint64_t kGateRays = uint64_t(1) << 31; // the lane launch's grid stay
 // Rays per wave of a one-ray-per-lane launch. A lone wave on a SIMD issues an instruction every 6
 // cycles against 2 to 4 with company, and a wave with fewer rays takes fewer of a step's paths, so a
 // batch that cannot fill the chip is spread: at most 4 rays per wave up to 4096 waves, then 2048 waves
-// (two per SIMD) up to 64. Measured (us, spread / 64 per wave, 1024^3): 64 rays 51 / 66, 1024 66 / 73,
-// 8192 80 / 100, 65536 108 / 120.
+// (two per SIMD) up to 64. Measured (us, spread / 64 per wave, 1024^3): 64 rays 28 / 38, 1024 48 / 62,
+// 8192 64 / 72, 65536 80 / 86.
 uint32_t lanes_per_wave(uint64_t n)
 {
     uint32_t g = 1;
@@ -932,9 +933,10 @@ uint32_t lanes_per_wave(uint64_t n)
 // Ids per wave of a launch over secondary rays (path-tracer bounces, shadow rays) whose count, at most
 // n and usually half of it, is known on the device only: neighbours start near each other, so that
 // short runs hold longer than for random rays, and no counters are cleared and claimed between two
-// launches. Frame times (ms) at K = 64, 128, 256 ids per wave, and claimed by 24 waves per CU: 2.1 M
-// paths 512^3 adjoint 0.85 / 0.89 / 1.01 / 1.08, 4.9 M at 512^3 1.02 / 1.04 / 1.10 / 1.17, 7.4 M at 1024^3
-// 1.79 / 1.75 / 1.84, 14.7 M at 1024^3 3.07 / 2.87 / 2.79 / 2.78.
+// launches. Frame times (ms) at K = 64, 128, 256 ids per wave: 2.1 M paths 512^3
+// adjoint 0.65 / 0.67 / 0.75, 4.9 M at 512^3 0.92 / 0.90 / 0.99, 7.4 M at 1024^3 1.49 / 1.39 / 1.44, 14.7 M
+// at 1024^3 2.49 / 2.24 / 2.14. Claimed by 24 waves per CU the same frames took 0 to 27 % longer (on an
+// earlier, longer step).
 uint32_t dealt_ids(uint64_t n)
 {
     return n <= (1u << 22) ? lanes_per_wave(n) : n <= (1u << 23) ? 128u : 256u;
@@ -1117,8 +1119,8 @@ namespace {
 
 // Host-buffer calls of up to this many rays are traced from and to pinned host memory, which the waves
 // read and write over the bus as they go: no copy before the launch and none after it, each a queued
-// operation of its own. Measured per call at 512^3 (MI355X, us, pinned / copied): 1 ray 29 / 38, 97
-// 63 / 76, 1000 67 / 84, 4096 78 / 93, 16384 106 / 131, 65536 243 / 343. The line bounds the memory held
+// operation of its own. Measured per call at 512^3 (MI355X, us, pinned / copied): 1 ray 25 / 35, 97
+// 42 / 54, 1000 61 / 78, 4096 71 / 85, 16384 94 / 120, 65536 229 / 288. The line bounds the memory held
 // (3.7 MB a context).
 constexpr uint64_t kPinnedRays = 1u << 16;
 
@@ -1141,8 +1143,8 @@ void* pinned_buffer(cqx_ctx* ctx, size_t bytes)
 
 // Up to this many rays an open batched launch deals its ids to the waves, 64 or fewer each (lanes_per_wave):
 // batches of camera rays keep together and no counters are cleared, claimed and found empty. Past it
-// the claims of persistent waves win. Measured (MI355X, us, dealt / claimed): 27 k rays of 5 volumes
-// 75 / 88, 1.65 M of 24 216 / 300, 2.47 M of 32 294 / 351, 11.1 M of 64 1508 / 1258.
+// the claims of persistent waves win. Measured (MI355X, us, dealt / claimed): 14 k rays of 5 volumes
+// 52 / 74, 1.43 M of 24 194 / 243, 1.85 M of 32 226 / 269, 14.7 M of 64 1667 / 1335.
 constexpr uint64_t kDealtBatchRays = 1u << 22;
 
 struct WalkLaunch {

@@ -100,8 +100,8 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 //                   otherwise claimed by the first `want` workgroups; the rest end at once, in the slots
 //                   that those leave free (as a launch of its own they took 17 us of 1.87 ms at 2^24 rays)
 // With `gate`, a kDealt launch runs only when the flag equals `want`.
-// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take 72 and 7 waves (24 volumes
-// 193 us with 6 waves, 189 with 7, 194 with 8 and 8 to 13 registers spilled).
+// At 64 VGPRs 8 waves fit a SIMD; the batched form's per-lane parameters take 72 and 7 waves (1.2 M rays of
+// 24 volumes 185 us with 6 waves, 183 with 7, 191 with 8 and registers spilled; 15 M of 64 1232, 1176, 1267).
 enum WalkForm { kClaimed, kDealt, kSampled };
 
 template <typename Source, bool kLod, WalkForm kForm>

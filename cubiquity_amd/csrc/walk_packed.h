@@ -20,15 +20,16 @@
 //     exclusive or and masks.
 //   * Per-axis choices are sign masks (a float difference's sign bit shifted over the word) instead
 //     of compare + select, and min/max of three values one instruction.
-// Measured against the raw-store walk (MI355X, default launch): 1024^3, 2^24 incoherent rays 3.13 ->
-// 2.21 ms; 4096^3, 4.0 M rays without surface properties 2.00 -> 1.18 ms; 1280x720 primary rays at
-// 1024^3 with LOD 0.30 -> 0.24 ms; reads from L2 5.5e8 -> 2.6e8 per 2^24-ray launch.
+// Measured against the raw-store walk (MI355X, default launches): 1024^3, 2^24 incoherent rays 3.13 ->
+// 1.85 ms; 4096^3, 4.0 M rays without surface properties 2.02 -> 0.98 ms; 1280x720 primary rays at
+// 1024^3 with LOD 0.30 -> 0.084 ms; 1021 incoherent rays at 512^3 0.116 -> 0.041 ms; reads from L2 5.8e8 ->
+// 2.7e8 per 2^24-ray launch.
 // A step's instructions matter twice: as issue cycles where waves fill the chip, and, where they do not
 // (small batches, the long rays a launch ends with), as the length of one wave's chain: about 170
 // instructions and a read's latency a step. So the child's entry planes are computed while its word is
 // in flight, a walk that left stands on node 0 instead of taking a branch of its own, and phases and the
 // stack base stay in registers the compiler cannot remake in every branch: 144 -> 113 VALU instructions
-// and 60 -> 37 scalar ones. 1280x720 camera rays with LOD at 1024^3 99 -> 80 us, 65536 camera rays 37.5 ->
+// and 60 -> 37 scalar ones. By that alone, 1280x720 camera rays with LOD at 1024^3 99 -> 80 us, 65536 camera rays 37.5 ->
 // 30 us, 1021 incoherent rays 51 -> 37 us, 2^24 2.07 -> 1.93 ms. (Reading the next word already at the end
 // of a step, with its waits where they belong, took 12 to 20 more instructions and 4 to 12 % longer.)
 // The sign masks and one-instruction minima need values without NaN, -0 and underflow: ray_plain() is true for rays where
