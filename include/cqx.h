@@ -268,15 +268,19 @@ cqx_status cqx_create(int device, cqx_ctx** out);
 cqx_status cqx_destroy(cqx_ctx* ctx);
 
 /* Upload a store (node_count x 32 B incl. the material nodes, as the reference's SSBO upload
- * does) and its SubDAGs (NULL: computed here). Validates the store first. */
+ * does) and its SubDAGs (NULL: computed here). Validates what the root reaches first. Stores of up to
+ * 2^24 nodes take the same memory again for the copy that launches walk (at most 512 MB; where it cannot be
+ * had, launches walk the store itself, slower). CQX_PACKED_NODES=<nodes> in the environment lowers that
+ * limit, 0 to keep no copies; updates and edits keep the copy in step with the store. */
 cqx_status cqx_volume_upload(cqx_ctx* ctx, const uint32_t* nodes, uint64_t node_count, uint32_t root,
                              const cqx_subdag sub[8], cqx_dvolume** out);
 cqx_status cqx_volume_free(cqx_ctx* ctx, cqx_dvolume* vol);
 /* Append-only delta after host edits (cqx_hv_edit_spheres): nodes [first, node_count) of the
  * host store are copied to the device (the first `first` nodes must be unchanged since the
  * upload), and the root and SubDAGs (NULL: recomputed) are replaced. Appended nodes may only
- * reference material nodes or earlier nodes. Waits for the device to be idle. (The reference
- * re-uploads nothing after edits: its GPU viewer has no onVolumeModified,
+ * reference material nodes or earlier nodes. `first` may lie before nodes of the upload or of device
+ * edits: they are replaced (their index is made again by the next device edit). Waits for the device
+ * to be idle. (The reference re-uploads nothing after edits: its GPU viewer has no onVolumeModified,
  * gpu_pathtracing_viewer.h:14-26.) */
 cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nodes, uint64_t node_count,
                              uint64_t first, uint32_t root, const cqx_subdag sub[8]);
@@ -293,7 +297,8 @@ cqx_status cqx_volume_update(cqx_ctx* ctx, cqx_dvolume* vol, const uint32_t* nod
 cqx_status cqx_volume_edit_spheres(cqx_ctx* ctx, cqx_dvolume* vol, const cqx_sphere_edit* edits, uint64_t n,
                                    uint64_t* first_new);
 /* Edit history of a device volume (Volume::checkpoint / undo / redo, storage.cpp:358-385): roots
- * recorded and switched; no node changes, the SubDAGs are recomputed on the device. */
+ * recorded and switched; no node changes, the SubDAGs are recomputed on the device. An edit of a state
+ * whose root an update cut off fails with CQX_ERR_INVALID_DAG. */
 cqx_status cqx_volume_checkpoint(cqx_ctx* ctx, cqx_dvolume* vol);
 cqx_status cqx_volume_undo(cqx_ctx* ctx, cqx_dvolume* vol);
 cqx_status cqx_volume_redo(cqx_ctx* ctx, cqx_dvolume* vol);
@@ -370,9 +375,10 @@ cqx_status cqx_autotune(cqx_ctx* ctx, const cqx_dvolume* vol, const cqx_ray* ray
                         cqx_launch_cfg* best, float* best_ms);
 cqx_status cqx_autotune_clear(cqx_ctx* ctx);
 
-/* Many (volume, ray batch) pairs in ONE persistent launch: the batches are laid end to end in
- * one ray-id space that the persistent waves drain together, so batches of very different sizes
- * and volumes of different depths share the GPU without a launch per batch. Per-ray semantics
+/* Many (volume, ray batch) pairs in ONE launch: the batches are laid end to end in one ray-id
+ * space, dealt to the waves up to 2^22 rays (cfg open, as cqx_launch_cfg says) and claimed by
+ * persistent waves beyond, so batches of very different sizes and volumes of different depths share the
+ * GPU without a launch per batch. Per-ray semantics
  * are intersectVolume's (raytracing.cpp:397-478). rays/hits are device pointers. One batched
  * launch in flight per context. (No reference counterpart: the reference raycasts one ray per
  * call.) */
