@@ -93,11 +93,11 @@ def build_cpp_checks(verbose=False, strict=True):
                 "core_emulation": emulation, "packed_emulation": emulation}
     for name, flags in programs.items():
         src, out = os.path.join(cpp, name + ".cpp"), os.path.join(cpp, name)
-        if os.path.exists(out):
-            os.remove(out)  # a test never runs the program of an older source
-        if not os.path.exists(src):
-            continue
         try:
+            if os.path.exists(out):
+                os.remove(out)  # a test never runs the program of an older source
+            if not os.path.exists(src):
+                continue
             _run([CXX, "-std=c++17", "-O2", src, "-o", out] + flags, verbose)
         except (RuntimeError, OSError) as e:
             if strict:
